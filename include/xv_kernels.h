@@ -435,6 +435,26 @@ int xv_dense_gemm(const void* x, int64_t x_stride, const void* w_packed, void* o
                   hipStream_t stream);
 
 /*
+ * Weight-streaming GEMM of a short batch over the weight in place: x[m, k] .
+ * w[n, k]^T, m <= 256, bf16 operands, fp32 accumulate.  The same products as
+ * xv_dense_gemm, without a packed copy of the weight and up to 256 rows.
+ *   x, w      row i at i * x_stride / i * w_stride (multiples of 8, >= k), 16-byte aligned.
+ *   mode 1    fp32 partial products of K split `parts` ways: out[p][i][j] at
+ *             p * part_stride + i * out_stride + j, 16-byte aligned, strides
+ *             multiples of 4; their sum over p is the product.
+ *   mode 2    w is the gate/up weight [2I, k] (gate rows first); bf16
+ *             out[m, I] = silu(g) * u with g, u the two products rounded to
+ *             bf16; 8-byte aligned, out_stride a multiple of 4; parts 1.
+ * xv_stream_gemm_parts gives the `parts` such a call takes (1 .. 8), or 0
+ * where these shapes are not taken: n / 16 tiles that do not divide into
+ * about 256 workgroups, or a K slice that is not whole stages (128 elements
+ * up to 64 rows, else 64).  Any other `parts` is hipErrorInvalidValue.
+ */
+int xv_stream_gemm_parts(int m, int n, int k, int mode);
+int xv_stream_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out, int64_t out_stride,
+                   int64_t part_stride, int m, int n, int k, int mode, int parts, hipStream_t stream);
+
+/*
  * Streaming copy of `bytes` (a multiple of 16; both pointers 16-byte aligned)
  * with non-temporal 16-byte loads and stores.  No counterpart in the
  * reference: a measurement yardstick for the HBM-bound kernels above (what a

@@ -1,0 +1,127 @@
+"""The in-place streaming GEMM (xv_stream_gemm) against a float64 product of
+the same bf16 operands, at the edges of its row classes (16, 32, 64, 128, 256
+rows) and over every tile count its rule picks.  Partial sums: the fp32 sum
+of K products in any order is within K 2^-24 sum |x w| of the exact one.
+SiLU-and-mul: g and u are rounded to bf16 before it and the result after
+it, rtol/atol 2e-2 over the bf16-rounded products as the packed kernel's test."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 15, 16, 17, 32, 33, 64, 65, 128, 129, 200, 256]
+# (n, k): tiles per workgroup over the row classes 1, 2 / 1, 2 / 2, 4 / 2, 8 / 5, 10 / 6
+SHAPES = [(1024, 2048), (1024, 3072), (4096, 1024), (4096, 12288), (5120, 25600), (6144, 4096)]
+
+
+def _operands(dev, m, n, k, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn((m, k), generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn((n, k), generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    return x, w
+
+
+def _check_parts(ps, x, w):
+    xd, wd = x.double(), w.double()
+    want, bound = xd @ wd.T, (xd.abs() @ wd.abs().T) * (x.shape[1] * 2.0**-24)
+    err = (ps.parts.double().sum(0) - want).abs() - bound
+    assert torch.isfinite(ps.parts).all()
+    assert (err <= 0).all(), f"max excess {err.max().item():.3g}"
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_parts(dev, shape):
+    from xvllm.layers.linear import GEMM_PARTS, PartialSums, in_place_parts, streamed_into_norm
+
+    n, k = shape
+    for m in ROWS:
+        p = in_place_parts(m, n, k, GEMM_PARTS)
+        print(f"stream gemm m {m} n {n} k {k} parts {p}", flush=True)
+        x, w = _operands(dev, m, n, k, m + n)
+        ps = streamed_into_norm(x, w)
+        assert isinstance(ps, PartialSums) and ps.parts.shape == (p, m, n)
+        _check_parts(ps, x, w)
+
+
+# blocks of 2 tiles, 4, 6 and 8 above 16 rows
+@pytest.mark.parametrize("inter", [3072, 4096 * 2, 12288, 16384])
+def test_silu_mul(dev, inter):
+    from xvllm.layers.linear import streamed_silu_mul
+
+    k = 512
+    for m in ROWS:
+        print(f"stream gemm silu m {m} I {inter}", flush=True)
+        x, w = _operands(dev, m, 2 * inter, k, m + inter)
+        gu = (x.double() @ w.double().T).to(torch.bfloat16).double()
+        g, u = gu[:, :inter], gu[:, inter:]
+        want = g * torch.sigmoid(g) * u
+        out = streamed_silu_mul(x, w)
+        assert out.shape == (m, inter) and out.dtype == torch.bfloat16
+        err = (out.double() - want).abs() - (2e-2 + 2e-2 * want.abs())
+        assert torch.isfinite(out).all() and (err <= 0).all(), f"max excess {err.max().item():.3g}"
+
+
+def test_strided_rows(dev):
+    """x and w as row-strided views, and x off its 16-byte alignment (copied first)."""
+    from xvllm.layers.linear import streamed_into_norm
+
+    x, w = _operands(dev, 40, 1024, 2048, 3)
+    wide_x = torch.full((40, 2048 + 64), float("nan"), dtype=torch.bfloat16, device=dev)
+    wide_w = torch.full((1024, 2048 + 128), float("nan"), dtype=torch.bfloat16, device=dev)
+    for off in (8, 32, 3):
+        wide_x[:, off : off + 2048] = x
+        wide_w[:, 64 : 64 + 2048] = w
+        _check_parts(streamed_into_norm(wide_x[:, off : off + 2048], wide_w[:, 64 : 64 + 2048]), x, w)
+
+
+def test_rows_are_independent(dev):
+    """Rows of infinities and NaN, and the row count itself, leave the other rows' bits alone."""
+    from xvllm.layers.linear import streamed_into_norm
+
+    x, w = _operands(dev, 64, 1024, 2048, 4)
+    ref = streamed_into_norm(x, w).parts
+    bad = x.clone()
+    bad[7], bad[40, 5] = float("nan"), float("inf")
+    got = streamed_into_norm(bad, w).parts
+    keep = [i for i in range(64) if i not in (7, 40)]
+    assert torch.equal(got[:, keep], ref[:, keep])
+    assert torch.isnan(got[:, 7]).all()
+    assert torch.equal(streamed_into_norm(x[:50], w).parts, ref[:, :50])
+
+
+@pytest.mark.parametrize("m", [1, 40, 64, 100, 256, 257])
+@pytest.mark.parametrize("width", ["0.6B", "8B"])
+def test_mlp_streams_and_matches_the_library(dev, m, width):
+    """The MLP, packed or not: packed models stream up to 256 rows, others the
+    products into a norm where linear_into_norm splits, all within the
+    bf16 tolerance of the library's product; with gradients on, an unpacked
+    model keeps the library's."""
+    from xvllm.config import QWEN3_0_6B, QWEN3_8B
+    from xvllm.layers.linear import PartialSums, split_factor
+    from xvllm.models.qwen3 import Qwen3MLP
+
+    s = QWEN3_0_6B if width == "0.6B" else QWEN3_8B
+    g = torch.Generator(device=dev).manual_seed(m)
+    with torch.device(dev):
+        mlp = Qwen3MLP(s.hidden_size, s.intermediate_size).to(torch.bfloat16)
+    with torch.no_grad():
+        for p in mlp.parameters():
+            p.normal_(0.0, 0.02, generator=g)
+        x = torch.randn((m, s.hidden_size), generator=g, device=dev).to(torch.bfloat16)
+        mlp.split_k = False
+        want = mlp(x).double()
+        mlp.split_k = True
+        split = split_factor(m, s.hidden_size, s.intermediate_size) > 1
+        outs = [mlp(x)]
+        assert isinstance(outs[0], PartialSums) == split
+        mlp.pack()
+        outs.append(mlp(x))
+        assert isinstance(outs[1], PartialSums) == (m <= 256)
+        mlp.pack(False)
+    library = mlp(x)  # gradients of the weights asked for
+    assert isinstance(library, PartialSums) == split
+    outs.append(library)
+    for out in outs:
+        got = (out.materialize() if isinstance(out, PartialSums) else out).double()
+        rel = (got - want).norm() / want.norm()
+        assert rel < 1e-2, f"relative L2 {rel:.3g}"

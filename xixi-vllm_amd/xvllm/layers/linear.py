@@ -1,13 +1,21 @@
-"""Dense GEMMs of the decoder: PyTorch (hipBLASLt) with a split-K form for
-the two whose output goes straight into a residual add + RMSNorm (o_proj and
-down_proj, reference src/compute/models/qwen3.py:64,115 feeding the norms of
-:150,:152), and, opt-in for decode batches of at most 64 rows of a model with
-packed weights, the weight-streaming gfx950 kernel (xv_dense_gemm) over
-packed weight tiles: gate_up fused with SiLU-and-mul, down and o as split-K
-partials for the same norm (dense_gemm and the streamed_* helpers at the end
-of this file; measured 11-27 % faster than the hipBLASLt forms below at M 8
-and 64, weights streamed from HBM).  The split-K measurements below are the
-hipBLASLt path, the default.
+"""Dense GEMMs of the decoder: up to 256 rows the gfx950 kernel that streams
+the [N, K] weight in place (xv_stream_gemm: gate_up fused with SiLU-and-mul,
+down and o as split-K partials for the norm that follows them, reference
+src/compute/models/qwen3.py:64,115 feeding the norms of :150,:152), above that
+and for shapes it does not take PyTorch (hipBLASLt) with a split-K form for the
+latter two.  pack_weight / dense_gemm are the older streamed form over packed
+weight tiles (at most 64 rows), kept where the in-place kernel does not take
+a shape: Qwen3-32B's gate_up (51200 x 5120) at 17 to 64 rows, 87 us at 32
+rows against hipBLASLt's 98.
+
+us with the weights streamed from HBM, hipBLASLt -> in place (gate_up with
+its SiLU; MI355X, graph replay, over 1 GB of weights cycled):
+    Qwen3-8B    gate_up  M 8: 46.5 -> 31.0   M 64: 47.8 -> 34.6   M 200: 64.5 -> 54.9
+                down     M 8: 22.1 -> 18.1   M 64: 23.6 -> 20.1   M 200: 34.6 -> 31.7
+                o        M 8: 10.3 -> 8.0    M 64: 14.8 -> 9.6    M 200: 18.1 -> 16.6
+    Qwen3-0.6B  gate_up  M 8: 10.3 -> 5.1    down M 8: 12.1 -> 4.0   o M 8: 9.7 -> 3.4
+
+The split-K measurements below are the hipBLASLt path.
 
 At decode batch sizes an [M, K] x [K, 4096] GEMM has few output tiles for 256
 CUs: hipBLASLt runs Qwen3-8B's o_proj (K 4096) and down_proj (K 12288) at
@@ -188,24 +196,21 @@ def dense_gemm(x: torch.Tensor, w: PackedWeight, mode: int = GEMM_BF16, *, col_t
     return PartialSums(out) if mode == GEMM_PARTS else out
 
 
-# Batches of up to this many rows take the weight-streaming kernel when the
-# model holds packed weights (pack_decode_weights): decode batches, and also
-# prefill chunks this short (the same products); larger batches stay on
-# hipBLASLt over the [N, K] weights.
-STREAM_MAX_ROWS = 64
-
-
 def stream_parts(k: int) -> int:
-    """K slices of a split-K streamed GEMM (the most of 8, 4, 2, 1 that cut K
-    into whole 4-step rounds)."""
+    """K slices of a split-K product over a packed weight (the most of 8, 4,
+    2, 1 that cut K into whole 4-step rounds)."""
     for p in (8, 4, 2, 1):
         if k % (p * 256) == 0:
             return p
     return 0
 
 
+# Rows up to which a packed weight is streamed (xv_dense_gemm).
+STREAM_MAX_ROWS = 64
+
+
 def streamable(w: torch.Tensor, mode: int) -> bool:
-    """Whether w [N, K] fits the shapes the streamed decode GEMMs use:
+    """Whether w [N, K] fits the shapes of the packed decode GEMMs:
     gate/up + SiLU with 2 tiles x 4 waves (2I % 128), split-K partials with
     1 tile x 8 waves (N % 128)."""
     n, k = w.shape
@@ -215,24 +220,104 @@ def streamable(w: torch.Tensor, mode: int) -> bool:
 
 
 def stream_rows(x: torch.Tensor) -> bool:
-    """Whether activations x [M, K] can take a streamed decode GEMM: at most
-    STREAM_MAX_ROWS rows, unit stride along K, 16-byte aligned rows (other
-    layouts stay on hipBLASLt)."""
+    """Whether activations x [M, K] can take a packed decode GEMM: at most
+    STREAM_MAX_ROWS rows, unit stride along K, 16-byte aligned rows."""
     return (0 < x.shape[0] <= STREAM_MAX_ROWS and x.stride(1) == 1 and x.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0)
 
 
-def streamed_silu_mul(x: torch.Tensor, w: PackedWeight) -> torch.Tensor:
-    """silu(x w_gate^T) * (x w_up^T) of a decode batch, bf16 [M, I]."""
-    return dense_gemm(x, w, GEMM_SILU_MUL, col_tiles=2, waves=4)
+def in_place_parts(m: int, n: int, k: int, mode: int) -> int:
+    """Partial sums of an [m, k] x [k, n] product on the kernel that streams
+    the [N, K] weight in place (xv_stream_gemm): 1 .. 8, or 0 where it does
+    not take the shape (more than 256 rows, or a column count that does not
+    divide evenly over the CUs)."""
+    from .. import _C
+
+    return _C.lib().xv_stream_gemm_parts(m, n, k, mode)
 
 
-def streamed_into_norm(x: torch.Tensor, w: PackedWeight) -> PartialSums:
-    """x @ w^T of a decode batch as split-K PartialSums for the next residual
-    add + RMSNorm, K cut P = 8 ways where it allows; up to 32 rows, K slices
+@torch.library.custom_op("xv::stream_gemm", mutates_args=())
+def _stream_gemm(x: torch.Tensor, w: torch.Tensor, mode: int, parts: int) -> torch.Tensor:
+    """x [M, K] against w [N, K] in place: fp32 [parts, M, N] partial sums
+    (GEMM_PARTS) or bf16 silu(x w_gate^T) * (x w_up^T) [M, N / 2] (GEMM_SILU_MUL)."""
+    from .. import _C
+    from .._torch_glue import aligned16, ptr, require_bf16, require_cuda, stream_of
+
+    require_cuda(x, w)
+    require_bf16(x, w)
+    m, k = x.shape
+    n = w.shape[0]
+    if w.shape[1] != k:
+        raise ValueError(f"stream_gemm: x {tuple(x.shape)} and w {tuple(w.shape)} disagree on K")
+    if x.stride(1) != 1 or x.stride(0) % 8 or not aligned16(x):
+        x = x.clone(memory_format=torch.contiguous_format)
+    if w.stride(1) != 1:
+        raise ValueError("stream_gemm: w needs unit stride along K")
+    if mode == GEMM_PARTS:
+        out = torch.empty((parts, m, n), dtype=torch.float32, device=x.device)
+        os_, ps = n, m * n
+    else:
+        out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+        os_, ps = n // 2, 0
+    _C.check(
+        _C.lib().xv_stream_gemm(ptr(x), x.stride(0), ptr(w), w.stride(0), ptr(out), os_, ps, m, n, k, mode, parts,
+                                stream_of(x)),
+        "xv_stream_gemm",
+    )
+    return out
+
+
+@_stream_gemm.register_fake
+def _stream_gemm_fake(x, w, mode, parts):
+    m, n = x.shape[0], w.shape[0]
+    if mode == GEMM_PARTS:
+        return x.new_empty((parts, m, n), dtype=torch.float32)
+    return x.new_empty((m, n // 2))
+
+
+def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int):
+    """What streamed_silu_mul / streamed_into_norm read the weight w [N, K]
+    from for activations x: w itself where the in-place kernel takes the
+    shape, else its packed copy (if it has one) up to STREAM_MAX_ROWS rows,
+    else None (the library GEMM).  `packed` is the operand a packed model
+    holds, None for a model that was not packed.  Such a model's callers get
+    PartialSums only where linear_into_norm splits, so its products into a
+    norm stream only there; and with gradients asked of x or w the library
+    keeps the product (streaming has no backward; a packed model is inference
+    only)."""
+    if not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2:
+        return None
+    m, k = x.shape
+    n = w.shape[0]
+    if packed is None:
+        if mode == GEMM_PARTS and split_factor(m, n, k) == 1:
+            return None
+        if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+            return None
+    if (w.stride(1) == 1 and w.stride(0) % 8 == 0 and w.storage_offset() % 8 == 0
+            and in_place_parts(m, n, k, mode) > 0):
+        return w
+    return packed if isinstance(packed, PackedWeight) and stream_rows(x) else None
+
+
+def streamed_silu_mul(x: torch.Tensor, w) -> torch.Tensor:
+    """silu(x w_gate^T) * (x w_up^T) of a short batch, bf16 [M, I]; w is the
+    [2I, K] weight or its PackedWeight."""
+    if isinstance(w, PackedWeight):
+        return dense_gemm(x, w, GEMM_SILU_MUL, col_tiles=2, waves=4)
+    return torch.ops.xv.stream_gemm(x, w, GEMM_SILU_MUL, 1)
+
+
+def streamed_into_norm(x: torch.Tensor, w) -> PartialSums:
+    """x @ w^T of a short batch as split-K PartialSums for the next residual
+    add + RMSNorm; w is the [N, K] weight or its PackedWeight.  A packed
+    weight's K is cut P = 8 ways where it allows; up to 32 rows, K slices
     under 1024 elements are halved instead (measured: Qwen3-8B o_proj at
     M 8, P 4 7.3 us against P 8 7.8; down_proj P 8 at every M)."""
-    p = stream_parts(w.k)
-    if x.shape[0] <= 32 and w.k // p < 1024 and p > 1:
-        p //= 2
-    return dense_gemm(x, w, GEMM_PARTS, col_tiles=1, waves=8, parts=p)
+    if isinstance(w, PackedWeight):
+        p = stream_parts(w.k)
+        if x.shape[0] <= 32 and w.k // p < 1024 and p > 1:
+            p //= 2
+        return dense_gemm(x, w, GEMM_PARTS, col_tiles=1, waves=8, parts=p)
+    p = in_place_parts(x.shape[0], w.shape[0], x.shape[1], GEMM_PARTS)
+    return PartialSums(torch.ops.xv.stream_gemm(x, w, GEMM_PARTS, p))

@@ -65,12 +65,13 @@ class ModelRunner:
         point below which the plain decode is faster); the runner records a
         plain and a cascade decode graph per bucket and replays the one the
         staged batch selects.
-        `stream_decode_gemms` (off by default: the dense GEMMs stay on
-        PyTorch / hipBLASLt): pack the model's gate_up / down / o weights
-        (model.pack_decode_weights) so that decode batches of at most 64 rows
-        run them on the weight-streaming kernel; the weights must be final.
-        The packed copies take model.packed_decode_bytes() of device memory
-        (Qwen3-8B: 12.1 GB) beside the weights, which a KV pool sized before
+        `stream_decode_gemms` (off by default): fix the model's gate_up / down
+        / o weights (model.pack_decode_weights) so that decode batches stream
+        all three at every size up to 256 rows; without it only gate_up and
+        the products linear_into_norm splits stream, the rest staying on
+        PyTorch / hipBLASLt.  The weights must be final.  Weights the in-place kernel
+        does not take get packed copies of model.packed_decode_bytes() in all
+        (none at Qwen3-8B) beside the weights, which a KV pool sized before
         this runner does not see: size it with that figure as reserve_bytes.
         Packed copies an earlier runner made are kept either way (its graphs
         read them), and every runner of the model then uses them."""

@@ -4,11 +4,10 @@ reference's tp=1, pp=1 case of src/compute/models/qwen3.py:44-238).
 Per layer: input RMSNorm (fused with the residual add after layer 0), fused
 qkv GEMM, per-head q/k RMSNorm + NeoX RoPE (one kernel, `xv::qk_norm_rope`),
 `vllm::attention` (KV store + paged decode / prefill), o GEMM, fused add +
-RMSNorm, gate_up GEMM, SiLU-and-mul, down GEMM.  GEMMs run on PyTorch
-(hipBLASLt), except at decode batch sizes (at most 64 rows) once
-pack_decode_weights has made packed copies of gate_up, down and o: then the
-gate_up GEMM + SiLU-and-mul is one weight-streaming kernel, and down and o
-are streamed as split-K partials into the next norm.  Weights are plain
+RMSNorm, gate_up GEMM, SiLU-and-mul, down GEMM.  Batches of up to 256 rows
+stream gate_up (with the SiLU-and-mul), down and o in place (xv_stream_gemm),
+down and o as split-K partials into the next norm; larger ones and shapes
+that kernel does not take run on PyTorch (hipBLASLt).  Weights are plain
 tensors (random init for the benchmarks; the reference's checkpoint loader is
 out of scope).
 """
@@ -22,8 +21,8 @@ from ..config import head_dim as _head_dim
 from ..config import rope_theta as _rope_theta
 from ..layers import Attention, AttnInputs, RMSNorm, RotaryEmbedding
 from ..layers.attention import kv_cache_of, kv_scales
-from ..layers.linear import (GEMM_PARTS, GEMM_SILU_MUL, linear_into_norm, pack_weight, stream_rows, streamable,
-                             streamed_into_norm, streamed_silu_mul)
+from ..layers.linear import (GEMM_PARTS, GEMM_SILU_MUL, STREAM_MAX_ROWS, in_place_parts, linear_into_norm, pack_weight,
+                             stream_operand, stream_rows, streamable, streamed_into_norm, streamed_silu_mul)
 from ..layers import ops as _ops  # noqa: F401  (registers the custom ops)
 from ..sampler import sample
 
@@ -48,29 +47,48 @@ def _check_stamp(module, stamp: tuple, *params) -> None:
                                  "(outside graph capture; re-capture the decode graphs)")
 
 
+def _needs_copy(w: torch.Tensor, mode: int) -> bool:
+    """Whether decode batches of up to STREAM_MAX_ROWS rows stream w from a
+    packed copy: the in-place kernel does not take the shape at every size
+    (its rule has one case up to 16 rows and one above)."""
+    return any(in_place_parts(m, *w.shape, mode) == 0 for m in (16, STREAM_MAX_ROWS))
+
+
+def _decode_operand(p: nn.Parameter, mode: int):
+    """The weight itself where the in-place kernel streams it, else a packed copy."""
+    return pack_weight(p.data) if _needs_copy(p, mode) else p.data
+
+
 class Qwen3MLP(nn.Module):
     def __init__(self, hidden: int, inter: int):
         super().__init__()
         self.gate_up_proj = nn.Parameter(torch.empty(2 * inter, hidden))  # [gate; up] (linear.py:297-304)
         self.down_proj = nn.Parameter(torch.empty(hidden, inter))
         self.split_k = True
-        self.packed = None  # (gate_up, down) PackedWeights for decode batches
+        self.packed = None  # (gate_up, down) decode operands of pack()
 
     def forward(self, x):
         """SiLU-MLP; the down GEMM may return PartialSums (split-K) for the
         next residual add + RMSNorm."""
-        if self.packed is not None and self.split_k and stream_rows(x):
+        if not self.split_k:
+            return F.linear(torch.ops.vllm.silu_and_mul(F.linear(x, self.gate_up_proj)), self.down_proj)
+        if self.packed is not None and stream_rows(x):
             _check_stamp(self, self._stamp, self.gate_up_proj, self.down_proj)
-            return streamed_into_norm(streamed_silu_mul(x, self.packed[0]), self.packed[1])
-        return linear_into_norm(torch.ops.vllm.silu_and_mul(F.linear(x, self.gate_up_proj)), self.down_proj,
-                                self.split_k)
+        gate_up, down = self.packed or (None, None)
+        w = stream_operand(x, self.gate_up_proj, gate_up, GEMM_SILU_MUL)
+        if w is not None:
+            act = streamed_silu_mul(x, w)
+        else:
+            act = torch.ops.vllm.silu_and_mul(F.linear(x, self.gate_up_proj))
+        w = stream_operand(act, self.down_proj, down, GEMM_PARTS)
+        return streamed_into_norm(act, w) if w is not None else linear_into_norm(act, self.down_proj)
 
     def pack(self, enabled: bool = True):
         if not enabled:
             self.packed = None
         elif self.packed is None and streamable(self.gate_up_proj, GEMM_SILU_MUL) and streamable(self.down_proj,
                                                                                                    GEMM_PARTS):
-            self.packed = (pack_weight(self.gate_up_proj.data), pack_weight(self.down_proj.data))
+            self.packed = (_decode_operand(self.gate_up_proj, GEMM_SILU_MUL), _decode_operand(self.down_proj, GEMM_PARTS))
             self._stamp = _weight_stamp(self.gate_up_proj, self.down_proj)
 
 
@@ -90,7 +108,7 @@ class Qwen3Attention(nn.Module):
         self.attn = Attention(self.num_heads, self.head_dim, self.num_kv_heads, layer_id=layer_id)
         self.eps = cfg.rms_norm_eps
         self.split_k = True
-        self.packed_o = None  # o_proj PackedWeight for decode batches
+        self.packed_o = None  # o_proj decode operand of pack()
 
     def forward(self, positions, hidden, attn: AttnInputs):
         """qkv -> q/k norm + RoPE -> attention -> o GEMM (PartialSums when
@@ -103,16 +121,18 @@ class Qwen3Attention(nn.Module):
         else:
             q, k, v = self._split_norm_rope(positions, qkv)
             o = self.attn(q.view(q.shape[0], self.q_size), k, v, attn)
-        if self.packed_o is not None and self.split_k and stream_rows(o):
+        if not self.split_k:
+            return F.linear(o, self.o_proj)
+        if self.packed_o is not None and stream_rows(o):
             _check_stamp(self, self._stamp, self.o_proj)
-            return streamed_into_norm(o, self.packed_o)
-        return linear_into_norm(o, self.o_proj, self.split_k)
+        w = stream_operand(o, self.o_proj, self.packed_o, GEMM_PARTS)
+        return streamed_into_norm(o, w) if w is not None else linear_into_norm(o, self.o_proj)
 
     def pack(self, enabled: bool = True):
         if not enabled:
             self.packed_o = None
         elif self.packed_o is None and streamable(self.o_proj, GEMM_PARTS):
-            self.packed_o = pack_weight(self.o_proj.data)
+            self.packed_o = _decode_operand(self.o_proj, GEMM_PARTS)
             self._stamp = _weight_stamp(self.o_proj)
 
     def _views(self, qkv):
@@ -195,31 +215,35 @@ class Qwen3ForCausalLM(nn.Module):
 
     @torch.no_grad()
     def pack_decode_weights(self, enabled: bool = True):
-        """Packed copies of every layer's gate_up, down and o weights for the
-        weight-streaming decode GEMMs; layers that have them keep them (the
-        graphs captured over them stay valid).  enabled=False drops them: only
-        when no captured graph still uses them.  Call once the weights are
-        final: the copies do not follow later writes (an eager forward raises
-        StalePackedWeights when a packed weight was written in place or
-        replaced since).  They add packed_decode_bytes() to the weights,
-        (2 I H + I H + H Hq D) x 2 bytes per layer (Qwen3-8B: 335 MB per
-        layer, 12.1 GB; the Qwen3-32B shape: 56 GB): size the KV pool after
-        packing, or pass that figure as KVPool.auto_num_blocks' reserve_bytes."""
+        """Fix every layer's gate_up, down and o weights for the streamed
+        decode GEMMs.  Weights whose shape the in-place kernel takes at every
+        decode size are read where they are; the others (the Qwen3-32B
+        shape's gate_up: 524 MB per layer) get a packed copy for batches of
+        up to STREAM_MAX_ROWS rows, packed_decode_bytes() in all.  Layers that have
+        copies keep them (the graphs captured over them stay valid).
+        enabled=False drops them: only when no captured graph still uses
+        them.  Call once the weights are final: the copies do not follow later
+        writes (an eager forward raises StalePackedWeights when a fixed
+        weight was written in place or replaced since).  Size the KV pool
+        after packing, or pass packed_decode_bytes() as
+        KVPool.auto_num_blocks' reserve_bytes."""
         for m in self.modules():
             if isinstance(m, (Qwen3Attention, Qwen3MLP)):
                 m.pack(enabled)
         return self
 
     def packed_decode_bytes(self) -> int:
-        """Bytes pack_decode_weights adds (counted for the layers whose
-        weights the streamed GEMMs take)."""
+        """Bytes pack_decode_weights adds (the weights it copies)."""
         total = 0
         for m in self.modules():
             if isinstance(m, Qwen3MLP) and streamable(m.gate_up_proj, GEMM_SILU_MUL) and streamable(m.down_proj,
                                                                                                   GEMM_PARTS):
-                total += (m.gate_up_proj.numel() + m.down_proj.numel()) * m.gate_up_proj.element_size()
+                pairs = ((m.gate_up_proj, GEMM_SILU_MUL), (m.down_proj, GEMM_PARTS))
             elif isinstance(m, Qwen3Attention) and streamable(m.o_proj, GEMM_PARTS):
-                total += m.o_proj.numel() * m.o_proj.element_size()
+                pairs = ((m.o_proj, GEMM_PARTS),)
+            else:
+                continue
+            total += sum(w.numel() * w.element_size() for w, mode in pairs if _needs_copy(w, mode))
         return total
 
     def compute_logits(self, hidden):
