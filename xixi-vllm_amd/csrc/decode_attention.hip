@@ -516,6 +516,10 @@ XV_INLINE void process_page(SplitState& st, const char* buf, const LaneOffsets& 
 // Stream positions per half of the page-id table.
 constexpr int kIdWindow = 128;
 
+// sl[b] in LDS: the tokens of sequence b, with the sign bit set where a shared
+// prefix precedes them (cascade decode).
+constexpr int kCtxMask = 0x7fffffff;
+
 // Uniform position of a page in the flat (sequence, kv head, page) space.
 struct Cursor {
   int b, kvh, pg;  // sequence, kv head, 16-token page within the sequence
@@ -539,7 +543,7 @@ XV_INLINE void advance(Cursor& c, const int* pref, const int* sl, int hkv, int b
     ++c.b;
     c.npb = __builtin_amdgcn_readfirstlane(pref[c.b + 1] - pref[c.b]);
   } while (c.npb == 0 && c.b < batch - 1);
-  c.ctx = __builtin_amdgcn_readfirstlane(sl[c.b]);
+  c.ctx = __builtin_amdgcn_readfirstlane(sl[c.b]) & kCtxMask;
 }
 
 // Sequence holding flat page f: the largest b with hkv*pref[b] <= f.
@@ -613,6 +617,52 @@ XV_INLINE void read_q(bf16x8_t (&qb)[4], const char* slot, int lane) {
       : "memory");
 }
 
+// The output stage of a finished segment, in asm: at a plain LDS access the
+// compiler, which cannot tell the stage from the page buffers that LDS-DMA is
+// filling, waits for every page in flight, so that each finished segment
+// restarted the wave's page pipeline (32 rows of 4200 .. 12000 tokens, 64 q / 8
+// kv heads, half of them sharing a prefix: 158.7 -> 154.9 us a call, the
+// wait for a.pre_tokens at each finish gone with it; other batches 0.4 %).
+// Reads carry their own wait; writes are ordered by the wave_sync of
+// finish_segment.
+XV_INLINE uint4 stage_read16(const char* p) {
+  u32x4_t v;
+  __asm__ __volatile__("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                       : "=&v"(v)
+                       : "v"((uint32_t)reinterpret_cast<uintptr_t>(p))
+                       : "memory");
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+XV_INLINE float stage_read4(const float* p) {
+  float v;
+  __asm__ __volatile__("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                       : "=&v"(v)
+                       : "v"((uint32_t)reinterpret_cast<uintptr_t>(p))
+                       : "memory");
+  return v;
+}
+
+// Elements 16 nn (bytes 32 nn) of a row from p: v[nn] rounded to bf16.
+XV_INLINE void stage_write_row(uint16_t* p, const float (&v)[8]) {
+  uint32_t h[8];
+#pragma unroll
+  for (int nn = 0; nn < 8; ++nn) h[nn] = f32_to_bf16(v[nn]);
+  __asm__ __volatile__(
+      "ds_write_b16 %0, %1\n\t"
+      "ds_write_b16 %0, %2 offset:32\n\t"
+      "ds_write_b16 %0, %3 offset:64\n\t"
+      "ds_write_b16 %0, %4 offset:96\n\t"
+      "ds_write_b16 %0, %5 offset:128\n\t"
+      "ds_write_b16 %0, %6 offset:160\n\t"
+      "ds_write_b16 %0, %7 offset:192\n\t"
+      "ds_write_b16 %0, %8 offset:224" ::"v"((uint32_t)reinterpret_cast<uintptr_t>(p)),
+      "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(h[4]), "v"(h[5]), "v"(h[6]), "v"(h[7])
+      : "memory");
+}
+XV_INLINE void stage_write4(float* p, float v) {
+  __asm__ __volatile__("ds_write_b32 %0, %1" ::"v"((uint32_t)reinterpret_cast<uintptr_t>(p)), "v"(v) : "memory");
+}
+
 // Write the finished segment (b, kvh): bf16 output if this wave covered the
 // whole segment, else the normalised partial (bf16, as the output is) and its log2-sum-exp in slot
 // part.  The O rows go through LDS `stage` (kQSlot<G> bytes: the q slot of
@@ -642,16 +692,19 @@ XV_INLINE void finish_segment(const DecodeArgs& a, const SplitState& st, int b, 
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_wave_barrier();
   };
+  auto write_row = [&](uint16_t* s16, int row, int RR) {
+    float v[8];
+#pragma unroll
+    for (int nn = 0; nn < 8; ++nn) v[nn] = st.o[nn][RR] * inv[RR];
+    stage_write_row(s16 + row * kD + i, v);
+  };
   const int head0 = kvh * G;
   if (full) {
     uint16_t* s16 = reinterpret_cast<uint16_t*>(stage);  // row r (head head0 + r) at r * 256 B
 #pragma unroll
     for (int RR = 0; RR < 4; ++RR) {
       const int row = 4 * g + RR;
-      if (row < G) {
-#pragma unroll
-        for (int nn = 0; nn < 8; ++nn) s16[row * kD + 16 * nn + i] = (uint16_t)f32_to_bf16(st.o[nn][RR] * inv[RR]);
-      }
+      if (row < G) write_row(s16, row, RR);
     }
     wave_sync();
     // the G heads' rows are contiguous in the output row of sequence b
@@ -660,7 +713,7 @@ XV_INLINE void finish_segment(const DecodeArgs& a, const SplitState& st, int b, 
 #pragma unroll
     for (int k = 0; k < (kBytes + 1023) / 1024; ++k) {
       const int off = 1024 * k + 16 * lane;
-      if (off < kBytes) *reinterpret_cast<uint4*>(dst + off) = *reinterpret_cast<const uint4*>(stage + off);
+      if (off < kBytes) *reinterpret_cast<uint4*>(dst + off) = stage_read16(stage + off);
     }
     return;
   }
@@ -671,10 +724,7 @@ XV_INLINE void finish_segment(const DecodeArgs& a, const SplitState& st, int b, 
 #pragma unroll
   for (int RR = 0; RR < 4; ++RR) {
     const int row = 4 * g + RR;
-    if (row < G) {
-#pragma unroll
-      for (int nn = 0; nn < 8; ++nn) s16[row * kD + 16 * nn + i] = (uint16_t)f32_to_bf16(st.o[nn][RR] * inv[RR]);
-    }
+    if (row < G) write_row(s16, row, RR);
   }
   wave_sync();
   {
@@ -685,7 +735,7 @@ XV_INLINE void finish_segment(const DecodeArgs& a, const SplitState& st, int b, 
       if (off < kBytes) {
         const int r = off / (kD * 2), w = off % (kD * 2);
         char* dst = reinterpret_cast<char*>(a.ws_ob + (wrow0 + (int64_t)r * a.max_parts) * kD) + w;
-        *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(stage + off);
+        *reinterpret_cast<uint4*>(dst) = stage_read16(stage + off);
       }
     }
   }
@@ -693,10 +743,10 @@ XV_INLINE void finish_segment(const DecodeArgs& a, const SplitState& st, int b, 
 #pragma unroll
   for (int RR = 0; RR < 4; ++RR) {
     const int row = 4 * g + RR;
-    if (i == 0 && row < G) s32[row] = lse[RR];
+    if (i == 0 && row < G) stage_write4(s32 + row, lse[RR]);
   }
   wave_sync();
-  if (lane < G) a.ws_lse[wrow0 + (int64_t)lane * a.max_parts] = s32[lane];
+  if (lane < G) a.ws_lse[wrow0 + (int64_t)lane * a.max_parts] = stage_read4(s32 + lane);
 }
 
 XV_INLINE void reset(SplitState& st) {
@@ -788,7 +838,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F8 ? XV_F8_W
   constexpr int QOFF = kPageBufBytes<G, F8>;  // the q slot within a page buffer
   __shared__ __attribute__((aligned(16))) char lds[NB * BUF];
   __shared__ int pref[kMaxBatch + 1];  // pages of sequences 0..b-1
-  __shared__ int sl[kMaxBatch];        // cache_seqlens
+  __shared__ int sl[kMaxBatch];        // cache_seqlens (kCtxMask)
   __shared__ __attribute__((aligned(16))) char idtab[2 * kIdWindow * 4];
   const int lane = threadIdx.x;
   // prefix sums of the page counts (every wave computes them)
@@ -796,6 +846,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F8 ? XV_F8_W
   for (int c = 0; c < a.batch; c += 64) {
     const int b = c + lane;
     const int ctx = b < a.batch ? max(a.seqlens[b], 0) : 0;
+    const bool pre = a.pre_tokens != nullptr && b < a.batch && a.pre_tokens[b] > 0;
     const int np = (ctx + kPage - 1) / kPage;
     max_np = max(max_np, np);
     int inc = np;
@@ -808,7 +859,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F8 ? XV_F8_W
     inc += __builtin_amdgcn_update_dpp(0, inc, 0x143, 0xc, 0xf, true);  // row_bcast:31 into rows 2, 3
     if (b < a.batch) {
       pref[b + 1] = carry + inc;
-      sl[b] = ctx;
+      sl[b] = pre ? ctx | ~kCtxMask : ctx;
     }
     carry += __builtin_amdgcn_readlane(inc, 63);
   }
@@ -826,7 +877,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F8 ? XV_F8_W
   Cursor c0;
   c0.b = __builtin_amdgcn_readfirstlane(seq_of(pref, a.batch, a.hkv, f0));
   c0.npb = __builtin_amdgcn_readfirstlane(pref[c0.b + 1] - pref[c0.b]);
-  c0.ctx = __builtin_amdgcn_readfirstlane(sl[c0.b]);
+  c0.ctx = __builtin_amdgcn_readfirstlane(sl[c0.b]) & kCtxMask;
   {
     const int r = (int)(f0 - (int64_t)a.hkv * pref[c0.b]);
     c0.kvh = __builtin_amdgcn_readfirstlane(r / c0.npb);
@@ -865,7 +916,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(F8 ? XV_F8_W
   auto finish = [&](const Cursor& c, char* stage) {
     const int64_t seg0 = (int64_t)a.hkv * pref[c.b] + (int64_t)c.kvh * c.npb;
     // a row with a shared prefix always leaves a partial: the merge combines it with the prefix pass's
-    const bool pre = a.pre_tokens != nullptr && __builtin_amdgcn_readfirstlane(a.pre_tokens[c.b]) > 0;
+    const bool pre = __builtin_amdgcn_readfirstlane(sl[c.b]) < 0;
     const bool full = seg0 >= f0 && seg0 + c.npb <= f0 + n && !pre;
     const int part = (int)(blockIdx.x - seg0 / L);
     finish_segment<G>(a, st, c.b, c.kvh, full, part, lane, stage);
