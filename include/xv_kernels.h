@@ -355,6 +355,23 @@ int xv_qk_norm_rope_store_fp8(const void* q, int64_t q_stride_tok, int64_t q_str
                               hipStream_t stream);
 
 /*
+ * xv_qk_norm_rope_store (or, with fp8 nonzero, xv_qk_norm_rope_store_fp8) whose
+ * q, k and v are the fp32 partial sums of a split-K qkv GEMM, as
+ * xv_stream_gemm leaves them: head h of token t (q heads, then k, then v) is
+ * bf16(sum_p parts[p]), part p at parts + p * part_stride + t * row_stride +
+ * h * head_dim (floats, strides multiples of 4); 1 <= num_parts <= 8.  The
+ * results equal those of the bf16 sum through that entry point.
+ */
+int xv_qk_norm_rope_store_parts(const float* parts, int64_t part_stride, int64_t row_stride, int num_parts,
+                                const void* q_weight, const void* k_weight, float eps,
+                                const int64_t* positions, const float* cos_sin_cache, void* q_out,
+                                void* k_cache, void* v_cache, int64_t cache_page_stride,
+                                int64_t cache_tok_stride, int64_t cache_head_stride, int block_size,
+                                const int32_t* slot_mapping, int64_t num_tokens, int num_q_heads,
+                                int num_kv_heads, int head_dim, int fp8, float k_scale, float v_scale,
+                                hipStream_t stream);
+
+/*
  * SiLU-and-mul.
  * Replaces vllm::silu_and_mul, src/compute/layers/ops.py:20-23 (gate first, up second).
  *   out[t, i] = silu(x[t, i]) * x[t, I + i]

@@ -1,0 +1,74 @@
+"""q/k norm + RoPE + KV store from split-K partial sums: bit-equal to the same
+kernel on the bf16 sum of the partials (part 0 first, rounded once), bf16 and
+fp8 caches of both page orders and block sizes, skipped slots, one to eight
+parts, padded strides; bad arguments raise."""
+import pytest
+import torch
+
+import xvllm.layers.ops  # noqa: F401  (registers the xv:: ops)
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _cache(dev, blocks, bs, hkv, hnd, dtype):
+    shape = (2, blocks, hkv, bs, D) if hnd else (2, blocks, bs, hkv, D)
+    c = torch.zeros(shape, device=dev, dtype=torch.bfloat16).to(dtype)
+    return c.transpose(2, 3) if hnd else c
+
+
+@pytest.mark.parametrize("tokens,parts,hq,hkv,bs,hnd,fp8", [
+    (1, 1, 16, 8, 16, True, False), (7, 8, 16, 8, 16, False, False), (64, 4, 32, 8, 16, True, True),
+    (33, 2, 64, 8, 256, True, False), (5, 3, 8, 8, 256, False, True), (200, 4, 32, 8, 16, True, False)])
+def test_equals_the_store_on_the_sum(dev, tokens, parts, hq, hkv, bs, hnd, fp8):
+    print(f"rope parts T {tokens} P {parts} heads {hq}/{hkv} block {bs} hnd {hnd} fp8 {fp8}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(tokens * 10 + parts)
+    width = (hq + 2 * hkv) * D
+    buf = torch.randn((parts, tokens, width + 8), generator=g, device=dev) * 0.7
+    p = buf[:, :, :width]
+    acc = p[0].clone()
+    for i in range(1, parts):
+        acc += p[i]
+    qkv = acc.to(torch.bfloat16)
+    qw = (1 + 0.1 * torch.randn(D, generator=g, device=dev)).to(torch.bfloat16)
+    kw = (1 + 0.1 * torch.randn(D, generator=g, device=dev)).to(torch.bfloat16)
+    pos = torch.randint(0, 512, (tokens,), generator=g, device=dev)
+    cs = torch.randn((512, D), generator=g, device=dev)
+    blocks = tokens // bs + 3
+    slots = torch.randperm(blocks * bs, generator=g, device=dev)[:tokens].to(torch.int32)
+    if tokens > 2:
+        slots[1] = -1
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    ca, cb = _cache(dev, blocks, bs, hkv, hnd, dt), _cache(dev, blocks, bs, hkv, hnd, dt)
+    scales = (0.03, 0.05) if fp8 else (1.0, 1.0)
+    q = qkv[:, : hq * D].view(tokens, hq, D)
+    k = qkv[:, hq * D : (hq + hkv) * D].view(tokens, hkv, D)
+    v = qkv[:, (hq + hkv) * D :].view(tokens, hkv, D)
+    want = torch.ops.xv.qk_norm_rope_store(q, k, v, qw, kw, 1e-6, pos, cs, ca[0], ca[1], slots, *scales)
+    got = torch.ops.xv.qk_norm_rope_store_parts(p, hq, qw, kw, 1e-6, pos, cs, cb[0], cb[1], slots, *scales)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert torch.equal(ca.contiguous().view(torch.uint8), cb.contiguous().view(torch.uint8))
+    assert got.abs().sum() > 0 and ca.contiguous().view(torch.uint8).any()
+
+
+def test_rejects_bad_arguments(dev):
+    hq, hkv = 16, 8
+    ones = torch.ones(D, dtype=torch.bfloat16, device=dev)
+    cache = _cache(dev, 2, 16, hkv, False, torch.bfloat16)
+    pos, cs = torch.zeros(3, dtype=torch.int64, device=dev), torch.zeros((4, D), device=dev)
+    slots = torch.zeros(3, dtype=torch.int32, device=dev)
+
+    def call(parts, slots=slots, cache=cache, scale=1.0):
+        return torch.ops.xv.qk_norm_rope_store_parts(parts, hq, ones, ones, 1e-6, pos, cs, cache[0], cache[1], slots,
+                                                     scale, 1.0)
+
+    good = torch.zeros((2, 3, (hq + 2 * hkv) * D), device=dev)
+    call(good)
+    for bad in (good.to(torch.bfloat16), good[0], good[:, :, : hq * D], good[:, :2]):
+        with pytest.raises(ValueError):
+            call(bad)
+    with pytest.raises(RuntimeError):  # nine partials
+        call(torch.zeros((9, 3, (hq + 2 * hkv) * D), device=dev))
+    with pytest.raises(RuntimeError):  # a zero fp8 scale
+        call(good, cache=_cache(dev, 2, 16, hkv, False, torch.float8_e4m3fn), scale=0.0)

@@ -779,6 +779,118 @@ extern "C" int xv_qk_norm_rope_store_fp8(const void* q, int64_t q_stride_tok, in
                                          num_q_heads, num_kv_heads, cd, stream);
 }
 
+// The same from the fp32 partial sums of a split-K qkv GEMM (part p of token t
+// at parts + p * part_stride + t * row_stride, its q, k and v heads in that
+// order): x = bf16(sum of parts), the value the unsplit GEMM would have
+// written, then exactly the rope_kernel arithmetic.  A decode batch has few
+// tokens, so what bounds it is the chain of loads (position, then its table
+// row) and not bytes: one 16-lane row per head instead of rope_kernel's wave per
+// token puts every head's loads in flight at once (Qwen3-8B, 64 rows, 4 parts:
+// 5.6 us against 5.7 for rope_kernel on the bf16 product, 4x fewer bytes).
+template <bool F8>
+__global__ __launch_bounds__(256) void rope_store_parts_kernel(
+    const float* __restrict__ parts, int64_t part_stride, int64_t row_stride, int np, const bf16_t* __restrict__ qw,
+    const bf16_t* __restrict__ kw, float eps, const int64_t* __restrict__ positions,
+    const float* __restrict__ cos_sin, bf16_t* __restrict__ q_out, int64_t num_tokens, int hq, int hkv, CacheDst cd) {
+  constexpr int D = 128;
+  const int heads = hq + 2 * hkv;
+  const int64_t id = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int64_t tok = id / heads;
+  if (tok >= num_tokens) return;
+  const int h = (int)(id - tok * heads), lane = threadIdx.x & 15;
+  const float* src = parts + tok * row_stride + h * D + lane * 8;
+  floatx4_t lo[kMaxParts], hi[kMaxParts];
+#pragma unroll
+  for (int p = 0; p < kMaxParts; ++p) {
+    if (p < np) {
+      const floatx4_t* v = reinterpret_cast<const floatx4_t*>(src + p * part_stride);
+      lo[p] = __builtin_nontemporal_load(v);
+      hi[p] = __builtin_nontemporal_load(v + 1);
+    }
+  }
+  const int32_t slot = h < hq ? 0 : cd.slots[tok];
+  const int page = slot / cd.block_size, t = slot - page * cd.block_size;
+  const int64_t cache_off = (int64_t)page * cd.ps + (int64_t)t * cd.ts + lane * 8;
+  const bool rotate = h < hq + hkv;
+  float c[8], sn[8], w[8];
+  if (rotate) {
+    const float* cs = cos_sin + positions[tok] * D + (lane & 7) * 8;
+    *reinterpret_cast<float4*>(c) = *reinterpret_cast<const float4*>(cs);
+    *reinterpret_cast<float4*>(c + 4) = *reinterpret_cast<const float4*>(cs + 4);
+    *reinterpret_cast<float4*>(sn) = *reinterpret_cast<const float4*>(cs + D / 2);
+    *reinterpret_cast<float4*>(sn + 4) = *reinterpret_cast<const float4*>(cs + D / 2 + 4);
+    unpack8(load_vec8((h < hq ? qw : kw) + lane * 8), w);
+  }
+  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < kMaxParts; ++p) {
+    if (p < np) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { a[e] += lo[p][e]; a[4 + e] += hi[p][e]; }
+    }
+  }
+  Vec8 out = pack8(a);  // the GEMM output's bf16 rounding
+  if (rotate) {
+    float x[8], r[8];
+    unpack8(out, x);
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+    ss = row16_sum(ss);
+    const float rcp = rsqrtf(ss / (float)D + eps);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = bf16_to_f32(f32_to_bf16((x[e] * rcp) * w[e]));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float partner = dpp_f<0x128>(x[e]);  // row_ror:8 -> lane j^8
+      r[e] = lane < 8 ? x[e] * c[e] - partner * sn[e] : x[e] * c[e] + partner * sn[e];
+    }
+    out = pack8(r);
+  }
+  if (h < hq) {
+    store_vec8_nt(q_out + (tok * hq + h) * D + lane * 8, out);
+  } else if (slot >= 0) {
+    const bool is_k = h < hq + hkv;
+    const int64_t off = cache_off + (int64_t)(h - hq - (is_k ? 0 : hkv)) * cd.hs;
+    bf16_t* dst = is_k ? cd.kc : cd.vc;
+    if constexpr (F8) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(dst) + off) = vec8_to_fp8(out, is_k ? cd.k_inv : cd.v_inv);
+    else store_vec8_nt(dst + off, out);
+  }
+}
+
+extern "C" int xv_qk_norm_rope_store_parts(const float* parts, int64_t part_stride, int64_t row_stride, int num_parts,
+                                           const void* q_weight, const void* k_weight, float eps,
+                                           const int64_t* positions, const float* cos_sin_cache, void* q_out,
+                                           void* k_cache, void* v_cache, int64_t cache_page_stride,
+                                           int64_t cache_tok_stride, int64_t cache_head_stride, int block_size,
+                                           const int32_t* slot_mapping, int64_t num_tokens, int num_q_heads,
+                                           int num_kv_heads, int head_dim, int fp8, float k_scale, float v_scale,
+                                           hipStream_t stream) {
+  if (head_dim != 128 || num_q_heads <= 0 || num_kv_heads <= 0 || num_tokens < 0 || block_size <= 0 ||
+      num_parts < 1 || num_parts > kMaxParts)
+    return (int)hipErrorInvalidValue;
+  if (fp8 && (!(k_scale > 0.0f) || !(v_scale > 0.0f) || !__builtin_isfinite(k_scale) || !__builtin_isfinite(v_scale)))
+    return (int)hipErrorInvalidValue;
+  if (!xv_al16(parts) || (part_stride | row_stride) & 3 || !xv_al16(q_weight) || !xv_al16(k_weight) ||
+      !xv_al16(cos_sin_cache) || !xv_al16(q_out) || !xv_al16(k_cache) || !xv_al16(v_cache) ||
+      !xv_st8(cache_page_stride) || !xv_st8(cache_tok_stride) || !xv_st8(cache_head_stride))
+    return (int)hipErrorInvalidValue;
+  if (num_tokens == 0) return 0;
+  CacheDst cd = {};
+  cd.kc = (bf16_t*)k_cache; cd.vc = (bf16_t*)v_cache;
+  cd.ps = cache_page_stride; cd.ts = cache_tok_stride; cd.hs = cache_head_stride; cd.block_size = block_size;
+  cd.slots = slot_mapping;
+  cd.k_inv = 1.0f / k_scale; cd.v_inv = 1.0f / v_scale;
+  const int64_t blocks = (num_tokens * (num_q_heads + 2 * num_kv_heads) + 15) / 16;
+  if (blocks > INT32_MAX) return (int)hipErrorInvalidValue;
+  auto kernel = fp8 ? rope_store_parts_kernel<true> : rope_store_parts_kernel<false>;
+  kernel<<<(unsigned)blocks, 256, 0, stream>>>(parts, part_stride, row_stride, num_parts, (const bf16_t*)q_weight,
+                                               (const bf16_t*)k_weight, eps, positions, cos_sin_cache, (bf16_t*)q_out,
+                                               num_tokens, num_q_heads, num_kv_heads, cd);
+  XV_CHECK_LAUNCH();
+  return 0;
+}
+
 extern "C" int xv_rotary_embedding(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
                                    const void* k, int64_t k_stride_tok, int64_t k_stride_head,
                                    const int64_t* positions, const float* cos_sin_cache,

@@ -1,7 +1,8 @@
 """Dense GEMMs of the decoder: up to 256 rows the gfx950 kernel that streams
 the [N, K] weight in place (xv_stream_gemm: gate_up fused with SiLU-and-mul,
 down and o as split-K partials for the norm that follows them, reference
-src/compute/models/qwen3.py:64,115 feeding the norms of :150,:152), above that
+src/compute/models/qwen3.py:64,115 feeding the norms of :150,:152, a decode
+batch's qkv as partials for its norm + RoPE + KV store), above that
 and for shapes it does not take PyTorch (hipBLASLt) with a split-K form for the
 latter two.  pack_weight / dense_gemm are the older streamed form over packed
 weight tiles (at most 64 rows), kept where the in-place kernel does not take
@@ -13,6 +14,7 @@ its SiLU; MI355X, graph replay, over 1 GB of weights cycled):
     Qwen3-8B    gate_up  M 8: 46.5 -> 31.0   M 64: 47.8 -> 34.6   M 200: 64.5 -> 54.9
                 down     M 8: 22.1 -> 18.1   M 64: 23.6 -> 20.1   M 200: 34.6 -> 31.7
                 o        M 8: 10.3 -> 8.0    M 64: 14.8 -> 9.6    M 200: 18.1 -> 16.6
+                qkv      M 8: 15.7 -> 11.3   M 64: 18.0 -> 11.9   M 200: 26.8 -> 21.1 (4 partial sums)
     Qwen3-0.6B  gate_up  M 8: 10.3 -> 5.1    down M 8: 12.1 -> 4.0   o M 8: 9.7 -> 3.4
 
 The split-K measurements below are the hipBLASLt path.
@@ -38,13 +40,10 @@ served from the 256 MB last-level cache; us, unsplit -> split):
     o_proj     M 1, 8: 15.3 -> 10.1 (P 4)  M 128: 24.2 -> 15.6 (P 8)
                M 32, 64, 256: gains below the partials' extra reads
 
-The other two GEMMs stay unsplit (same measurement, bmm over the same views):
+On hipBLASLt gate_up stays unsplit (same measurement, bmm over the same views):
 gate_up (K 4096, N 24576) M 32-128: 45-51 unsplit, no split faster; M 256:
 65.5 -> 59.6 (P 2), less than its 50 MB of fp32 partials cost to write and
-read back.  qkv (N 6144) M 64: 17.5 -> 15.4 (P 4), M 128: 25.0 -> 17.7,
-M 256: 39.3 -> 23.1; its consumer is the fused q/k-norm + RoPE + KV-store
-kernel, which would need a partial-summing form for gains of a few us per
-layer at the largest serving batches.
+read back.
 """
 from __future__ import annotations
 
@@ -275,14 +274,14 @@ def _stream_gemm_fake(x, w, mode, parts):
     return x.new_empty((m, n // 2))
 
 
-def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int):
+def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int, *, internal: bool = False):
     """What streamed_silu_mul / streamed_into_norm read the weight w [N, K]
     from for activations x: w itself where the in-place kernel takes the
     shape, else its packed copy (if it has one) up to STREAM_MAX_ROWS rows,
     else None (the library GEMM).  `packed` is the operand a packed model
     holds, None for a model that was not packed.  Such a model's callers get
     PartialSums only where linear_into_norm splits, so its products into a
-    norm stream only there; and with gradients asked of x or w the library
+    norm stream only there (unless they stay `internal` to the layer); and with gradients asked of x or w the library
     keeps the product (streaming has no backward; a packed model is inference
     only)."""
     if not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2:
@@ -290,7 +289,7 @@ def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int):
     m, k = x.shape
     n = w.shape[0]
     if packed is None:
-        if mode == GEMM_PARTS and split_factor(m, n, k) == 1:
+        if mode == GEMM_PARTS and not internal and split_factor(m, n, k) == 1:
             return None
         if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
             return None

@@ -268,3 +268,56 @@ def qk_norm_rope_store(
 def _qk_norm_rope_store_fake(q, k, v, q_weight, k_weight, eps, positions, cos_sin_cache, k_cache, v_cache,
                              slot_mapping, k_scale=1.0, v_scale=1.0):
     return torch.empty(q.shape, dtype=q.dtype, device=q.device)
+
+
+@torch.library.custom_op("xv::qk_norm_rope_store_parts", mutates_args=("k_cache", "v_cache"))
+def qk_norm_rope_store_parts(
+    parts: torch.Tensor,
+    num_q_heads: int,
+    q_weight: torch.Tensor,
+    k_weight: torch.Tensor,
+    eps: float,
+    positions: torch.Tensor,
+    cos_sin_cache: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    slot_mapping: torch.Tensor,
+    k_scale: float = 1.0,
+    v_scale: float = 1.0,
+) -> torch.Tensor:
+    """qk_norm_rope_store on the fp32 partial sums [P, T, (Hq + 2 Hkv) D] of a
+    split-K qkv GEMM: q, k and v are the heads of bf16(parts.sum(0))."""
+    require_cuda(parts, k_cache, v_cache, slot_mapping)
+    fp8 = k_cache.dtype == torch.float8_e4m3fn
+    require_bf16(q_weight, k_weight, *(() if fp8 else (k_cache, v_cache)))
+    if fp8 and v_cache.dtype != torch.float8_e4m3fn:
+        raise TypeError("k_cache and v_cache must share one dtype")
+    if parts.dtype != torch.float32 or parts.dim() != 3 or parts.stride(-1) != 1 or not aligned16(parts):
+        raise ValueError("qk_norm_rope_store_parts needs fp32 partial sums [P, T, (Hq + 2 Hkv) D], rows contiguous")
+    if cos_sin_cache.dtype != torch.float32:
+        raise TypeError("cos_sin_cache must be float32 (reference rotary.py:41-51)")
+    p, n, width = parts.shape
+    hkv, d = k_cache.shape[2], k_cache.shape[3]
+    if width != (num_q_heads + 2 * hkv) * d or slot_mapping.numel() != n or positions.numel() != n:
+        raise ValueError(f"shapes: parts {tuple(parts.shape)}, {num_q_heads} q heads, cache {tuple(k_cache.shape)}, "
+                         f"{slot_mapping.numel()} slots, {positions.numel()} positions")
+    ps, ts, hs, bs = _cache_strides(k_cache)
+    assert v_cache.stride() == k_cache.stride()
+    slots = slot_mapping.to(torch.int32).contiguous()
+    pos = positions.to(torch.int64).contiguous()
+    qo = torch.empty((n, num_q_heads, d), dtype=q_weight.dtype, device=parts.device)
+    _C.check(
+        _C.lib().xv_qk_norm_rope_store_parts(
+            ptr(parts), parts.stride(0), parts.stride(1), p, ptr(q_weight.contiguous()), ptr(k_weight.contiguous()),
+            float(eps), ptr(pos), ptr(cos_sin_cache.contiguous()), ptr(qo), ptr(k_cache), ptr(v_cache), ps, ts, hs, bs,
+            ptr(slots), n, num_q_heads, hkv, d, int(fp8), float(k_scale), float(v_scale), stream_of(parts),
+        ),
+        "xv_qk_norm_rope_store_parts",
+    )
+    return qo
+
+
+@qk_norm_rope_store_parts.register_fake
+def _qk_norm_rope_store_parts_fake(parts, num_q_heads, q_weight, k_weight, eps, positions, cos_sin_cache, k_cache,
+                                   v_cache, slot_mapping, k_scale=1.0, v_scale=1.0):
+    return q_weight.new_empty((parts.shape[1], num_q_heads, k_cache.shape[3]))

@@ -6,7 +6,8 @@ qkv GEMM, per-head q/k RMSNorm + NeoX RoPE (one kernel, `xv::qk_norm_rope`),
 `vllm::attention` (KV store + paged decode / prefill), o GEMM, fused add +
 RMSNorm, gate_up GEMM, SiLU-and-mul, down GEMM.  Batches of up to 256 rows
 stream gate_up (with the SiLU-and-mul), down and o in place (xv_stream_gemm),
-down and o as split-K partials into the next norm; larger ones and shapes
+down and o as split-K partials into the next norm, decode batches also qkv, as
+partials into the norm + RoPE + KV store kernel; larger ones and shapes
 that kernel does not take run on PyTorch (hipBLASLt).  Weights are plain
 tensors (random init for the benchmarks; the reference's checkpoint loader is
 out of scope).
@@ -113,13 +114,19 @@ class Qwen3Attention(nn.Module):
     def forward(self, positions, hidden, attn: AttnInputs):
         """qkv -> q/k norm + RoPE -> attention -> o GEMM (PartialSums when
         split along K, for post_attention_layernorm)."""
-        qkv = F.linear(hidden, self.qkv_proj)
-        if not attn.is_prefill:
+        w = None if attn.is_prefill or not self.split_k else stream_operand(hidden, self.qkv_proj, None, GEMM_PARTS,
+                                                                            internal=True)
+        if w is not None:
+            # decode: the qkv partial sums go into norm + RoPE + KV store (k and v reach attention through the cache)
+            q = self._norm_rope_store_parts(positions, streamed_into_norm(hidden, w).parts, attn.slot_mapping)
+            q = q.view(q.shape[0], self.q_size)
+            o = self.attn(q, q, q, attn._replace(slot_mapping=None))
+        elif not attn.is_prefill:
             # decode: norm + RoPE + KV store in one kernel, attention reads the cache
-            q, k, v = self._split_norm_rope_store(positions, qkv, attn.slot_mapping)
+            q, k, v = self._split_norm_rope_store(positions, F.linear(hidden, self.qkv_proj), attn.slot_mapping)
             o = self.attn(q.view(q.shape[0], self.q_size), k, v, attn._replace(slot_mapping=None))
         else:
-            q, k, v = self._split_norm_rope(positions, qkv)
+            q, k, v = self._split_norm_rope(positions, F.linear(hidden, self.qkv_proj))
             o = self.attn(q.view(q.shape[0], self.q_size), k, v, attn)
         if not self.split_k:
             return F.linear(o, self.o_proj)
@@ -151,6 +158,14 @@ class Qwen3Attention(nn.Module):
             k_cache, v_cache, slot_mapping, ks, vs,
         )
         return q, k, v
+
+    def _norm_rope_store_parts(self, positions, parts, slot_mapping):
+        k_cache, v_cache = kv_cache_of(self.attn.layer_id)
+        ks, vs = kv_scales()
+        return torch.ops.xv.qk_norm_rope_store_parts(
+            parts, self.num_heads, self.q_norm.weight, self.k_norm.weight, self.eps, positions,
+            self.rotary_emb.cos_sin_cache, k_cache, v_cache, slot_mapping, ks, vs,
+        )
 
     def _split_norm_rope(self, positions, qkv):
         """split -> per-head q/k RMSNorm -> RoPE (reference qwen3.py:117-128),
