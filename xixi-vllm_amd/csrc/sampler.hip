@@ -3,7 +3,7 @@
 // arithmetic below: one 1024-thread workgroup per row (sample_kernel), the
 // all-greedy argmax over several workgroups per row (greedy_segment_kernel),
 // the sampled path over several workgroups per row for batches of up to
-// kSegMaxBatch rows (seg_stats / seg_hist / row_finish), and for calls whose every
+// kSegMaxBatch rows (seg_count / row_count), and for calls whose every
 // top_k is at most 64 a two-launch top-k path (seg_topk / row_topk); all give
 // the same ids.
 //
@@ -105,11 +105,27 @@ XV_INLINE void load8(const bf16_t* row, int V, int base, bool vec_ok, uint32_t (
   }
 }
 
+// The same as packed words (two ids each, the lower in the low half): half the
+// registers while several vectors are in flight.
+XV_INLINE void load8_words(const bf16_t* row, int V, int base, bool vec_ok, uint32_t (&w)[4]) {
+  if (vec_ok && base + 8 <= V) {
+    const Vec8 v = load_vec8(row + base);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = v.w[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      w[k] = (base + 2 * k < V ? (uint32_t)row[base + 2 * k] : 0xffffu) |
+             (base + 2 * k + 1 < V ? (uint32_t)row[base + 2 * k + 1] : 0xffffu) << 16;
+  }
+}
+XV_INLINE uint32_t bits_of(const uint32_t (&w)[4], int k) { return (w[k >> 1] >> (16 * (k & 1))) & 0xffffu; }
+
 // Apply f(bits, id) to every id of this thread's contiguous range
 // [t*C, t*C + C), C a multiple of 8: chunks of kChunk 16-byte loads are issued
 // together, so a pass over the row costs a few memory round trips, not one
 // per vector.  Thread order is id order.
-constexpr int kChunk = 8;
+constexpr int kChunk = 4;  // 8 took more registers and no less time (600 rows, top-p: 643 against 605 us)
 XV_INLINE int range_len(int V) { return ((V + kThreads - 1) / kThreads + 7) / 8 * 8; }
 // Apply f(bits, id) to the ids of a coalesced, lane-interleaved layout: in
 // step c, vector v of thread t is id 8*((c*kChunk + v)*kThreads + t).  Ids
@@ -118,18 +134,18 @@ template <typename F>
 XV_INLINE void for_each_strided(const bf16_t* row, int V, bool vec_ok, F&& f) {
   const int nvec = (V + 7) / 8;
   for (int c = 0; c * kChunk * kThreads < nvec; ++c) {
-    uint32_t bits[kChunk][8];
+    uint32_t w[kChunk][4];
 #pragma unroll
     for (int v = 0; v < kChunk; ++v) {
       const int vi = (c * kChunk + v) * kThreads + threadIdx.x;
-      if (vi < nvec) load8(row, V, vi * 8, vec_ok, bits[v]);
+      if (vi < nvec) load8_words(row, V, vi * 8, vec_ok, w[v]);
     }
 #pragma unroll
     for (int v = 0; v < kChunk; ++v) {
       const int vi = (c * kChunk + v) * kThreads + threadIdx.x;
       if (vi < nvec)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) f(bits[v][k], vi * 8 + k);
+        for (int k = 0; k < 8; ++k) f(bits_of(w[v], k), vi * 8 + k);
     }
   }
 }
@@ -139,16 +155,16 @@ XV_INLINE void for_each_elem(const bf16_t* row, int V, bool vec_ok, F&& f) {
   const int C = range_len(V);
   const int i0 = threadIdx.x * C, i1 = min(V, i0 + C);
   for (int c = i0; c < i1; c += 8 * CH) {
-    uint32_t bits[CH][8];
+    uint32_t w[CH][4];
 #pragma unroll
     for (int v = 0; v < CH; ++v)
-      if (c + 8 * v < i1) load8(row, V, c + 8 * v, vec_ok, bits[v]);
+      if (c + 8 * v < i1) load8_words(row, V, c + 8 * v, vec_ok, w[v]);
 #pragma unroll
     for (int v = 0; v < CH; ++v)
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const int id = c + 8 * v + k;
-        if (id < i1) f(bits[v][k], id);
+        if (id < i1) f(bits_of(w[v], k), id);
       }
   }
 }
@@ -285,6 +301,20 @@ XV_INLINE int64_t wave_incl_scan_l(int64_t x) {
   return x;
 }
 
+template <int CTRL, int ROWS>
+XV_INLINE int dpp_scan_i(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, true);
+}
+XV_INLINE int wave_incl_scan_i(int x) {
+  x += dpp_scan_i<0x111, 0xf>(x);
+  x += dpp_scan_i<0x112, 0xf>(x);
+  x += dpp_scan_i<0x114, 0xf>(x);
+  x += dpp_scan_i<0x118, 0xf>(x);
+  x += dpp_scan_i<0x142, 0xa>(x);
+  x += dpp_scan_i<0x143, 0xc>(x);
+  return x;
+}
+
 XV_INLINE uint32_t block_max_u(Shared& s, uint32_t x) {
   x = wave_max_u(x);
   const int w = threadIdx.x >> 6;
@@ -341,32 +371,6 @@ XV_INLINE int64_t block_excl_scan(Shared& s, int64_t x, int64_t* total) {
   return before + inc - x;
 }
 
-// Two exclusive prefix sums over the block at once (one pair of barriers).
-XV_INLINE void block_excl_scan2(Shared& s, int64_t x, int64_t y, int64_t* ex, int64_t* ey, int64_t* tx,
-                                int64_t* ty) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t ix = wave_incl_scan_l(x), iy = wave_incl_scan_l(y);
-  __syncthreads();
-  if (lane == 63) {
-    s.red_l[w] = ix;
-    s.red_l2[w] = iy;
-  }
-  __syncthreads();
-  int64_t bx = 0, by = 0, sx = 0, sy = 0;
-  for (int i = 0; i < kWaves; ++i) {
-    if (i < w) {
-      bx += s.red_l[i];
-      by += s.red_l2[i];
-    }
-    sx += s.red_l[i];
-    sy += s.red_l2[i];
-  }
-  *ex = bx + ix - x;
-  *ey = by + iy - y;
-  *tx = sx;
-  *ty = sy;
-}
-
 struct Boundary {
   uint32_t key;  // kept: key > key, or key == key with tie index <= tie
   int64_t tie;   // kTieAll: every tie of `key` kept
@@ -378,7 +382,7 @@ XV_INLINE bool earlier(const Boundary& a, const Boundary& b) {
 // Call f(bits, id) for every slot of a lane-interleaved layout like that of
 // for_each_strided (kChunkAll vectors per step) on every lane of every wave: slots at or past V come as
 // 0xffff (key 0), so f may use wave-wide operations.
-constexpr int kChunkAll = 8;
+constexpr int kChunkAll = 2;  // few registers: see row_count_kernel
 template <typename F>
 XV_INLINE void for_each_strided_all(const bf16_t* row, int V, bool vec_ok, F&& f) {
   const int nvec = (V + 7) / 8;
@@ -1202,28 +1206,26 @@ __global__ __launch_bounds__(kGreedyThreads) void greedy_segment_kernel(const bf
 // ---------------------------------------------------------------------------
 // Sampled rows over several workgroups per row (batches given a workspace).
 //
-// A row is cut into R segments of whole 8-id vectors, one kSegThreads
-// workgroup each, and the one-workgroup algorithm above runs as three
-// launches (a launch boundary makes one kernel's global writes visible to the
-// next, across XCDs):
-//   1. seg_stats:  per segment, the largest and smallest key and the greedy best;
-//   2. seg_hist:   per segment, bucket counts and masses, the min-p key, and the
-//                  segment's total mass (its kept mass when the row has no cut);
-//   3. row_finish: per row, one 1024-thread workgroup: the summed histograms
-//                  give the bucket(s) holding the cut-offs (greedy and all-NaN
-//                  rows finish here); the workgroup gathers those buckets'
-//                  candidates from the row into LDS, makes the exact cut (by
-//                  per-key counts, or a sort) and the kept mass (top-k rows
-//                  draw from the list and finish), then draws: the segment
-//                  holding floor(u * M), then the id in it.  A row whose
-//                  buckets hold more candidates than LDS runs sample_row.
-//                  Each segment's kept mass follows without another pass over
-//                  the logits: its masses of the buckets before the cut's
-//                  bucket (every candidate there is kept) plus its candidates
-//                  up to the cut (exact integer sums of the same per-candidate
-//                  masses).
-// Buckets, masses, cuts and the draw are those of the one-workgroup path, so
-// the ids are identical to it.
+// A candidate's mass depends on its bf16 key alone, so exact counts per key
+// replace per-id masses: the row is cut into R segments of whole 8-id vectors
+// and two launches sample it (a launch boundary makes one kernel's global
+// writes visible to the next, across XCDs):
+//   1. seg_count:  one workgroup per segment counts its logits by value: the
+//                  8192 keys of magnitudes in [2^-22, 2^10) exactly, zeros,
+//                  smaller magnitudes (listed), larger ones; greedy rows take
+//                  the segment's best instead;
+//   2. row_count:  one workgroup per row sums the segments' counts, evaluates
+//                  one exp2 per key, cuts by ranks and masses over the keys,
+//                  takes each segment's kept mass from its own counts, and
+//                  draws: the segment holding floor(u * M), then the id in it.
+// The masses and their sums are exact integers, so cuts and draws are those
+// of the one-workgroup path and the ids are identical to it.
+// Top-p 0.95 at V 151936, 32 rows: 7 + 16 us, 27.9 us a call with its gaps.
+// Three launches (row extremes, 256-bucket mass histograms, one workgroup per
+// row gathering the cut's bucket from the whole row) took 4.7 + 13.1 + 35.6,
+// 58.6 a call; 52.3 -> 20.9 us a call in a captured loop, 1 row 42.0 -> 18.0,
+// 512 rows 224 -> 80, and rows whose cut bucket overflowed LDS (a spread of
+// 2.5 at 256 rows) 861 -> 42.
 
 constexpr int kSegThreads = 256;
 constexpr int kSegWaves = kSegThreads / 64;
@@ -1233,29 +1235,19 @@ constexpr int kSegWaves = kSegThreads / 64;
 #ifndef XV_SEG_CHUNK
 #define XV_SEG_CHUNK 4
 #endif
-#ifndef XV_SEG_TARGET
-#define XV_SEG_TARGET 2048
-#endif
 constexpr int kMaxSegs = XV_SEG_MAX;
 constexpr int kSegChunk = XV_SEG_CHUNK;
 // Rows of the multi-workgroup sampled path; larger batches take one workgroup
-// per row.  Up to 512 rows the path measured faster than one workgroup per row
-// (top-p 0.9 at V 151936: 103 against 233 us at 192 rows, 241 against 465 at
-// 512; its workspace holds kMaxCand candidates per row, 64 KB).
+// per row (top-p at V 151936: 80 us at 512 rows, 605 at 600), since the
+// workspace of a batch reserves 64 KB and more per row.
 constexpr int kSegMaxBatch = 512;
-
-enum : int { kPlanDone = 0, kPlanGather = 1, kPlanDraw = 2, kPlanFallback = 3 };
-
-struct __attribute__((aligned(128))) RowPlan {
-  int status;
-  int use_k;           // the list is the top-k candidates (draw from the list)
-  int cut_p, cut_m;    // the top-p / min-p cut falls in the gathered bucket
-  uint32_t kminp;      // min-p key (0xffffffff: none)
-  uint32_t key_cut;
-  uint32_t klo, khi;   // keys of buckets lo..hi: exactly [klo, khi]
-  float zmax, inv_t;
-  int64_t thr, mp_before, m_before, id_cut, M;
-};
+// Segments per row of the counting path: more split the counting and the draw
+// further, but the row's workgroup reads 16 KB of counts for each (32 rows of
+// 151936: 4 segments 23.2 us, 8 20.7, 12 24.0, 16 24.4).  Large batches take
+// fewer, about kCntTarget workgroups in all (256 rows: 512 workgroups 42.4,
+// 1024 41.4, 2048 42.8).
+constexpr int kCntSegs = 8;
+constexpr int kCntTarget = 1024;
 
 struct SegArgs {
   const bf16_t* logits;
@@ -1267,15 +1259,10 @@ struct SegArgs {
   const float* min_ps;
   const float* uniforms;
   int64_t* out_ids;
-  uint32_t* seg_kmax;           // [B * R]
-  uint32_t* seg_kmin;           // [B * R]
-  uint32_t* seg_minp;           // [B * R]
   unsigned long long* seg_best; // [B * R] greedy (key << 32 | ~id)
-  int64_t* seg_kept;            // [B * R]
-  uint32_t* seg_cnt;            // [B * R * kBuckets]
-  unsigned long long* seg_mass; // [B * R * kBuckets]
-  unsigned long long* cand;     // [B * cand_stride]
-  int64_t cand_stride;          // candidates per row: kMaxCand, or R * kTopList on the top-k path
+  uint32_t* seg_cnt;            // [B * R * kSegWords]
+  unsigned long long* cand;     // top-k path: [B * cand_stride]
+  int64_t cand_stride;          // R * kTopList
 };
 
 struct RowParams {
@@ -1301,145 +1288,56 @@ XV_INLINE RowParams row_params(const SegArgs& a, int b) {
 }
 
 // f(bits, id) for every id of segment [beg, end) on every lane: vector vi of
-// the segment is (c * kSegChunk + v) * kSegThreads + t; ids ascend within a
-// lane; slots outside the segment come as 0xffff (key 0).
+// the segment is (c * kSegChunk + v) * kThreads + t; ids ascend within a lane;
+// slots of the last vector outside the segment come as 0xffff (key 0).
 template <typename F>
-XV_INLINE void for_seg_chunks(const bf16_t* row, bool vec_ok, int beg, int end, F&& f) {
+XV_INLINE void for_seg(const bf16_t* row, bool vec_ok, int beg, int end, F&& f) {
   const int nvec = (end - beg + 7) / 8;
-  for (int c = 0; c * kSegChunk * kSegThreads < nvec; ++c) {
+  for (int c = 0; c * kSegChunk * kThreads < nvec; ++c) {
     uint32_t w[kSegChunk][4];
 #pragma unroll
     for (int v = 0; v < kSegChunk; ++v) {
-      const int base = beg + ((c * kSegChunk + v) * kSegThreads + (int)threadIdx.x) * 8;
-      if (vec_ok && base + 8 <= end) {
-        const Vec8 x = load_vec8(row + base);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) w[v][k] = x.w[k];
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          w[v][k] = (base + 2 * k < end ? (uint32_t)row[base + 2 * k] : 0xffffu) |
-                    (base + 2 * k + 1 < end ? (uint32_t)row[base + 2 * k + 1] : 0xffffu) << 16;
-      }
+      const int base = beg + ((c * kSegChunk + v) * kThreads + (int)threadIdx.x) * 8;
+      if (base < end) load8_words(row, end, base, vec_ok, w[v]);
     }
-    f(w, c);
-  }
-}
-template <typename F>
-XV_INLINE void for_seg(const bf16_t* row, bool vec_ok, int beg, int end, F&& f) {
-  for_seg_chunks(row, vec_ok, beg, end, [&](const uint32_t (&w)[kSegChunk][4], int c) {
 #pragma unroll
     for (int v = 0; v < kSegChunk; ++v) {
-      const int base = beg + ((c * kSegChunk + v) * kSegThreads + (int)threadIdx.x) * 8;
+      const int base = beg + ((c * kSegChunk + v) * kThreads + (int)threadIdx.x) * 8;
+      if (base < end)
 #pragma unroll
-      for (int k = 0; k < 8; ++k) f((w[v][k >> 1] >> (16 * (k & 1))) & 0xffffu, base + k);
+        for (int k = 0; k < 8; ++k) f(bits_of(w[v], k), base + k);
     }
-  });
+  }
 }
 
-// f(word) for every 32-bit word (two ids, the lower in the low half) of the
-// segment's vectors, in for_seg's order; slots outside the segment come as
-// 0xffff halves.
-template <typename F>
-XV_INLINE void for_seg_words(const bf16_t* row, bool vec_ok, int beg, int end, F&& f) {
-  for_seg_chunks(row, vec_ok, beg, end, [&](const uint32_t (&w)[kSegChunk][4], int) {
-#pragma unroll
-    for (int v = 0; v < kSegChunk; ++v)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) f(w[v][k]);
-  });
+// A segment's counts in the workspace: kSegWords words, the 16-bit counts of
+// the 2 * kMagBins window keys in descending order (position pos < kMagBins:
+// the positive magnitude kMagLo + kMagBins - 1 - pos, past it the negative one
+// kMagLo + pos - kMagBins; two to a word), then the header, then up to
+// kTinyList 16-bit logits of magnitudes in (0, 2^-22).
+constexpr int kMagBins = 4096;                  // 32 octaves of 128 bf16 magnitudes
+constexpr uint32_t kMagLo = (127 - 22) << 7;    // 2^-22; the window ends at 2^10
+constexpr uint32_t kInfMag = 0x7f80u;
+constexpr int kTinyList = 64;
+constexpr int kMaxSegIds = 65528;               // a count fits 16 bits
+// header words; kHFarMag and kHFirst hold 0xffff - value (a cleared word is "none")
+enum : int { kHPosZero = 0, kHNegZero, kHFar, kHFarMag, kHTop, kHTiny, kHFirst, kHWords = 8 };
+constexpr int kSegWords = (kMagBins + kHWords + kTinyList / 2 + 63) / 64 * 64;
+// Window position of raw bits with m = magnitude - kMagLo < kMagBins, and back.
+XV_INLINE uint32_t window_pos(uint32_t bits, uint32_t m) {
+  return (bits & 0x8000u) ? (uint32_t)kMagBins + m : (uint32_t)(kMagBins - 1) - m;
+}
+XV_INLINE uint32_t pos_bits(int pos) {
+  return pos < kMagBins ? kMagLo + (uint32_t)(kMagBins - 1 - pos) : 0x8000u | (kMagLo + (uint32_t)(pos - kMagBins));
 }
 
-struct SegRed {
-  unsigned long long u[kSegWaves];
-  int64_t l[kSegWaves];
-};
-XV_INLINE uint32_t seg_max_u(SegRed& r, uint32_t x) {
-  x = wave_max_u(x);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) r.u[threadIdx.x >> 6] = x;
-  __syncthreads();
-  uint32_t m = (uint32_t)r.u[0];
-  for (int i = 1; i < kSegWaves; ++i) m = max(m, (uint32_t)r.u[i]);
-  return m;
-}
-XV_INLINE uint32_t seg_min_u(SegRed& r, uint32_t x) {
-  x = wave_min_u(x);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) r.u[threadIdx.x >> 6] = x;
-  __syncthreads();
-  uint32_t m = (uint32_t)r.u[0];
-  for (int i = 1; i < kSegWaves; ++i) m = min(m, (uint32_t)r.u[i]);
-  return m;
-}
-XV_INLINE unsigned long long seg_max_ull(SegRed& r, unsigned long long x) {
-  x = wave_max_ull(x);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) r.u[threadIdx.x >> 6] = x;
-  __syncthreads();
-  unsigned long long m = r.u[0];
-  for (int i = 1; i < kSegWaves; ++i) m = r.u[i] > m ? r.u[i] : m;
-  return m;
-}
-XV_INLINE int64_t seg_sum_l(SegRed& r, int64_t x) {
-  x = wave_sum_l(x);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) r.l[threadIdx.x >> 6] = x;
-  __syncthreads();
-  int64_t m = 0;
-  for (int i = 0; i < kSegWaves; ++i) m += r.l[i];
-  return m;
-}
-XV_INLINE int64_t seg_min_l(SegRed& r, int64_t x) {
-  x = wave_min_l(x);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) r.l[threadIdx.x >> 6] = x;
-  __syncthreads();
-  int64_t m = r.l[0];
-  for (int i = 1; i < kSegWaves; ++i) m = r.l[i] < m ? r.l[i] : m;
-  return m;
-}
-// Inclusive prefix sum over the workgroup (thread order).
-XV_INLINE int64_t seg_incl_scan(SegRed& r, int64_t x) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  x = wave_incl_scan_l(x);
-  __syncthreads();
-  if (lane == 63) r.l[w] = x;
-  __syncthreads();
-  for (int i = 0; i < w; ++i) x += r.l[i];
-  return x;
-}
-
-// Row max / min keys from the segment stats, and the row constants.
-struct RowConsts {
-  uint32_t kmax, kmin;
-  float inv_t, zmax, bs;
-};
-// From lane values already loaded (segment `lane` of the row, or 0 / ~0).
-XV_INLINE RowConsts row_consts_of(uint32_t kmax_lane, uint32_t kmin_lane, float temp) {
-  RowConsts c;
-  c.kmax = wave_max_u(kmax_lane);
-  c.kmin = wave_min_u(kmin_lane);
-  c.inv_t = 1.0f / temp;
-  c.zmax = bf16_to_f32(key_to_bits(c.kmax)) * c.inv_t;
-  c.bs = c.kmax ? bucket_scale(log2_ratio(key_to_bits(c.kmin), c.inv_t, c.zmax)) : 16.0f;
-  return c;
-}
-XV_INLINE RowConsts row_consts(const SegArgs& a, int b, float temp) {
-  // every wave reduces the R <= 64 segment values itself: one load per lane
-  RowConsts c;
-  const int lane = threadIdx.x & 63;
-  c.kmax = wave_max_u(lane < a.R ? a.seg_kmax[b * a.R + lane] : 0u);
-  c.kmin = wave_min_u(lane < a.R ? a.seg_kmin[b * a.R + lane] : 0xffffffffu);
-  c.inv_t = 1.0f / temp;
-  c.zmax = bf16_to_f32(key_to_bits(c.kmax)) * c.inv_t;
-  c.bs = c.kmax ? bucket_scale(log2_ratio(key_to_bits(c.kmin), c.inv_t, c.zmax)) : 16.0f;
-  return c;
-}
-
-__global__ __launch_bounds__(kSegThreads) void seg_stats_kernel(SegArgs a) {
-  __shared__ SegRed red;
-  const int b = blockIdx.y, r = blockIdx.x;
+// One workgroup per segment counts the segment's logits by value.  Bound by
+// the LDS atomics and its two ends (clearing and writing 16 KB): 16-bit
+// counts, two to a word, halve both against 32-bit ones.
+__global__ __launch_bounds__(kThreads) void seg_count_kernel(SegArgs a) {
+  __shared__ __attribute__((aligned(16))) uint32_t h[kSegWords];
+  __shared__ unsigned long long wbest[kWaves];
+  const int b = blockIdx.y, r = blockIdx.x, t = threadIdx.x, lane = t & 63;
   const bf16_t* row = a.logits + (int64_t)b * a.stride;
   const bool vec_ok = ((reinterpret_cast<uintptr_t>(row) & 15u) == 0);
   const int beg = r * a.seg_len, end = min(a.V, beg + a.seg_len);
@@ -1453,114 +1351,77 @@ __global__ __launch_bounds__(kSegThreads) void seg_stats_kernel(SegArgs a) {
       bid = better ? id : bid;
       nid = (nid < 0 && id < end && !order_key(bits)) ? id : nid;
     });
-    unsigned long long best = greedy_word(fm, bid, nid);
-    best = seg_max_ull(red, best);
-    if (threadIdx.x == 0) a.seg_best[b * a.R + r] = best;
+    unsigned long long best = wave_max_ull(greedy_word(fm, bid, nid));
+    if (lane == 0) wbest[t >> 6] = best;
+    __syncthreads();
+    if (t < 64) {
+      best = wave_max_ull(t < kWaves ? wbest[t] : 0ull);
+      if (t == 0) a.seg_best[b * a.R + r] = best;
+    }
     return;
   }
-  // Order keys two per packed op (x ^ 0x8000, or ~x for a set sign bit):
-  // finite keys lie in [0x7f, 0xff80], padding (0xffff) gives key 0, and
-  // the smallest key is taken as min(key - 1) + 1 so that key 0 wraps above
-  // every other.  NaN bits land outside [0x7f, 0xff80]; a lane that holds
-  // one redoes its ids one at a time with order_key (NaN: key 0).
-  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-  typedef short s16x2 __attribute__((ext_vector_type(2)));
-  const u16x2 top2 = {(unsigned short)0x8000u, (unsigned short)0x8000u}, one2 = {(unsigned short)1u, (unsigned short)1u};
-  u16x2 hi2 = {(unsigned short)0u, (unsigned short)0u}, lo2 = {(unsigned short)0xffffu, (unsigned short)0xffffu};
-  for_seg_words(row, vec_ok, beg, end, [&](uint32_t wd) {
-    const u16x2 w2 = __builtin_bit_cast(u16x2, wd);
-    const u16x2 sg = __builtin_bit_cast(u16x2, (s16x2)(__builtin_bit_cast(s16x2, w2) >> (short)15));
-    const u16x2 k2 = w2 ^ (sg | top2);
-    hi2 = __builtin_elementwise_max(hi2, k2);
-    lo2 = __builtin_elementwise_min(lo2, (u16x2)(k2 - one2));
-  });
-  uint32_t kmax = max((uint32_t)hi2.x, (uint32_t)hi2.y);
-  const uint32_t km1 = min((uint32_t)lo2.x, (uint32_t)lo2.y);
-  uint32_t kmin = km1 == 0xffffu ? 0xffffffffu : km1 + 1u;
-  if (kmax > 0xff80u || kmin < 0x7fu) {
-    kmax = 0;
-    kmin = 0xffffffffu;
-    for_seg(row, vec_ok, beg, end, [&](uint32_t bits, int) {
-      const uint32_t key = order_key(bits);
-      kmax = max(kmax, key);
-      kmin = min(kmin, key ? key : 0xffffffffu);
-    });
-  }
-  kmax = seg_max_u(red, kmax);
-  kmin = seg_min_u(red, kmin);
-  if (threadIdx.x == 0) {
-    a.seg_kmax[b * a.R + r] = kmax;
-    a.seg_kmin[b * a.R + r] = kmin;
-  }
-}
-
-__global__ __launch_bounds__(kSegThreads) void seg_hist_kernel(SegArgs a) {
-  __shared__ SegRed red;
-  __shared__ uint32_t wcnt[kSegWaves][kBuckets];
-  __shared__ unsigned long long wmass[kSegWaves][kBuckets];
-  const int b = blockIdx.y, r = blockIdx.x, t = threadIdx.x, w = t >> 6;
-  const RowParams p = row_params(a, b);
-  if (p.greedy) return;
-  const RowConsts rc = row_consts(a, b, p.temp);
-  const bf16_t* row = a.logits + (int64_t)b * a.stride;
-  const bool vec_ok = ((reinterpret_cast<uintptr_t>(row) & 15u) == 0);
-  const int beg = r * a.seg_len, end = min(a.V, beg + a.seg_len);
-  for (int i = t; i < kSegWaves * kBuckets; i += kSegThreads) {
-    (&wcnt[0][0])[i] = 0u;
-    (&wmass[0][0])[i] = 0ull;
-  }
+  uint4* h4 = reinterpret_cast<uint4*>(h);
+  for (int i = t; i < kSegWords / 4; i += kThreads) h4[i] = make_uint4(0u, 0u, 0u, 0u);
   __syncthreads();
-  int64_t far_c = 0, far_m = 0;
-  uint32_t kminp = 0xffffffffu;
-  if (p.use_k) {
-    // counts only: the sorted top-k list gives every mass the cut needs; the
-    // min-p key needs an exp only within half a binary order of its threshold
-    const float d_lo = __log2f(p.min_p) - 0.5f;
-    for_seg(row, vec_ok, beg, end, [&](uint32_t bits, int) {
-      const uint32_t key = order_key(bits);
-      if (!key) return;
-      const float d = log2_ratio(bits, rc.inv_t, rc.zmax);
-      const int bkt = bucket_of(d, rc.bs);
-      if (bkt < kBuckets - 1) atomicAdd(&wcnt[w][bkt], 1u);
-      else far_c += 1;
-      if (p.use_m && d >= d_lo && sampler_exp2(d) >= p.min_p) kminp = min(kminp, key);
-    });
-  } else {
-    for_seg(row, vec_ok, beg, end, [&](uint32_t bits, int) {
-      const uint32_t key = order_key(bits);
-      if (!key) return;
-      const float d = log2_ratio(bits, rc.inv_t, rc.zmax);
-      const float e = sampler_exp2(d);
-      const int64_t q = mass_of(e);
-      const int bkt = bucket_of(d, rc.bs);
-      if (bkt < kBuckets - 1) {
-        atomicAdd(&wcnt[w][bkt], 1u);
-        atomicAdd(&wmass[w][bkt], (unsigned long long)q);
+  uint32_t* head = h + kMagBins;
+  uint16_t* tiny = reinterpret_cast<uint16_t*>(head + kHWords);
+  // few-valued kinds of logits count in registers: masked rows hold thousands of one of them
+  uint32_t pz = 0, nz = 0, far = 0, far_mag = 0xffffu;
+  for_seg(row, vec_ok, beg, end, [&](uint32_t bits, int) {
+    const uint32_t mag = bits & 0x7fffu, m = mag - kMagLo;
+    if (m < (uint32_t)kMagBins) {
+      const uint32_t i = window_pos(bits, m);
+      atomicAdd(&h[i >> 1], (i & 1) ? 0x10000u : 1u);
+    } else if (mag <= kInfMag) {  // NaN (and padding) drops out
+      if (mag >= kMagLo) {
+        if (bits & 0x8000u) {
+          ++far;
+          far_mag = min(far_mag, mag);
+        } else {
+          head[kHTop] = 1u;
+        }
+      } else if (mag == 0u) {
+        if (bits) ++nz; else ++pz;
       } else {
-        far_c += 1;
-        far_m += q;
+        const uint32_t i = atomicAdd(&head[kHTiny], 1u);
+        if (i < (uint32_t)kTinyList) tiny[i] = (uint16_t)bits;
       }
-      if (p.use_m && e >= p.min_p) kminp = min(kminp, key);
-    });
+    }
+  });
+  if (__ballot(pz | nz)) {
+    pz = (uint32_t)wave_sum_l(pz);
+    nz = (uint32_t)wave_sum_l(nz);
+    if (lane == 0) {
+      atomicAdd(&head[kHPosZero], pz);
+      atomicAdd(&head[kHNegZero], nz);
+    }
   }
-  far_c = seg_sum_l(red, far_c);
-  far_m = seg_sum_l(red, far_m);
-  kminp = seg_min_u(red, kminp);
+  if (__ballot(far)) {
+    far = (uint32_t)wave_sum_l(far);
+    far_mag = wave_min_u(far_mag);
+    if (lane == 0) {
+      atomicAdd(&head[kHFar], far);
+      atomicMax(&head[kHFarMag], 0xffffu - far_mag);
+    }
+  }
   __syncthreads();
-  const int64_t o = ((int64_t)b * a.R + r) * kBuckets;
-  static_assert(kSegThreads == kBuckets, "one thread per bucket");
-  uint32_t c = 0;
-  unsigned long long m = 0;
-  for (int ww = 0; ww < kSegWaves; ++ww) { c += wcnt[ww][t]; m += wmass[ww][t]; }
-  if (t == kBuckets - 1) { c += (uint32_t)far_c; m += (unsigned long long)far_m; }
-  a.seg_cnt[o + t] = c;
-  if (!p.use_k) a.seg_mass[o + t] = m;  // top-k rows take their masses from the list
-  // the segment's total mass: its kept mass if the row has no cut (rows with
-  // a cut take theirs from the cut; top-k rows never reach the draw)
-  const int64_t total = seg_sum_l(red, p.use_k ? 0 : (int64_t)m);
-  if (t == 0) {
-    a.seg_minp[b * a.R + r] = kminp;
-    a.seg_kept[b * a.R + r] = total;
+  uint4* o = reinterpret_cast<uint4*>(a.seg_cnt + ((int64_t)b * a.R + r) * kSegWords);
+  static_assert(kMagBins == 4 * kThreads && kSegWords / 4 - kThreads <= 64, "four words per thread, the rest by wave 0");
+  const uint4 v = h4[t];
+  o[t] = v;
+  const uint32_t at = v.x ? 8 * t + (v.x & 0xffffu ? 0 : 1)
+                          : v.y ? 8 * t + (v.y & 0xffffu ? 2 : 3)
+                                : v.z ? 8 * t + (v.z & 0xffffu ? 4 : 5)
+                                      : v.w ? 8 * t + (v.w & 0xffffu ? 6 : 7) : 0xffffu;
+  const uint32_t first = wave_min_u(at);
+  if (lane == 0) wbest[t >> 6] = 0xffffu - first;
+  __syncthreads();
+  if (t < kSegWords / 4 - kThreads) {
+    uint4 x = h4[kThreads + t];
+    uint32_t f = 0;
+    for (int i = 0; i < kWaves; ++i) f = max(f, (uint32_t)wbest[i]);
+    if (t == kHFirst / 4) x.z = f;  // word kHFirst
+    o[kThreads + t] = x;
   }
 }
 
@@ -1626,223 +1487,54 @@ XV_INLINE int64_t wave_first(bool pred, int64_t none) {
   return m ? (int64_t)__builtin_ctzll(m) : none;
 }
 
-// The cut of a list of n <= 64 candidates, wave 0 alone: the same cut, kept
-// mass and draw as the workgroup list functions.
-// c: this lane's candidate (0 past n), in any order unless `sorted` says the
-// lanes hold the list sorted descending already.
-// segk: per segment in LDS, the kept mass of the buckets before the cut's
-// (rows without top-k; the list's part is added here).
-XV_INLINE void row_cut_wave_list(const SegArgs& a, RowPlan& plan, const RowParams& p, int b, int n,
-                                 unsigned long long c, unsigned long long* segk, bool sorted = false) {
+// The cut and the draw of a row's top_k list of n <= 64 candidates, sorted
+// descending (lane j's candidate c, 0 past n), by one wave.  kminp: the lowest
+// listed key that reaches min_p (0xffffffff: none).
+XV_INLINE void row_cut_wave_list(const SegArgs& a, const RowParams& p, float inv_t, float zmax, uint32_t kminp, int b,
+                                 int n, unsigned long long c) {
   const int lane = threadIdx.x & 63;
-  const float inv_t = plan.inv_t, zmax = plan.zmax;
-  if (!sorted) c = wave_sort_desc(c);
   const int64_t q = lane < n ? cand_mass(c, inv_t, zmax) : 0;
   const int64_t incl = wave_incl_scan_l(q);
   const uint32_t key = cand_key(c);
-  const uint32_t kminp = plan.kminp;
-  int64_t jcut;
-  if (plan.use_k) {
-    const int64_t total_k = wave_sum_l(lane < p.top_k ? q : 0);
-    jcut = (int64_t)p.top_k - 1;
-    if (p.use_p) {
-      const int64_t thr = (int64_t)floor((double)p.top_p * (double)total_k);
-      jcut = min(jcut, wave_first(lane < n && incl > thr, n));
-    }
-    const uint32_t last = cand_key(__shfl(c, n - 1));
-    if (p.use_m && kminp != 0xffffffffu && kminp >= last)
-      jcut = min(jcut, (int64_t)__popcll(__ballot(lane < n && key >= kminp)) - 1);
-  } else {
-    jcut = kTieAll;
-    if (plan.cut_p) jcut = min(jcut, wave_first(lane < n && plan.mp_before + incl > plan.thr, n));
-    if (plan.cut_m) jcut = min(jcut, (int64_t)__popcll(__ballot(lane < n && key >= kminp)) - 1);
+  const int64_t total_k = wave_sum_l(lane < p.top_k ? q : 0);
+  int64_t jcut = (int64_t)p.top_k - 1;
+  if (p.use_p) {
+    const int64_t thr = (int64_t)floor((double)p.top_p * (double)total_k);
+    jcut = min(jcut, wave_first(lane < n && incl > thr, n));
   }
+  const uint32_t last = cand_key(__shfl(c, n - 1));
+  if (p.use_m && kminp != 0xffffffffu && kminp >= last)
+    jcut = min(jcut, (int64_t)__popcll(__ballot(lane < n && key >= kminp)) - 1);
   if (jcut >= n) jcut = n - 1;
   if (jcut < 0) jcut = 0;
-  const unsigned long long edge = __shfl(c, (int)jcut);
   const int64_t m_list = wave_sum_l(lane <= jcut ? q : 0);
-  if (plan.use_k) {
-    // the kept list in ascending id order: re-keyed (~id << 32 | key), sorted descending
-    const float u = a.uniforms ? a.uniforms[b] : 0.5f;
-    const int64_t rdraw = draw_point(u, m_list);
-    // no mass in the list (z_max not finite, see lowest_id_of_key): its first candidate
-    const int64_t first = cand_id(__shfl(c, 0));
-    int64_t fid;
-    if (a.V <= (1 << 26)) {
-      // 32-bit words (0x3ffffff - id) << 6 | lane, sorted descending: ids
-      // ascending, each word naming the lane that holds its mass
-      uint32_t e = lane <= jcut ? (0x3ffffffu - (uint32_t)cand_id(c)) << 6 | (uint32_t)lane : 0u;
-      e = wave_sort_desc32(e);
-      const int64_t qe = (int64_t)__shfl((long long)q, (int)(e & 63u));
-      const int64_t ie = wave_incl_scan_l(lane <= jcut ? qe : 0);
-      const int64_t fi = wave_first(lane <= jcut && ie > rdraw, -1);
-      const uint32_t ef = __shfl(e, fi < 0 ? 0 : (int)fi);
-      fid = fi < 0 ? first : (int64_t)(0x3ffffffu - (ef >> 6));
-    } else {
-      unsigned long long e =
-          lane <= jcut ? ((unsigned long long)(0xffffffffu - (uint32_t)cand_id(c)) << 32) | cand_key(c) : 0ull;
-      e = wave_sort_desc(e);
-      const int64_t qe = lane <= jcut ? mass_of(exp_of(key_to_bits((uint32_t)(e & 0xffffffffu)), inv_t, zmax)) : 0;
-      const int64_t ie = wave_incl_scan_l(qe);
-      const int64_t fi = wave_first(lane <= jcut && ie > rdraw, -1);
-      const unsigned long long ef = __shfl(e, fi < 0 ? 0 : (int)fi);
-      fid = fi < 0 ? first : (int64_t)(0xffffffffu - (uint32_t)(ef >> 32));
-    }
-    if (lane == 0) {
-      a.out_ids[b] = fid;
-      plan.status = kPlanDone;
-    }
-    return;
-  }
-  // each segment's kept mass: its earlier buckets plus its listed candidates up to the cut
-  if (lane <= jcut) atomicAdd(&segk[cand_id(c) / a.seg_len], (unsigned long long)q);
-  if (lane == 0) {
-    plan.key_cut = cand_key(edge);
-    plan.id_cut = cand_id(edge);
-    plan.M = plan.m_before + m_list;
-    plan.status = kPlanDraw;
-  }
-}
-
-// The cut of a gathered bucket list of a row without top-k, by per-key counts
-// instead of a sort.  A candidate's mass depends on its key alone and the
-// list's order is key descending, ties by ascending id, so a prefix of the
-// list is a key plus the number of that key's lowest ids, and the mass before
-// a key is a sum of count x mass over the keys above it.  Bin j of the count
-// array holds key khi - j.  Returns false, having written nothing, when the
-// keys span more bins than the array holds or the cut splits a tie group of
-// more than kTieRank ids (the sort then takes the list); the result is the
-// sort's in every other case.
-constexpr int kKeyBins = kWaves * kBuckets;  // the per-wave histograms' LDS, unused here
-constexpr int kTieRank = 512;
-XV_INLINE bool row_cut_by_keys(const SegArgs& a, RowPlan& plan, Shared& s, FastShared& fs, int n,
-                               uint32_t* tie_ids, unsigned long long* segk) {
-  const int t = threadIdx.x;
-  const uint32_t klo = plan.klo, khi = plan.khi;
-  if (khi < klo || khi - klo >= (uint32_t)kKeyBins) return false;
-  const int K = (int)(khi - klo) + 1;
-  const float inv_t = plan.inv_t, zmax = plan.zmax;
-  uint32_t* kcnt = &fs.wcnt[0][0];
-  for (int j = t; j < K; j += kThreads) kcnt[j] = 0u;
-  __syncthreads();
-  for (int i = t; i < n; i += kThreads) atomicAdd(&kcnt[khi - cand_key(fs.cand[i])], 1u);
-  __syncthreads();
-  constexpr int kPerT = kKeyBins / kThreads;  // consecutive bins of one thread
-  static_assert(kPerT * kThreads == kKeyBins, "bins per thread");
-  const int j0 = t * kPerT;
-  uint32_t c[kPerT];
-  int64_t m[kPerT];
-  int64_t local = 0;
-  int64_t first = kTieAll, last = -1;  // present bins of this thread
-#pragma unroll
-  for (int k = 0; k < kPerT; ++k) {
-    const int j = j0 + k;
-    c[k] = j < K ? kcnt[j] : 0u;
-    m[k] = c[k] ? mass_of(exp_of(key_to_bits(khi - (uint32_t)j), inv_t, zmax)) : 0;
-    local += (int64_t)c[k] * m[k];
-    if (c[k]) {
-      first = first < j ? first : j;
-      last = j;
-    }
-  }
-  int64_t list_mass;  // unused
-  const int64_t before = block_excl_scan(s, local, &list_mass);  // mass of the bins before this thread's
-  // cut position (bin << 32 | ties kept): kTieAll keeps the whole list, -1 only its first candidate
-  int64_t pos = kTieAll;
-  if (plan.cut_p) {  // first candidate whose inclusive mass (after the earlier buckets') exceeds thr
-    const int64_t thr = plan.thr;
-    int64_t cum = plan.mp_before + before, found = kTieAll;
-#pragma unroll
-    for (int k = 0; k < kPerT; ++k) {
-      const int64_t w = (int64_t)c[k] * m[k];
-      if (found == kTieAll && c[k] && cum + w > thr) {
-        int64_t i = m[k] > 0 ? (thr - cum) / m[k] + 1 : 1;
-        i = i < 1 ? 1 : (i > (int64_t)c[k] ? (int64_t)c[k] : i);
-        found = ((int64_t)(j0 + k) << 32) | i;
-      }
-      cum += w;
-    }
-    pos = block_min_l(s, found);
-  }
-  if (plan.cut_m) {  // the candidates with key >= kminp, a prefix of the list
-    const uint32_t kminp = plan.kminp;
-    int64_t lastm = -1;
-    if (kminp <= khi) {
-      const int64_t jm = (int64_t)(khi - kminp);
-#pragma unroll
-      for (int k = 0; k < kPerT; ++k)
-        if (c[k] && j0 + k <= jm) lastm = ((int64_t)(j0 + k) << 32) | c[k];
-    }
-    lastm = -block_min_l(s, -lastm);
-    pos = lastm < pos ? lastm : pos;
-  }
-  int jc;
-  int64_t ic;
-  if (pos == kTieAll) {  // (uniform branches: the block reductions run on every thread)
-    jc = (int)-block_min_l(s, -last);
-    ic = kTieAll;
-  } else if (pos < 0) {
-    jc = (int)block_min_l(s, first);
-    ic = 1;
+  // the kept list in ascending id order: re-keyed (~id << 32 | key), sorted descending
+  const float u = a.uniforms ? a.uniforms[b] : 0.5f;
+  const int64_t rdraw = draw_point(u, m_list);
+  // no mass in the list (z_max not finite, see lowest_id_of_key): its first candidate
+  const int64_t first = cand_id(__shfl(c, 0));
+  int64_t fid;
+  if (a.V <= (1 << 26)) {
+    // 32-bit words (0x3ffffff - id) << 6 | lane, sorted descending: ids
+    // ascending, each word naming the lane that holds its mass
+    uint32_t e = lane <= jcut ? (0x3ffffffu - (uint32_t)cand_id(c)) << 6 | (uint32_t)lane : 0u;
+    e = wave_sort_desc32(e);
+    const int64_t qe = (int64_t)__shfl((long long)q, (int)(e & 63u));
+    const int64_t ie = wave_incl_scan_l(lane <= jcut ? qe : 0);
+    const int64_t fi = wave_first(lane <= jcut && ie > rdraw, -1);
+    const uint32_t ef = __shfl(e, fi < 0 ? 0 : (int)fi);
+    fid = fi < 0 ? first : (int64_t)(0x3ffffffu - (ef >> 6));
   } else {
-    jc = (int)(pos >> 32);
-    ic = pos & 0xffffffffll;
+    unsigned long long e =
+        lane <= jcut ? ((unsigned long long)(0xffffffffu - (uint32_t)cand_id(c)) << 32) | cand_key(c) : 0ull;
+    e = wave_sort_desc(e);
+    const int64_t qe = lane <= jcut ? mass_of(exp_of(key_to_bits((uint32_t)(e & 0xffffffffu)), inv_t, zmax)) : 0;
+    const int64_t ie = wave_incl_scan_l(qe);
+    const int64_t fi = wave_first(lane <= jcut && ie > rdraw, -1);
+    const unsigned long long ef = __shfl(e, fi < 0 ? 0 : (int)fi);
+    fid = fi < 0 ? first : (int64_t)(0xffffffffu - (uint32_t)(ef >> 32));
   }
-  const uint32_t key_cut = khi - (uint32_t)jc;
-  const int64_t cnt_c = kcnt[jc];
-  if (ic >= cnt_c) ic = kTieAll;
-  int64_t id_cut = kTieAll;
-  if (ic != kTieAll) {
-    // the ic-th smallest id of key_cut: each of its ids counts the smaller ones
-    if (cnt_c > kTieRank) return false;
-    __syncthreads();
-    if (t == 0) fs.ncand = 0;
-    __syncthreads();
-    for (int i = t; i < n; i += kThreads) {
-      const unsigned long long e = fs.cand[i];
-      if (cand_key(e) == key_cut) tie_ids[atomicAdd(&fs.ncand, 1)] = (uint32_t)cand_id(e);
-    }
-    __syncthreads();
-    const int nt = fs.ncand, nt4 = (nt + 3) & ~3;
-    if (t >= nt && t < nt4) tie_ids[t] = 0xffffffffu;
-    __syncthreads();
-    if (t < nt) {
-      const uint32_t mine = tie_ids[t];
-      const uint4* v = reinterpret_cast<const uint4*>(tie_ids);
-      int rank = 0;
-      for (int q = 0; q < nt4 / 4; ++q) {
-        const uint4 x = v[q];
-        rank += (x.x < mine) + (x.y < mine) + (x.z < mine) + (x.w < mine);
-      }
-      if (rank == ic - 1) s.b_id = mine;
-    }
-    __syncthreads();
-    id_cut = s.b_id;
-  }
-  // kept mass of the list: the bins before jc, and ic (or all) ties of jc
-  if (jc >= j0 && jc < j0 + kPerT) {
-    int64_t kept = plan.m_before + before;
-#pragma unroll
-    for (int k = 0; k < kPerT; ++k)
-      if (j0 + k < jc) kept += (int64_t)c[k] * m[k];
-      else if (j0 + k == jc) kept += (ic == kTieAll ? (int64_t)c[k] : ic) * m[k];
-    s.b_total = kept;
-  }
-  for (int i = t; i < n; i += kThreads) {
-    const unsigned long long e = fs.cand[i];
-    const uint32_t key = cand_key(e);
-    const int64_t id = cand_id(e);
-    if (key > key_cut || (key == key_cut && id <= id_cut))
-      atomicAdd(&segk[id / a.seg_len], (unsigned long long)cand_mass(e, inv_t, zmax));
-  }
-  __syncthreads();
-  if (t == 0) {
-    plan.key_cut = key_cut;
-    plan.id_cut = id_cut;
-    plan.M = s.b_total;
-    plan.status = kPlanDraw;
-  }
-  return true;
+  if (lane == 0) a.out_ids[b] = fid;
 }
 
 // ---------------------------------------------------------------------------
@@ -1864,7 +1556,6 @@ XV_INLINE bool row_cut_by_keys(const SegArgs& a, RowPlan& plan, Shared& s, FastS
 constexpr int kTopList = 64;
 constexpr int kTopVecs = 4;  // 8-id vectors per thread in registers: segments of up to 8192 ids
 
-XV_INLINE int wave_incl_scan_i(int x) { return (int)wave_incl_scan_l(x); }
 
 // Each wave selects the top kTopList of its own ids (vectors v * kSegThreads
 // + 64 w + lane of the segment, ids ascending in (v, lane, k) order) with no
@@ -2155,479 +1846,543 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(SegArgs a) {
     if (t == 0) a.out_ids[b] = n ? cand_id(top) : 0;
     return;
   }
-  RowPlan pl;
-  pl.use_k = 1;
-  pl.inv_t = 1.0f / p.temp;
-  pl.zmax = bf16_to_f32(key_to_bits(cand_key(top))) * pl.inv_t;
+  const float inv_t = 1.0f / p.temp;
+  const float zmax = bf16_to_f32(key_to_bits(cand_key(top))) * inv_t;
   uint32_t kminp = 0xffffffffu;
   if (p.use_m && t < n) {
     const uint32_t key = cand_key(c);
-    if (sampler_exp2(log2_ratio(key_to_bits(key), pl.inv_t, pl.zmax)) >= p.min_p) kminp = key;
+    if (exp_of(key_to_bits(key), inv_t, zmax) >= p.min_p) kminp = key;
   }
-  pl.kminp = wave_min_u(kminp);
-  row_cut_wave_list(a, pl, p, b, n, c, nullptr, true);  // top-k: drawn from the list, no per-segment masses
+  row_cut_wave_list(a, p, inv_t, zmax, wave_min_u(kminp), b, n, c);
 }
 
 
 // ---------------------------------------------------------------------------
-// Per row, after seg_stats and seg_hist, in one launch (row_finish_kernel):
-// the plan (the bucket or buckets holding the cut-offs, from the summed
-// segment histograms), the candidates of those buckets gathered from the row
-// by this workgroup, the cut, and the draw.
+// Per row, after seg_count: the cut and the draw from the counts.
+//
+// A candidate's mass depends on its key alone, so rank and mass prefixes over
+// the window's positions give every cut exactly: the top-k rank, the first
+// rank whose inclusive mass exceeds floor(top_p * mass), the rank of the
+// lowest key that reaches min_p; the smallest of them cuts.  Between the
+// positive and the negative window lie the zeros and the listed magnitudes
+// below 2^-22 (`mid`), after the window the values of -2^10 and below
+// (`far`).  Rows the counts don't settle (a value of 2^10 or above, a maximum
+// or a cut in mid, far values with mass, no value at all) run sample_row.
+//
+// One workgroup works alone on its CU, so the time is latency and issue, not
+// bandwidth: wave w takes positions 256 w .. of each half, four per lane, so
+// the dense octaves of usual rows spread over most waves; masses are held as
+// doubles (integers of at most 2^40; products and sums over up to 8190 ids
+// stay below 2^53, so the full-rate fp64 FMA replaces 64-bit integer products
+// exactly); the masses go into an LDS table, which the draw reads instead of
+// an exp2 per id.  The kernel keeps out of scratch memory: with any, its
+// sixteen waves started over 3.6 us instead of 0.2, and the row took 18.8 us
+// in place of 13.5 (the row loads of the one-workgroup code inside it run
+// kChunk packed vectors at a time for that).
+constexpr int kHalfPos = kMagBins;  // positions per half
+constexpr int kCntLoads = 8;        // segments whose counts load together
+static_assert(kHalfPos == 4 * kThreads, "four positions per thread and half");
 
-constexpr uint32_t kInfKey = 0xff80u;  // +inf: the keys of non-NaN values are [1, kInfKey]
+struct RowCut {
+  int pos;       // the cut key's position; 2 * kMagBins: none (every window key kept)
+  int ties;      // ids of the cut key kept
+  int64_t M;     // kept mass
+  int n;         // rank of the cut (2^31 - 1: none)
+  int fail;      // the cut falls in mid
+};
+struct RowShared {
+  RowCut cut[3];  // the top-k set's end, top-p's cut, the row's cut
+  int ccnt[32];        // totals of the chunks (half, wave)
+  int64_t cmass[32];
+  int nm[kWaves];
+  unsigned long long segm[kMaxSegs];  // kept masses of the window keys before the cut's
+  int64_t midq[kMaxSegs];
+  int t0;        // the draw: the thread whose ids hold the draw point, its mass and ties before
+  int tie;
+  int64_t cum;
+};
 
-// Smallest key in [1, kInfKey] at which pred holds (pred is false below some
-// key and true from it on), kInfKey + 1 if it holds at none.  Each round
-// probes 64 keys at once, so three or four rounds cover the key range; every
-// lane of the calling wave returns the result.
-template <typename P>
-XV_INLINE uint32_t wave_first_key(P&& pred) {
-  const uint32_t lane = threadIdx.x & 63;
-  uint32_t l = 1, h = kInfKey + 1;  // the result is in [l, h]: pred holds at h, or h is past the keys
-  while (l < h) {
-    const uint32_t span = h - l, step = (span + 63) / 64;
-    const uint32_t k = l + lane * step;
-    const unsigned long long m = __ballot(k < h && pred(k));
-    if (m) {
-      const uint32_t i = (uint32_t)__builtin_ctzll(m);
-      h = l + i * step;
-      if (i) l = h - step + 1;  // the probe before it failed
-    } else {
-      l += ((span + step - 1) / step - 1) * step + 1;  // past the last probe below h
-    }
-  }
-  return l;
+// Eight values per lane summed over the wave: lane l (a multiple of 8) gets
+// the sum of value l / 8.  Each of the first three exchanges halves the values
+// a lane still carries.
+XV_INLINE int64_t wave_sum8(int64_t (&v)[8]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    v[k] = ((lane & 32) ? v[k + 4] : v[k]) + (int64_t)xor_lane64<32>((uint64_t)((lane & 32) ? v[k] : v[k + 4]));
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    v[k] = ((lane & 16) ? v[k + 2] : v[k]) + (int64_t)xor_lane64<16>((uint64_t)((lane & 16) ? v[k] : v[k + 2]));
+  int64_t x = ((lane & 8) ? v[1] : v[0]) + (int64_t)xor_lane64<8>((uint64_t)((lane & 8) ? v[0] : v[1]));
+  x += (int64_t)xor_lane64<4>((uint64_t)x);
+  x += (int64_t)xor_lane64<2>((uint64_t)x);
+  return x + (int64_t)xor_lane64<1>((uint64_t)x);
 }
 
-// Append every id of the row whose key lies in [klo, khi] (klo >= 1) to
-// fs.cand as (key << 32) | ~id; fs.ncand counts them, also past kMaxCand.
-// The key transform and the range test run on two logits per 32-bit word (the
-// key of raw bits b is b ^ 0xffff for a negative b, else b ^ 0x8000; a
-// saturating subtract leaves 0 exactly for the keys in range), so a vector
-// without a hit costs a few instructions.  Ids with a hit are checked exactly
-// (a NaN's key is 0 there).  The loads of a step go out together: every lane
-// loads whole vectors (vectors past the row's last whole one reload it and
-// are masked), and the ids past the last whole vector are taken one by one at
-// the end.
-constexpr int kGatherChunk = 10;  // 16-byte loads in flight per thread (more spill registers)
-constexpr int kGatherRec = 4;     // vectors with a hit a lane records for later
-XV_INLINE void gather_key_range(FastShared& fs, const bf16_t* row, int V, bool vec_ok, uint32_t klo,
-                                uint32_t khi) {
-  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-  typedef short s16x2 __attribute__((ext_vector_type(2)));
-  auto append = [&](uint32_t bits, int id) {
-    const uint32_t key = order_key(bits);
-    if (key >= klo && key <= khi) {
-      const int slot = atomicAdd(&fs.ncand, 1);
-      if (slot < kMaxCand)
-        fs.cand[slot] = ((unsigned long long)key << 32) | (unsigned long long)(0xffffffffu - (uint32_t)id);
+// A mass as a double: the same integer as mass_of's.
+XV_INLINE double mass_d(float e) { return __builtin_trunc((double)e * 1099511627776.0); }
+constexpr uint32_t kExactIds = 4095;  // ids per thread and half whose mass sum (of both halves) is exact in fp64
+
+// Sampled row b from its segments' counts; false (on every thread) if the
+// counts don't settle it.  qtab: masses of the 2 * kMagBins window keys by
+// magnitude (kMagBins + magnitude for negative ones).
+XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& s, double* qtab, int b) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const bf16_t* row = a.logits + (int64_t)b * a.stride;
+  const bool vec_ok = ((reinterpret_cast<uintptr_t>(row) & 15u) == 0);
+  const uint32_t* cnts = a.seg_cnt + (int64_t)b * a.R * kSegWords;
+  // f(segment, its counts of this thread's positions: [half][j]): a group's
+  // loads all go out before any is used (segments past R reload the last)
+  auto each_group = [&](auto&& f) {
+    for (int r0 = 0; r0 < a.R; r0 += kCntLoads) {
+      uint2 kc[kCntLoads][2];
+#pragma unroll
+      for (int r = 0; r < kCntLoads; ++r)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          kc[r][h] = *reinterpret_cast<const uint2*>(cnts + (int64_t)min(r0 + r, a.R - 1) * kSegWords +
+                                                     h * (kHalfPos / 2) + 2 * t);
+      f(r0, kc);
     }
   };
-  const int t = threadIdx.x;
-  const int nfull = vec_ok ? V / 8 : 0;  // a row not 16-byte aligned goes id by id
-  const u16x2 lo2 = {(unsigned short)klo, (unsigned short)klo};
-  const u16x2 sp2 = {(unsigned short)(khi - klo), (unsigned short)(khi - klo)};
-  const u16x2 top2 = {(unsigned short)0x8000u, (unsigned short)0x8000u};
-  auto test = [&](const uint32_t (&wd)[4], uint32_t (&z)[4]) {  // true if some id may be in range
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const u16x2 w2 = __builtin_bit_cast(u16x2, wd[k]);
-      const u16x2 sg = __builtin_bit_cast(u16x2, (s16x2)(__builtin_bit_cast(s16x2, w2) >> (short)15));
-      z[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat((u16x2)((w2 ^ (sg | top2)) - lo2), sp2));
-    }
-    const u16x2 m2 = __builtin_elementwise_min(
-        __builtin_elementwise_min(__builtin_bit_cast(u16x2, z[0]), __builtin_bit_cast(u16x2, z[1])),
-        __builtin_elementwise_min(__builtin_bit_cast(u16x2, z[2]), __builtin_bit_cast(u16x2, z[3])));
-    return m2.x == 0 || m2.y == 0;
+  auto count_of = [](const uint2 (&k)[2], int h, int j) {
+    return ((j < 2 ? k[h].x : k[h].y) >> (16 * (j & 1))) & 0xffffu;
   };
-  auto hits = [&](const uint32_t (&wd)[4], const uint32_t (&z)[4], int vi) {
+  const uint32_t* head = cnts + (int64_t)min(lane, a.R - 1) * kSegWords + kMagBins;
+  const uint4 h0 = *reinterpret_cast<const uint4*>(head), h1 = *reinterpret_cast<const uint4*>(head + 4);
+  if (t < 3) s.cut[t] = RowCut{2 * kMagBins, 0, 0, 0x7fffffff, 0};
+  if (t < kMaxSegs) s.segm[t] = 0ull;
+  uint32_t c[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+  each_group([&](int r0, const uint2 (&kc)[kCntLoads][2]) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (((z[k >> 1] >> (16 * (k & 1))) & 0xffffu) == 0u) append((wd[k >> 1] >> (16 * (k & 1))) & 0xffffu, vi * 8 + k);
-  };
-  // Vectors with a hit are recorded (up to kGatherRec per lane, 16-bit indices)
-  // and their ids handled after the scan, so a wave runs the per-id work a few
-  // times instead of in most steps when hits are spread over the row.
-  const bool defer = nfull <= 65536;
-  unsigned long long rec = 0;
-  int nrec = 0;
-  for (int c0 = 0; c0 < nfull; c0 += kGatherChunk * kThreads) {
-    uint32_t wv[kGatherChunk][4];
+    for (int r = 0; r < kCntLoads; ++r)
+      if (r0 + r < a.R)
 #pragma unroll
-    for (int v = 0; v < kGatherChunk; ++v) {
-      const int vi = c0 + v * kThreads + t;
-      const Vec8 x = load_vec8(row + 8u * (uint32_t)min(vi, nfull - 1));
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) wv[v][k] = x.w[k];
+          for (int j = 0; j < 4; ++j) c[h][j] += count_of(kc[r], h, j);
+  });
+  // lane r < R: segment r's header
+  const bool seg_lane = lane < a.R;
+  const int first = (int)(0xffffu - wave_max_u(seg_lane ? h1.z : 0u));  // 0xffff: no window value
+  const uint32_t zeros = seg_lane ? h0.x + h0.y : 0u, ntiny = seg_lane ? h1.y : 0u;
+  const bool has_mid = __ballot(zeros | ntiny) != 0, has_far = __ballot(seg_lane && h0.z) != 0;
+  const float inv_t = 1.0f / p.temp;
+  const float zmax = bf16_to_f32(pos_bits(min(first, 2 * kMagBins - 1))) * inv_t;
+  bool settled = first < 2 * kMagBins && !(first >= kMagBins && has_mid) && __builtin_isfinite(zmax) &&
+                 !__ballot(seg_lane && (h1.x != 0u || ntiny > (uint32_t)kTinyList));
+  int far = 0;
+  if (has_far) {
+    far = (int)wave_sum_l(seg_lane ? h0.z : 0u);
+    const uint32_t far_mag = 0xffffu - wave_max_u(seg_lane ? h0.w : 0u);
+    const float e = exp_of(0x8000u | far_mag, inv_t, zmax);  // the largest: the others' masses are no larger
+    settled = settled && mass_of(e) == 0 && !(p.use_m && e >= p.min_p);
+  }
+  // mid: counts and masses, lane r its segment's
+  int64_t mid_q = 0;
+  int mid_c = 0;
+  bool mid_in = false;  // mid reaches min_p (all of it, or the row isn't settled)
+  if (settled && has_mid) {
+    const float ez = exp_of(0u, inv_t, zmax);
+    int64_t mid_qr = (int64_t)zeros * mass_of(ez);
+    bool any_in = zeros && ez >= p.min_p, any_out = zeros && !(ez >= p.min_p);
+    for (unsigned long long m = __ballot(ntiny != 0); m; m &= m - 1) {
+      const int r = __builtin_ctzll(m);
+      const int n = (int)__shfl((int)ntiny, r);
+      float e = 0.0f;
+      if (lane < n) {
+        const uint16_t* list = reinterpret_cast<const uint16_t*>(cnts + (int64_t)r * kSegWords + kMagBins + kHWords);
+        e = exp_of(list[lane], inv_t, zmax);
+        any_in |= e >= p.min_p;
+        any_out |= !(e >= p.min_p);
+      }
+      const int64_t q = wave_sum_l(mass_of(e));
+      mid_qr += lane == r ? q : 0;
     }
+    if (p.use_m) {
+      mid_in = __ballot(any_in) != 0;
+      settled = !(mid_in && __ballot(any_out) != 0);
+    }
+    mid_c = (int)wave_sum_l(zeros + ntiny);
+    mid_q = wave_sum_l(mid_qr);
+    if (t < a.R) s.midq[t] = mid_qr;
+  }
+  if (!settled) return false;
+
+  // masses; per half, the rank and mass prefixes over its positions
+  int cex[2], cn[2], nm[2];  // exclusive rank prefixes, counts, ranks reaching min_p
+  int64_t mex[2], ms[2];
+  const int pre_c = t == 0 ? mid_c : 0;  // mid: before half 1's first position
+  const int64_t pre_q = t == 0 ? mid_q : 0;
+  // position pos's entry of the table
+  auto tab_of = [](int pos) { return pos < kHalfPos ? kHalfPos - 1 - pos : pos; };
+  {
+    // one position per step of a rolled loop (the counts rotate through c[0][0])
+    int n_h = 0, nm_h = 0;
+    int64_t m_h = 0;
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t ci = c[0][0];
 #pragma unroll
-    for (int v = 0; v < kGatherChunk; ++v) {
-      const int vi = c0 + v * kThreads + t;
-      uint32_t z[4];
-      if (test(wv[v], z) && vi < nfull) {
-        if (defer && nrec < kGatherRec) {
-          rec |= (unsigned long long)(uint32_t)vi << (16 * nrec);
-          ++nrec;
-        } else {
-          hits(wv[v], z, vi);
+      for (int j = 0; j < 7; ++j) c[j >> 2][j & 3] = c[(j + 1) >> 2][(j + 1) & 3];
+      c[1][3] = ci;
+      const int pos = (i >> 2) * kHalfPos + 4 * t + (i & 3);
+      double qd = 0.0;
+      if (ci) {
+        const float e = exp_of(pos_bits(pos), inv_t, zmax);
+        qd = mass_d(e);
+        n_h += (int)ci;
+        m_h += (int64_t)((uint64_t)ci * (uint64_t)qd);
+        if (p.use_m && e >= p.min_p) nm_h = n_h;
+      }
+      qtab[tab_of(pos)] = qd;
+      if (i == 3) {
+        cn[0] = n_h, ms[0] = m_h, nm[0] = nm_h;
+        n_h = pre_c, m_h = pre_q, nm_h = mid_in ? pre_c : 0;
+      }
+    }
+    cn[1] = n_h + (t == kThreads - 1 ? far : 0), ms[1] = m_h, nm[1] = nm_h;
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    int ci = 0;
+    int64_t mi = 0;
+    if (__ballot(cn[h] != 0)) {
+      ci = wave_incl_scan_i(cn[h]);
+      mi = wave_incl_scan_l(ms[h]);
+    }
+    cex[h] = ci - cn[h];
+    mex[h] = mi - ms[h];
+    if (lane == 63) {
+      s.ccnt[16 * h + w] = ci;
+      s.cmass[16 * h + w] = mi;
+    }
+  }
+  // this thread's masses again, and whether some lane holds more than
+  // kExactIds ids of a half (uniform in the wave)
+  double q[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q[h][j] = qtab[tab_of(h * kHalfPos + 4 * t + j)];
+  bool big = false;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) big |= c[h][0] + c[h][1] + c[h][2] + c[h][3] > kExactIds;
+  big = __ballot(big) != 0;
+  static_assert(kWaves == 16, "32 chunks, one per lane of half a wave");
+  __syncthreads();
+  int ctot;
+  int64_t mtot;
+  {
+    const int cc = lane < 32 ? s.ccnt[lane] : 0;
+    const int64_t cm = lane < 32 ? s.cmass[lane] : 0;
+    const int ci = wave_incl_scan_i(cc);
+    const int64_t mi = wave_incl_scan_l(cm);
+    ctot = __shfl(ci, 31);
+    mtot = __shfl(mi, 31);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      cex[h] += __shfl(ci - cc, 16 * h + w);
+      mex[h] += __shfl(mi - cm, 16 * h + w);
+    }
+  }
+
+  // rank n - 1's key, by the thread that holds it: its position, the ids of
+  // the key up to the rank, and the mass through the rank
+  auto locate = [&](int n, RowCut& cut) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (!(cex[h] < n && n <= cex[h] + cn[h])) continue;
+      int left = n - cex[h] - (h ? pre_c : 0);
+      int64_t m = mex[h] + (h ? pre_q : 0);
+      if (left <= 0) {
+        cut.fail = 1;
+        continue;
+      }
+      int pos = 2 * kMagBins, ties = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (left > 0) {
+          const bool here = left <= (int)c[h][j];
+          if (here) {
+            pos = h * kHalfPos + 4 * t + j;
+            ties = left;
+          }
+          m += (int64_t)((uint64_t)(here ? left : (int)c[h][j]) * (uint64_t)q[h][j]);
+          left -= (int)c[h][j];
         }
+      }
+      cut.pos = pos;  // a rank in far (left > 0 still): every window key kept, far has no mass
+      cut.ties = ties;
+      cut.M = m;
+      cut.n = n;
+    }
+  };
+  int n = ctot;
+  if (p.use_k && p.top_k < n) n = p.top_k;
+  int64_t base = mtot;
+  if (p.use_p && n < ctot) {
+    locate(n, s.cut[0]);
+    __syncthreads();
+    base = s.cut[0].M;
+    if (s.cut[0].fail) return false;
+  }
+  if (p.use_p) {
+    // the first rank whose inclusive mass exceeds thr (a negative thr: the first rank)
+    const int64_t thr = (int64_t)floor((double)p.top_p * (double)base);
+    if (thr < 0) {
+      locate(1, s.cut[1]);
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (!(mex[h] <= thr && thr < mex[h] + ms[h])) continue;
+        int64_t left = thr - mex[h], m = mex[h];
+        int k = cex[h];
+        if (h) {
+          if (left < pre_q) {
+            s.cut[1].fail = 1;
+            continue;
+          }
+          left -= pre_q;
+          k += pre_c;
+          m += pre_q;
+        }
+        int64_t qk = 1;
+        int pos = -1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (pos < 0) {
+            const int64_t mj = (int64_t)((uint64_t)c[h][j] * (uint64_t)q[h][j]);
+            if (left < mj) {
+              pos = h * kHalfPos + 4 * t + j;
+              qk = (int64_t)q[h][j];
+            } else {
+              left -= mj;
+              m += mj;
+              k += (int)c[h][j];
+            }
+          }
+        }
+        // left / qk, below the key's count: the double quotient is off by at most one
+        int64_t i = (int64_t)((double)left / (double)qk);
+        if (i * qk > left) --i;
+        if ((i + 1) * qk <= left) ++i;
+        s.cut[1] = RowCut{pos, (int)i + 1, m + (i + 1) * qk, k + (int)i + 1, 0};
       }
     }
   }
-  for (int r = 0; __ballot(nrec > r); ++r) {
-    if (nrec > r) {
-      const int vi = (int)((rec >> (16 * r)) & 0xffffu);
-      const Vec8 x = load_vec8(row + 8u * (uint32_t)vi);
-      const uint32_t wd[4] = {x.w[0], x.w[1], x.w[2], x.w[3]};
-      uint32_t z[4];
-      test(wd, z);
-      hits(wd, z, vi);
+  int n_m = 0;
+  if (p.use_m) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) n_m = max(n_m, nm[h] ? cex[h] + nm[h] : 0);
+    n_m = (int)wave_max_u((uint32_t)n_m);
+    if (lane == 0) s.nm[w] = n_m;
+  }
+  __syncthreads();
+  RowCut cut = s.cut[1];  // no top-p: none
+  if (cut.fail) return false;
+  n = min(n, cut.n);
+  if (p.use_m) {
+    n_m = (int)wave_max_u(lane < kWaves ? (uint32_t)s.nm[lane] : 0u);
+    if (n_m > 0) n = min(n, n_m);
+  }
+  if (n >= ctot) {
+    cut.pos = 2 * kMagBins;
+    cut.ties = 0;
+    cut.M = mtot;
+  } else if (n != cut.n) {
+    locate(n, s.cut[2]);
+    __syncthreads();
+    cut = s.cut[2];
+    if (cut.fail) return false;
+  }
+  const int pos = __builtin_amdgcn_readfirstlane(cut.pos), cut_ties = __builtin_amdgcn_readfirstlane(cut.ties);
+  const int64_t cut_m = cut.M;
+
+  // each segment's kept mass: its positions before the cut's, then (lane r)
+  // mid and its share of the cut key's ids, the lowest ids first
+  uint32_t tie_word = 0;
+  if (pos < 2 * kMagBins && seg_lane) tie_word = cnts[(int64_t)lane * kSegWords + (pos >> 1)];
+  bool some = false;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    double* qo = qtab + (h ? kHalfPos + 4 * t : kHalfPos - 4 - 4 * t);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      q[h][j] = h * kHalfPos + 4 * t + j < pos ? q[h][j] : 0.0;
+      some |= q[h][j] != 0.0;
     }
+    double2* q2 = reinterpret_cast<double2*>(qo);
+    q2[0] = h ? make_double2(q[h][0], q[h][1]) : make_double2(q[h][3], q[h][2]);
+    q2[1] = h ? make_double2(q[h][2], q[h][3]) : make_double2(q[h][1], q[h][0]);
   }
-  for (int id = nfull * 8 + t; id < V; id += kThreads) append((uint32_t)row[id], id);
-}
+  if (__ballot(some)) {
+    each_group([&](int r0, const uint2 (&kc)[kCntLoads][2]) {
+      int64_t v[8];
+      static_assert(kCntLoads == 8, "wave_sum8");
+      if (!big) {
+        double d[8];
+#pragma unroll
+        for (int r = 0; r < kCntLoads; ++r) d[r] = 0.0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if (__ballot(q[h][0] + q[h][1] + q[h][2] + q[h][3] != 0.0))
+#pragma unroll
+            for (int r = 0; r < kCntLoads; ++r)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) d[r] = __builtin_fma((double)count_of(kc[r], h, j), q[h][j], d[r]);
+#pragma unroll
+        for (int r = 0; r < kCntLoads; ++r) v[r] = (int64_t)d[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < kCntLoads; ++r) {
+          v[r] = 0;
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[r] += (int64_t)((uint64_t)count_of(kc[r], h, j) * (uint64_t)q[h][j]);
+        }
+      }
+      const int64_t m = wave_sum8(v);
+      if ((lane & 7) == 0 && r0 + (lane >> 3) < a.R) atomicAdd(&s.segm[r0 + (lane >> 3)], (unsigned long long)m);
+    });
+  }
+  __syncthreads();
+  const uint32_t cut_bits = pos < 2 * kMagBins ? pos_bits(pos) : 0x10000u;  // no cut key: equals no logit
+  const int64_t q_cut = mass_of(exp_of(cut_bits & 0xffffu, inv_t, zmax));
+  const int tie_cr = (int)((tie_word >> (16 * (pos & 1))) & 0xffffu);
+  const int tie_ex = wave_incl_scan_i(tie_cr) - tie_cr;
+  const int ties_r = max(0, min(tie_cr, cut_ties - tie_ex));
+  int64_t sm = seg_lane ? (int64_t)s.segm[lane] : 0;
+  if (seg_lane) sm += ties_r * q_cut + (has_mid && pos >= kMagBins ? s.midq[lane] : 0);
 
-XV_INLINE int64_t kept_mass_of(uint32_t bits, int id, uint32_t key_cut, int64_t id_cut, float inv_t, float zmax) {
-  const uint32_t key = order_key(bits);
-  const bool kept = key && (key > key_cut || (key == key_cut && (int64_t)id <= id_cut));
-  return kept ? mass_of(exp_of(bits, inv_t, zmax)) : 0;
-}
-
-// The draw of a row whose cut is made: the segment holding floor(u * M) by
-// the segments' kept masses, then in that segment, in id order, the first kept
-// id whose inclusive mass exceeds the rest of the draw point.  Each thread
-// takes a run of consecutive ids of the segment.
-constexpr int kDrawRegs = 16;  // ids per thread whose masses the draw keeps in registers
-XV_INLINE void row_draw(const SegArgs& a, Shared& s, const RowPlan& lp, const unsigned long long* segk, int b) {
-  const int t = threadIdx.x, lane = t & 63;
+  // the draw: the segment holding floor(u * M), then in id order the first
+  // kept id whose inclusive mass exceeds the rest.  Each thread sums a run of
+  // C consecutive ids; one wave then goes through the run that holds the point.
   const float u = a.uniforms ? a.uniforms[b] : 0.5f;
-  const int64_t rdraw = draw_point(u, lp.M);
-  // every wave finds the segment itself: R <= 64, one segment per lane
-  const int64_t sm = lane < a.R ? (int64_t)segk[lane] : 0;
+  const int64_t rdraw = draw_point(u, cut_m);
   const int64_t incl = wave_incl_scan_l(sm);
-  const int r = (int)wave_first(lane < a.R && rdraw < incl, kMaxSegs);
-  if (r >= a.R) {  // no kept mass (cannot happen for a row with a finite logit)
-    if (t == 0) a.out_ids[b] = 0;
-    return;
-  }
-  const int64_t rr = rdraw - (__shfl(incl, r) - (int64_t)segk[r]);
-  const uint32_t key_cut = lp.key_cut;
-  const int64_t id_cut = lp.id_cut;
-  const float inv_t = lp.inv_t, zmax = lp.zmax;
-  const bf16_t* row = a.logits + (int64_t)b * a.stride;
-  const bool vec_ok = ((reinterpret_cast<uintptr_t>(row) & 15u) == 0);
+  const int r = __builtin_amdgcn_readfirstlane(min((int)wave_first(seg_lane && rdraw < incl, kMaxSegs), a.R - 1));
+  const int64_t rr = rdraw - (__shfl(incl, r) - __shfl(sm, r));
+  const int ties = __builtin_amdgcn_readlane(ties_r, r);
   const int beg = r * a.seg_len, end = min(a.V, beg + a.seg_len);
   const int C = ((end - beg + kThreads - 1) / kThreads + 7) / 8 * 8;
   const int i0 = min(end, beg + t * C), i1 = min(end, i0 + C);
-  if (C <= kDrawRegs) {
-    // the thread's masses stay in registers for the second step
-    int64_t q[kDrawRegs];
+  // mass of an id before the cut key (0 for others)
+  const bool mid_kept = has_mid && pos >= kMagBins;
+  auto id_mass = [&](uint32_t bits) -> double {
+    const uint32_t mag = bits & 0x7fffu, m = mag - kMagLo;
+    if (m < (uint32_t)kMagBins) return qtab[(bits >> 15) * kMagBins + m];
+    return mid_kept && mag < kMagLo ? mass_d(exp_of(bits, inv_t, zmax)) : 0.0;
+  };
+  double mine_d = 0.0;
+  int mties = 0;
+  constexpr int kVecs = 4;  // vectors in flight
+  static_assert(kMaxSegIds / kThreads < (int)kExactIds, "a run's mass is exact in fp64");
+  for (int i = i0; i < i1; i += 8 * kVecs) {
+    uint32_t wd[kVecs][4];
 #pragma unroll
-    for (int v = 0; v < kDrawRegs / 8; ++v) {
-      uint32_t bits[8];
-      const int base = i0 + 8 * v;
-      if (base < i1) load8(row, i1, base, vec_ok, bits);  // i0 and C are multiples of 8
+    for (int v = 0; v < kVecs; ++v)
+      if (i + 8 * v < i1) load8_words(row, i1, i + 8 * v, vec_ok, wd[v]);  // ids past i1: NaN
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
-        q[8 * v + k] = base + k < i1 ? kept_mass_of(bits[k], base + k, key_cut, id_cut, inv_t, zmax) : 0;
+    for (int v = 0; v < kVecs; ++v)
+      if (i + 8 * v < i1)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const uint32_t bits = bits_of(wd[v], k);
+          mine_d += id_mass(bits);
+          mties += bits == cut_bits;
+        }
+  }
+  {
+    const int64_t mine = (int64_t)mine_d, mi = wave_incl_scan_l(mine);
+    const int ti = wave_incl_scan_i(mties);
+    if (lane == 63) {
+      s.cmass[w] = mi;
+      s.ccnt[w] = ti;
     }
-    int64_t mine = 0;
-#pragma unroll
-    for (int k = 0; k < kDrawRegs; ++k) mine += q[k];
-    int64_t seg_total;
-    int64_t cum = block_excl_scan(s, mine, &seg_total);
+    if (t == 0) s.t0 = -1;
     __syncthreads();
-    if (t == 0) s.b_id = -1;
-    __syncthreads();
-    if (cum <= rr && rr < cum + mine) {
-      int found = -1;
-#pragma unroll
-      for (int k = 0; k < kDrawRegs; ++k) {
-        cum += q[k];
-        if (found < 0 && cum > rr) found = i0 + k;
-      }
-      s.b_id = found;
-    }
-  } else {
-    auto scan_range = [&](auto&& f) {
-      for (int i = i0; i < i1; i += 8 * kSegChunk) {
-        uint32_t bits[kSegChunk][8];
-#pragma unroll
-        for (int v = 0; v < kSegChunk; ++v)
-          if (i + 8 * v < i1) load8(row, i1, i + 8 * v, vec_ok, bits[v]);
-#pragma unroll
-        for (int v = 0; v < kSegChunk; ++v)
-#pragma unroll
-          for (int k = 0; k < 8; ++k)
-            if (i + 8 * v + k < i1) f(bits[v][k], i + 8 * v + k);
-      }
-    };
-    int64_t mine = 0;
-    scan_range([&](uint32_t bits, int id) { mine += kept_mass_of(bits, id, key_cut, id_cut, inv_t, zmax); });
-    int64_t seg_total;
-    int64_t cum = block_excl_scan(s, mine, &seg_total);
-    __syncthreads();
-    if (t == 0) s.b_id = -1;
-    __syncthreads();
-    if (cum <= rr && rr < cum + mine) {
-      int64_t found = -1;
-      scan_range([&](uint32_t bits, int id) {
-        if (found >= 0) return;
-        cum += kept_mass_of(bits, id, key_cut, id_cut, inv_t, zmax);
-        if (cum > rr) found = id;
-      });
-      s.b_id = found;
+    const int64_t wm = lane < kWaves ? s.cmass[lane] : 0;
+    const int wt = lane < kWaves ? s.ccnt[lane] : 0;
+    const int64_t me = mi - mine + __shfl(wave_incl_scan_l(wm) - wm, w);
+    const int te = ti - mties + __shfl(wave_incl_scan_i(wt) - wt, w);
+    const int64_t cum = me + min(ties, te) * q_cut;
+    const int64_t upto = me + mine + min(ties, te + mties) * q_cut;
+    if (cum <= rr && rr < upto) {
+      s.t0 = t;
+      s.cum = cum;
+      s.tie = te;
     }
   }
   __syncthreads();
-  if (t == 0) a.out_ids[b] = s.b_id >= 0 ? s.b_id : 0;
+  if (t >= 64) return true;
+  const int t0 = s.t0;
+  int64_t cum = s.cum;
+  int te = s.tie;
+  const int j0 = min(end, beg + t0 * C), j1 = min(end, j0 + C);
+  for (int i = j0; t0 >= 0 && i < j1; i += 64) {
+    const uint32_t bits = i + lane < j1 ? (uint32_t)row[i + lane] : 0xffffu;
+    const bool tie = bits == cut_bits;
+    const int rank = te + __popcll(__ballot(tie) & ((1ull << lane) - 1));
+    const int64_t m = tie ? (rank < ties ? q_cut : 0) : (int64_t)id_mass(bits);
+    const int64_t inc = cum + wave_incl_scan_l(m);
+    const unsigned long long hit = __ballot(inc > rr);
+    if (hit) {
+      if (lane == 0) a.out_ids[b] = i + __builtin_ctzll(hit);
+      break;
+    }
+    cum = __shfl(inc, 63);
+    te += __popcll(__ballot(tie));
+  }
+  return true;
 }
 
-__global__ __launch_bounds__(kThreads) void row_finish_kernel(SegArgs a) {
+__global__ __launch_bounds__(kThreads) void row_count_kernel(SegArgs a) {
   __shared__ Shared s;
   __shared__ FastShared fs;
-  __shared__ RowPlan lp;
-  __shared__ unsigned long long segk[kMaxSegs];
-  __shared__ __attribute__((aligned(16))) uint32_t tie_ids[kTieRank];
-  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
+  __shared__ RowShared rs;
+  static_assert(kMaxCand >= 2 * kMagBins, "the candidate list's LDS holds the mass table");
+  const int b = blockIdx.x, t = threadIdx.x;
   const RowParams p = row_params(a, b);
   if (p.greedy) {  // the best of the segments' best words (torch.argmax order)
-    if (w == 0) {
-      const unsigned long long best = wave_max_ull(lane < a.R ? a.seg_best[b * a.R + lane] : 0ull);
-      if (lane == 0) a.out_ids[b] = best ? (int64_t)(0xffffffffu - (uint32_t)best) : 0;
+    if (t < 64) {
+      const unsigned long long best = wave_max_ull(t < a.R ? a.seg_best[b * a.R + t] : 0ull);
+      if (t == 0) a.out_ids[b] = best ? (int64_t)(0xffffffffu - (uint32_t)best) : 0;
     }
     return;
   }
-  // Every load the plan needs goes out before any is used: the row's segment
-  // statistics, and of bucket t % kBuckets the histogram entries of segments
-  // t / kBuckets + kGroups * j.  Segment indices past R reload segment R - 1
-  // (no branch between the loads) and are masked below.
-  constexpr int kGroups = kThreads / kBuckets, kSegPerGroup = kMaxSegs / kGroups;
-  static_assert(kGroups * kBuckets == kThreads && kSegPerGroup * kGroups == kMaxSegs, "bucket x segment layout");
-  const int bt = t & (kBuckets - 1), g = t / kBuckets;
-  uint32_t hc[kSegPerGroup];
-  unsigned long long hm[kSegPerGroup];
-#pragma unroll
-  for (int j = 0; j < kSegPerGroup; ++j) {
-    const int64_t o = ((int64_t)b * a.R + min(g + kGroups * j, a.R - 1)) * kBuckets + bt;
-    hc[j] = a.seg_cnt[o];
-    hm[j] = p.use_k ? 0ull : a.seg_mass[o];  // top-k rows take their masses from the list
-  }
-  const int sl = min(lane, a.R - 1);
-  const uint32_t kmax_l = a.seg_kmax[b * a.R + sl], kmin_l = a.seg_kmin[b * a.R + sl];
-  const uint32_t minp_l = a.seg_minp[b * a.R + sl];
-  const RowConsts rc = row_consts_of(lane < a.R ? kmax_l : 0u, lane < a.R ? kmin_l : 0xffffffffu, p.temp);
-  if (rc.kmax == 0) {  // every logit NaN: nothing has mass
-    if (t == 0) a.out_ids[b] = 0;
-    return;
-  }
-  if (!__builtin_isfinite(rc.zmax)) {  // no mass anywhere: the lowest id of the largest key
-    const bf16_t* row = a.logits + (int64_t)b * a.stride;
-    const int64_t id = lowest_id_of_key(s, row, a.V, ((reinterpret_cast<uintptr_t>(row) & 15u) == 0), rc.kmax);
-    if (t == 0) a.out_ids[b] = id;
-    return;
-  }
-  const uint32_t kminp = wave_min_u(lane < a.R ? minp_l : 0xffffffffu);
-  if (t < kMaxSegs) segk[t] = 0ull;  // (ordered before its atomics by the scan's barriers)
-  {  // each group's partial sums of the buckets, then thread t < kBuckets adds the groups'
-    uint32_t c = 0;
-    unsigned long long m = 0;
-#pragma unroll
-    for (int j = 0; j < kSegPerGroup; ++j)
-      if (g + kGroups * j < a.R) {
-        c += hc[j];
-        m += hm[j];
-      }
-    fs.wcnt[g][bt] = c;
-    fs.wmass[g][bt] = m;
-  }
-  __syncthreads();
-  int64_t cnt = 0, mass = 0;
-  if (t < kBuckets) {
-#pragma unroll
-    for (int gg = 0; gg < kGroups; ++gg) {
-      cnt += fs.wcnt[gg][t];
-      mass += p.use_k ? 0 : (int64_t)fs.wmass[gg][t];
-    }
-  }
-  int64_t cnt_excl, mass_excl, cnt_all, total;
-  block_excl_scan2(s, cnt, mass, &cnt_excl, &mass_excl, &cnt_all, &total);
-  const int64_t cnt_incl = cnt_excl + cnt, mass_incl = mass_excl + mass;
-  int status = kPlanDraw, lo = 0, hi = 0, cut_p = 0, cut_m = 0;
-  int64_t thr = 0, m_before = 0;
-  if (p.use_k) {
-    // rank k-1 lies in the first bucket whose inclusive count reaches k
-    const int bk = (int)block_min_l(s, (t < kBuckets && cnt_incl >= p.top_k) ? t : kBuckets);
-    __syncthreads();
-    if (t == bk) s.b_long[0] = cnt_incl;  // candidates in buckets 0..bk
-    __syncthreads();
-    const int64_t upto = bk < kBuckets ? s.b_long[0] : 0;
-    status = (bk >= kBuckets - 1 || upto > kMaxCand) ? kPlanFallback : kPlanGather;
-    hi = bk;
-  } else if (p.use_p || p.use_m) {
-    int bp = kBuckets;
-    if (p.use_p) {
-      thr = (int64_t)floor((double)p.top_p * (double)total);
-      bp = (int)block_min_l(s, (t < kBuckets && mass_incl > thr) ? t : kBuckets);
-    }
-    int bm = kBuckets;
-    if (p.use_m && kminp != 0xffffffffu) bm = bucket_of(log2_ratio(key_to_bits(kminp), rc.inv_t, rc.zmax), rc.bs);
-    const int bf = min(bp, bm);
-    if (bf < kBuckets) {
-      __syncthreads();
-      if (t == bf) {
-        s.b_long[0] = cnt;
-        s.b_long[1] = mass_incl - mass;  // mass of the buckets before bf
-      }
-      __syncthreads();
-      m_before = s.b_long[1];
-      status = s.b_long[0] > kMaxCand ? kPlanFallback : kPlanGather;
-      lo = hi = bf;
-      cut_p = bp == bf;
-      cut_m = bm == bf;
-    }
-  }
-  bool fallback = status == kPlanFallback;  // the boundary does not fit in LDS
-  if (t == 0) {
-    lp.status = status;
-    lp.use_k = p.use_k;
-    lp.cut_p = cut_p;
-    lp.cut_m = cut_m;
-    lp.kminp = kminp;
-    lp.zmax = rc.zmax;
-    lp.inv_t = rc.inv_t;
-    lp.thr = thr;
-    lp.mp_before = m_before;
-    lp.m_before = m_before;
-    lp.key_cut = 1u;  // no cut: every candidate kept
-    lp.id_cut = kTieAll;
-    lp.M = total;
-    fs.ncand = 0;
-  }
-  if (fallback) {
-  } else if (status == kPlanDraw) {  // no cut: the segments' total masses are their kept masses
-    if (t < a.R) segk[t] = (unsigned long long)a.seg_kept[b * a.R + t];
-  } else {
-    // Buckets fall as keys rise over the keys of non-NaN values, so buckets
-    // lo..hi hold exactly the keys of an interval: its ends by the same bucket
-    // function.
-    auto bkt = [&](uint32_t k) { return bucket_of(log2_ratio(key_to_bits(k), rc.inv_t, rc.zmax), rc.bs); };
-    if (w == 0) {
-      const uint32_t klo = wave_first_key([&](uint32_t k) { return bkt(k) <= hi; });
-      if (lane == 0) lp.klo = klo;
-    } else if (w == 1) {
-      const uint32_t kend = wave_first_key([&](uint32_t k) { return bkt(k) < lo; });
-      if (lane == 0) lp.khi = kend - 1;
-    }
-    // rows without top-k: each segment's mass of the buckets before lo (all
-    // of whose candidates are kept; the list's part is added by the cut)
-    if (!p.use_k) {
-#pragma unroll
-      for (int j = 0; j < kSegPerGroup; ++j) {
-        const int r = g + kGroups * j;
-        const int64_t v = wave_sum_l((r < a.R && bt < lo) ? (int64_t)hm[j] : 0);
-        if (lane == 0 && r < a.R) atomicAdd(&segk[r], (unsigned long long)v);
-      }
-    }
-  }
-  __syncthreads();
-  if (status == kPlanGather) {
-    const bf16_t* row = a.logits + (int64_t)b * a.stride;
-    const bool vec_ok = ((reinterpret_cast<uintptr_t>(row) & 15u) == 0);
-    const uint32_t klo = lp.klo, khi = lp.khi;
-    if (klo <= khi) gather_key_range(fs, row, a.V, vec_ok, klo, khi);
-    __syncthreads();
-    const int n = fs.ncand;
-    // the cut's bucket holds its own boundary candidate, and the histograms
-    // counted the list; should either fail, the one-workgroup path takes the row
-    const float inv_t = rc.inv_t, zmax = rc.zmax;
-    if (n == 0 || n > kMaxCand) {
-      fallback = true;
-    } else if (n <= 64) {
-      if (t < 64) row_cut_wave_list(a, lp, p, b, n, lane < n ? fs.cand[lane] : 0ull, segk);
-    } else if (p.use_k || !row_cut_by_keys(a, lp, s, fs, n, tie_ids, segk)) {
-      sort_cand_desc(fs, n);
-      int64_t jcut;
-      if (p.use_k) {
-        // the list is every candidate down to rank k-1 (as topk_boundary)
-        const int64_t total_k = list_mass_prefix(s, fs, n, p.top_k, inv_t, zmax);
-        jcut = (int64_t)p.top_k - 1;
-        if (p.use_p) {
-          const int64_t thr_k = (int64_t)floor((double)p.top_p * (double)total_k);
-          jcut = min(jcut, list_first_exceed(s, fs, n, 0, thr_k, inv_t, zmax));
-        }
-        if (p.use_m && kminp != 0xffffffffu && kminp >= cand_key(fs.cand[n - 1]))
-          jcut = min(jcut, list_count_ge(s, fs, n, kminp) - 1);
-      } else {
-        // the list is the bucket of the earliest cut (as fast_boundary)
-        jcut = kTieAll;
-        if (cut_p) jcut = min(jcut, list_first_exceed(s, fs, n, m_before, thr, inv_t, zmax));
-        if (cut_m) jcut = min(jcut, list_count_ge(s, fs, n, kminp) - 1);
-      }
-      if (jcut >= n) jcut = n - 1;
-      if (jcut < 0) jcut = 0;
-      const unsigned long long edge = fs.cand[jcut];
-      if (p.use_k) {
-        const int64_t M = list_mass_prefix(s, fs, n, jcut + 1, inv_t, zmax);
-        const float u = a.uniforms ? a.uniforms[b] : 0.5f;
-        const int64_t found = list_draw(s, fs, (int)jcut + 1, inv_t, zmax, draw_point(u, M));
-        if (t == 0) {
-          a.out_ids[b] = found == kTieAll ? 0 : found;
-          lp.status = kPlanDone;
-        }
-      } else {
-        const int64_t M = m_before + list_mass_prefix(s, fs, n, jcut + 1, inv_t, zmax);
-        for (int i = t; i <= jcut; i += kThreads)
-          atomicAdd(&segk[cand_id(fs.cand[i]) / a.seg_len], (unsigned long long)cand_mass(fs.cand[i], inv_t, zmax));
-        if (t == 0) {
-          lp.key_cut = cand_key(edge);
-          lp.id_cut = cand_id(edge);
-          lp.M = M;
-          lp.status = kPlanDraw;
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (fallback) {
-    sample_row(s, fs, b, a.logits, a.stride, a.V, a.temps, a.top_ps, a.top_ks, a.min_ps, a.uniforms,
+  if (!row_from_counts(a, p, rs, reinterpret_cast<double*>(fs.cand), b)) {
+    int rb = b;
+    __asm__ volatile("" : "+s"(rb)::"memory");
+    sample_row(s, fs, rb, a.logits, a.stride, a.V, a.temps, a.top_ps, a.top_ks, a.min_ps, a.uniforms,
                a.flags & ~XV_SAMPLE_ALL_GREEDY, a.out_ids);
-    return;
   }
-  if (lp.status == kPlanDraw) row_draw(a, s, lp, segk, b);
 }
 }  // namespace
 
 // Workspace: one 128-byte line per row (a 64-bit slot and a 32-bit arrival
-// counter) for the multi-workgroup greedy path, then the per-segment
-// statistics and histograms of the multi-workgroup sampled path, and room for
-// kMaxCand candidates per row, which the top-k path's lists use (it sets how
-// many rows that path takes; the sampled path keeps its candidates in LDS).
+// counter) for the multi-workgroup greedy path, then the segments' counts of
+// the multi-workgroup sampled path, or room for kMaxCand candidates per row,
+// which the top-k path's lists use (it sets how many rows that path takes).
 namespace {
 struct SegLayout {
   int R, seg_len;
-  size_t kmax, kmin, minp, best, kept, cnt, mass, cand, total;
+  size_t best, cnt, total;
 };
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 SegLayout seg_layout(int batch, int vocab) {
   SegLayout L;
-  // about 2048 segment workgroups in all, at least 2048 ids per segment
-  int segs = max(1, min(kMaxSegs, XV_SEG_TARGET / max(batch, 1)));
+  int segs = max(1, min(kCntSegs, kCntTarget / max(batch, 1)));
   segs = max(1, min(segs, vocab / 2048));
+  segs = max(segs, (vocab + kMaxSegIds - 1) / kMaxSegIds);
   L.seg_len = ((vocab + segs - 1) / segs + 7) / 8 * 8;
   L.R = (vocab + L.seg_len - 1) / L.seg_len;
   const size_t B = (size_t)max(batch, 0), BR = B * L.R;
   size_t o = 0;  // offsets within the sampled path's region
-  L.kmax = o;  o = align256(o + BR * 4);
-  L.kmin = o;  o = align256(o + BR * 4);
-  L.minp = o;  o = align256(o + BR * 4);
   L.best = o;  o = align256(o + BR * 8);
-  L.kept = o;  o = align256(o + BR * 8);
-  L.cnt = o;   o = align256(o + BR * kBuckets * 4);
-  L.mass = o;  o = align256(o + BR * kBuckets * 8);
-  L.cand = o;  o = align256(o + B * kMaxCand * 8);
-  L.total = o;
+  L.cnt = o;   o = align256(o + BR * kSegWords * 4);
+  L.total = max(o, align256(B * kMaxCand * 8));  // at least the top-k path's lists
   return L;
 }
 
@@ -2707,27 +2462,20 @@ extern "C" int xv_sample(const void* logits, int64_t logits_stride, int batch, i
   }
   // Sampled (or mixed) batches of up to kSegMaxBatch rows: several workgroups
   // per row.  Larger batches take one workgroup per row.
-  if (workspace != nullptr && batch <= kSegMaxBatch && workspace_bytes >= xv_sampler_workspace_size(batch, vocab)) {
+  if (workspace != nullptr && batch <= kSegMaxBatch && vocab <= kMaxSegs * kMaxSegIds &&
+      workspace_bytes >= xv_sampler_workspace_size(batch, vocab)) {
     const SegLayout L = seg_layout(batch, vocab);
     char* w = (char*)workspace + ((workspace_bytes - L.total) & ~(size_t)255);  // region at the top
-    SegArgs a;
+    SegArgs a = {};
     a.logits = (const bf16_t*)logits; a.stride = logits_stride;
     a.V = vocab; a.R = L.R; a.seg_len = L.seg_len; a.flags = flags & ~XV_SAMPLE_ALL_GREEDY;
     a.temps = temperatures; a.top_ps = top_ps; a.top_ks = top_ks; a.min_ps = min_ps; a.uniforms = uniforms;
     a.out_ids = out_ids;
-    a.seg_kmax = (uint32_t*)(w + L.kmax);
-    a.seg_kmin = (uint32_t*)(w + L.kmin);
-    a.seg_minp = (uint32_t*)(w + L.minp);
     a.seg_best = (unsigned long long*)(w + L.best);
-    a.seg_kept = (int64_t*)(w + L.kept);
     a.seg_cnt = (uint32_t*)(w + L.cnt);
-    a.seg_mass = (unsigned long long*)(w + L.mass);
-    const dim3 segs((unsigned)L.R, (unsigned)batch), rows((unsigned)batch);
-    seg_stats_kernel<<<segs, kSegThreads, 0, stream>>>(a);
+    seg_count_kernel<<<dim3((unsigned)L.R, (unsigned)batch), kThreads, 0, stream>>>(a);
     XV_CHECK_LAUNCH();
-    seg_hist_kernel<<<segs, kSegThreads, 0, stream>>>(a);
-    XV_CHECK_LAUNCH();
-    row_finish_kernel<<<rows, kThreads, 0, stream>>>(a);
+    row_count_kernel<<<dim3((unsigned)batch), kThreads, 0, stream>>>(a);
     XV_CHECK_LAUNCH();
     return 0;
   }
