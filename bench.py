@@ -384,8 +384,8 @@ def decode_e2e(torch, dev, ctx: list[int], steps: int = 20, sampled: bool = Fals
     given per-sequence contexts: hipGraph replay of the decode body + LM head +
     sampler, steady state (metadata staged once).  fp8: the KV pool in the
     optional fp8 (e4m3fn) page format.  stream_gemms: the runner's opt-in
-    weight-streaming decode GEMMs (packed copies of gate_up / down / o beside
-    the weights; their bytes are reported).  Returns (record, model)."""
+    streaming of every decode product (the bytes of packed copies beside the
+    weights, if any, are reported).  Returns (record, model)."""
     from xvllm.batch import SeqSchedule
     from xvllm.config import QWEN3_8B
     from xvllm.kv_pool import KVPool
@@ -454,8 +454,9 @@ def decode_e2e(torch, dev, ctx: list[int], steps: int = 20, sampled: bool = Fals
     assert ids.shape[0] == bsz
     return {"batch": bsz, "mean_ctx": round(sum(ctx) / bsz, 1), "sampling": "T0.7/k50/p0.9" if sampled else "greedy",
             "kv_pages": "fp8 e4m3fn" if fp8 else "bf16",
-            "dense_gemms": ("weight-streaming kernel at <= 64 rows (opt-in), packed weight copies of "
-                            f"{packed} B beside the weights") if stream_gemms else "PyTorch / hipBLASLt",
+            "dense_gemms": ("weight-streaming kernel in place at <= 256 rows, every product; packed weight copies of "
+                            f"{packed} B beside the weights") if stream_gemms else
+                           "weight-streaming kernel in place (gate_up, qkv, split o and down), LM head PyTorch / hipBLASLt",
             "ms_per_step": round(ms, 4), "tok_per_s": round(bsz / (ms * 1e-3), 1),
             "roofline_ms": round(roof_ms, 4), "roofline_tok_per_s": round(bsz / (roof_ms * 1e-3), 1),
             "frac_of_roofline": round(roof_ms / ms, 4), "weight_bytes": wbytes, "kv_bytes": kvbytes}, model
@@ -1022,7 +1023,7 @@ def main() -> int:
         line["decode_tok_per_s"] = line["decode_e2e"]["tok_per_s"]
         # the same step on an fp8 (e4m3fn) KV pool, the pool's optional page format
         line["decode_e2e_fp8"], model = decode_e2e(torch, dev, ctx, fp8=True, model=model)
-        # the opt-in weight-streaming decode GEMMs (12.1 GB of packed weights beside the 16.4 GB of weights)
+        # the opt-in streaming of every decode product (the record says what packed copies it holds)
         line["decode_e2e_streamed_gemms"], model = decode_e2e(torch, dev, ctx, model=model, stream_gemms=True)
         del model
         torch.cuda.empty_cache()
