@@ -125,3 +125,42 @@ def test_mlp_streams_and_matches_the_library(dev, m, width):
         got = (out.materialize() if isinstance(out, PartialSums) else out).double()
         rel = (got - want).norm() / want.norm()
         assert rel < 1e-2, f"relative L2 {rel:.3g}"
+
+
+@pytest.mark.parametrize("m", [8, 40, 100])
+def test_layouts_the_library_takes(dev, m):
+    """x whose rows are expanded or overlap, and weights that are expanded,
+    overlap or start off a 16-byte boundary, give the library's product."""
+    import torch.nn.functional as F
+
+    from xvllm.layers.linear import PartialSums
+    from xvllm.models.qwen3 import Qwen3MLP
+
+    h, inter = 1024, 3072
+    g = torch.Generator(device=dev).manual_seed(m)
+
+    def randn(*shape, std=1.0):
+        return (torch.randn(shape, generator=g, device=dev) * std).to(torch.bfloat16)
+
+    flat = randn(8 * m + h)
+    off = torch.from_dlpack(randn(2 * inter * h + 3, std=0.02)[3:])  # a storage of its own, off by 6 bytes
+    assert off.storage_offset() == 0 and off.data_ptr() % 16
+    weights = {"plain": randn(2 * inter, h, std=0.02), "expanded": randn(1, h, std=0.02).expand(2 * inter, h),
+               "overlapping": randn(2 * inter * 8 + h, std=0.02).as_strided((2 * inter, h), (8, 1)),
+               "off": off.view(2 * inter, h)}
+    with torch.device(dev):
+        mlp = Qwen3MLP(h, inter).to(torch.bfloat16)
+    with torch.no_grad():
+        mlp.down_proj.copy_(randn(h, inter, std=0.02))
+        for name, w in weights.items():
+            mlp.gate_up_proj = torch.nn.Parameter(w, requires_grad=False)
+            for x in (randn(m, h), randn(1, h).expand(m, h), flat.as_strided((m, h), (8, 1)), randn(h, m).t()):
+                print(f"layouts m {m} w {name} x stride {tuple(x.stride())}", flush=True)
+                out = mlp(x)
+                out = out.materialize() if isinstance(out, PartialSums) else out
+                gu = F.linear(x.contiguous(), w.contiguous()).double()
+                act = (gu[:, :inter] * torch.sigmoid(gu[:, :inter]) * gu[:, inter:]).to(torch.bfloat16)
+                want = F.linear(act, mlp.down_proj)
+                # both sides round g, u, the activation and the product to bf16: 2^-8 each
+                rel = (out.double() - want.double()).norm() / want.double().norm()
+                assert rel < 4 * 2.0**-8, (name, tuple(x.stride()), rel.item())

@@ -52,6 +52,7 @@ from typing import NamedTuple
 
 import torch
 import torch.nn.functional as F
+from torch._subclasses.fake_tensor import FakeTensor
 
 
 class PartialSums(NamedTuple):
@@ -248,7 +249,7 @@ def _stream_gemm(x: torch.Tensor, w: torch.Tensor, mode: int, parts: int) -> tor
     n = w.shape[0]
     if w.shape[1] != k:
         raise ValueError(f"stream_gemm: x {tuple(x.shape)} and w {tuple(w.shape)} disagree on K")
-    if x.stride(1) != 1 or x.stride(0) % 8 or not aligned16(x):
+    if x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < k or not aligned16(x):  # (expanded and overlapping rows: stride < K)
         x = x.clone(memory_format=torch.contiguous_format)
     if w.stride(1) != 1:
         raise ValueError("stream_gemm: w needs unit stride along K")
@@ -274,6 +275,15 @@ def _stream_gemm_fake(x, w, mode, parts):
     return x.new_empty((m, n // 2))
 
 
+def _streams_in_place(w: torch.Tensor) -> bool:
+    """Whether w [N, K] has the layout xv_stream_gemm reads: rows of unit
+    stride, whole (not expanded, not overlapping) and 16-byte aligned."""
+    if w.stride(1) != 1 or w.stride(0) % 8 or w.stride(0) < w.shape[1] or w.storage_offset() % 8:
+        return False
+    # a storage need not start aligned (memory imported from elsewhere); a traced tensor has no address
+    return isinstance(w, FakeTensor) or w.data_ptr() % 16 == 0
+
+
 def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int, *, internal: bool = False):
     """What streamed_silu_mul / streamed_into_norm read the weight w [N, K]
     from for activations x: w itself where the in-place kernel takes the
@@ -284,7 +294,7 @@ def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int, *, inter
     norm stream only there (unless they stay `internal` to the layer); and with gradients asked of x or w the library
     keeps the product (streaming has no backward; a packed model is inference
     only)."""
-    if not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2:
+    if not x.is_cuda or x.device != w.device or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2:
         return None
     m, k = x.shape
     n = w.shape[0]
@@ -293,8 +303,7 @@ def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int, *, inter
             return None
         if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
             return None
-    if (w.stride(1) == 1 and w.stride(0) % 8 == 0 and w.storage_offset() % 8 == 0
-            and in_place_parts(m, n, k, mode) > 0):
+    if _streams_in_place(w) and in_place_parts(m, n, k, mode) > 0:
         return w
     return packed if isinstance(packed, PackedWeight) and stream_rows(x) else None
 
