@@ -72,3 +72,43 @@ def test_rejects_bad_arguments(dev):
         call(torch.zeros((9, 3, (hq + 2 * hkv) * D), device=dev))
     with pytest.raises(RuntimeError):  # a zero fp8 scale
         call(good, cache=_cache(dev, 2, 16, hkv, False, torch.float8_e4m3fn), scale=0.0)
+
+
+def _decode_attention(dev, rows, slack=0, seed=0):
+    """A decode call of one Qwen3Attention (1024 wide, 16 q / 8 kv heads) whose
+    qkv product streams: (layer, its arguments, the pool's attention context)."""
+    from xvllm.config import Qwen3Shape
+    from xvllm.kv_pool import KVPool
+    from xvllm.layers.attention import AttnInputs, AttnMetadata, attention_context
+    from xvllm.models.qwen3 import Qwen3Attention
+
+    cfg = Qwen3Shape(1024, 16, 8, D, 3072, 1, max_position_embeddings=1024)
+    g = torch.Generator(device=dev).manual_seed(seed)
+    with torch.device(dev):
+        layer = Qwen3Attention(cfg, 0).to(torch.bfloat16)
+    with torch.no_grad():
+        layer.qkv_proj.normal_(0.0, 0.02, generator=g)
+        layer.o_proj.normal_(0.0, 0.02, generator=g)
+        hidden = torch.randn((rows, 1024), generator=g, device=dev).to(torch.bfloat16)
+    pool = KVPool(cfg, num_blocks=4 * rows, block_size=16, device=dev, dtype=torch.bfloat16)
+    pool.kv_cache.normal_(generator=g)
+    lens = torch.randint(1, 64, (rows,), generator=g, device=dev, dtype=torch.int32)
+    bt = torch.arange(4 * rows, dtype=torch.int32, device=dev).view(rows, 4)
+    last = (lens - 1).long()
+    slots = bt.gather(1, (last // 16)[:, None])[:, 0] * 16 + (last % 16).to(torch.int32)
+    pad = lambda t, value: torch.cat([t, t.new_full((slack,), value)])  # noqa: E731
+    attn = AttnInputs(slot_mapping=pad(slots, -1), is_prefill=False, block_tables=bt, cache_seqlens=lens)
+    return layer, (pad(last, 0), hidden, attn), pool, attention_context(AttnMetadata(kv_cache=pool.kv_cache))
+
+
+@pytest.mark.parametrize("rows", [3, 64])
+def test_decode_takes_buffers_of_a_larger_batch(dev, rows):
+    """Positions and slots longer than the batch: its own rows are read, as
+    the store of the unsplit product does."""
+    outs = []
+    for slack in (0, 9):
+        layer, args, pool, ctx = _decode_attention(dev, rows, slack)
+        with torch.no_grad(), ctx:
+            out = layer(*args)
+        outs.append((getattr(out, "parts", out), pool.kv_cache))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])

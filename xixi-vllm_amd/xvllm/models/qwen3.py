@@ -162,9 +162,10 @@ class Qwen3Attention(nn.Module):
     def _norm_rope_store_parts(self, positions, parts, slot_mapping):
         k_cache, v_cache = kv_cache_of(self.attn.layer_id)
         ks, vs = kv_scales()
+        t = parts.shape[1]  # positions and slots may come from buffers of a larger batch
         return torch.ops.xv.qk_norm_rope_store_parts(
-            parts, self.num_heads, self.q_norm.weight, self.k_norm.weight, self.eps, positions,
-            self.rotary_emb.cos_sin_cache, k_cache, v_cache, slot_mapping, ks, vs,
+            parts, self.num_heads, self.q_norm.weight, self.k_norm.weight, self.eps, positions.reshape(-1)[:t],
+            self.rotary_emb.cos_sin_cache, k_cache, v_cache, slot_mapping.reshape(-1)[:t], ks, vs,
         )
 
     def _split_norm_rope(self, positions, qkv):
