@@ -112,3 +112,42 @@ def test_decode_takes_buffers_of_a_larger_batch(dev, rows):
             out = layer(*args)
         outs.append((getattr(out, "parts", out), pool.kv_cache))
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("how", ["pre_hook", "hook", "global", "forward"])
+def test_observers_of_attention_see_k_and_v(dev, how):
+    """Hooks on the decoder's Attention, and a forward in its place, get the
+    projection's k and v [T, Hkv, D], and the output does not change."""
+    import torch.nn.functional as F
+
+    rows = 5
+    layer, args, _, ctx = _decode_attention(dev, rows)
+    seen = []
+
+    def see(*a):
+        inputs = a if how == "forward" else a[1]
+        if how != "global" or a[0] is layer.attn:
+            seen.append((inputs[1], inputs[2]))
+
+    with torch.no_grad(), ctx:
+        plain = layer(*args)
+        if how == "pre_hook":
+            handle = layer.attn.register_forward_pre_hook(see)
+        elif how == "hook":
+            handle = layer.attn.register_forward_hook(see)
+        elif how == "global":
+            handle = torch.nn.modules.module.register_module_forward_pre_hook(see)
+        else:
+            own, handle = layer.attn.forward, None
+            layer.attn.forward = lambda *a: (see(*a), own(*a))[1]
+        out = layer(*args)
+        if handle is not None:
+            handle.remove()
+        qkv = F.linear(args[1].double(), layer.qkv_proj.double())
+    (k, v), = seen
+    for got, want in ((k, qkv[:, layer.q_size : layer.q_size + layer.kv_size]), (v, qkv[:, layer.q_size + layer.kv_size :])):
+        assert got.shape == (rows, layer.num_kv_heads, D) and got.dtype == torch.bfloat16
+        # an fp32 sum rounded to bf16 once
+        err = (got.double().reshape(rows, -1) - want).norm() / want.norm()
+        assert err < 2.0**-8, err.item()
+    assert torch.equal(getattr(out, "parts", out), getattr(plain, "parts", plain))

@@ -60,6 +60,13 @@ def _decode_operand(p: nn.Parameter, mode: int):
     return pack_weight(p.data) if _needs_copy(p, mode) else p.data
 
 
+def _is_observed(attn: nn.Module) -> bool:
+    """Whether something besides Attention.forward sees the arguments of a
+    call of `attn`: hooks, or a module or a forward put in its place."""
+    return bool(type(attn) is not Attention or "forward" in vars(attn) or attn._forward_hooks or attn._forward_pre_hooks
+                or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks)
+
+
 class Qwen3MLP(nn.Module):
     def __init__(self, hidden: int, inter: int):
         super().__init__()
@@ -117,10 +124,14 @@ class Qwen3Attention(nn.Module):
         w = None if attn.is_prefill or not self.split_k else stream_operand(hidden, self.qkv_proj, None, GEMM_PARTS,
                                                                             internal=True)
         if w is not None:
-            # decode: the qkv partial sums go into norm + RoPE + KV store (k and v reach attention through the cache)
-            q = self._norm_rope_store_parts(positions, streamed_into_norm(hidden, w).parts, attn.slot_mapping)
-            q = q.view(q.shape[0], self.q_size)
-            o = self.attn(q, q, q, attn._replace(slot_mapping=None))
+            # decode: the qkv partial sums go into norm + RoPE + KV store
+            qkv = streamed_into_norm(hidden, w)
+            q = self._norm_rope_store_parts(positions, qkv.parts, attn.slot_mapping)
+            q = k = v = q.view(q.shape[0], self.q_size)
+            if _is_observed(self.attn):
+                _, k, v = self._views(qkv.materialize())
+            # Attention itself takes k and v from the cache (no slots to store at) and reads neither argument
+            o = self.attn(q, k, v, attn._replace(slot_mapping=None))
         elif not attn.is_prefill:
             # decode: norm + RoPE + KV store in one kernel, attention reads the cache
             q, k, v = self._split_norm_rope_store(positions, F.linear(hidden, self.qkv_proj), attn.slot_mapping)
