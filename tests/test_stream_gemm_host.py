@@ -83,3 +83,23 @@ def test_fake_shapes():
         act = torch.ops.xv.stream_gemm(x, w, GEMM_SILU_MUL, 1)
     assert parts.shape == (2, 5, 6144) and parts.dtype == torch.float32
     assert act.shape == (5, 3072) and act.dtype == torch.bfloat16
+
+
+def test_long_batches_do_not_ask_the_library(monkeypatch):
+    """Above 256 rows the choice falls on the row count alone: a prefill
+    step's layers ask for each of their products."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from xvllm.layers import linear
+
+    asked = []
+    monkeypatch.setattr(linear, "in_place_parts", lambda *a: asked.append(a) or 1)
+    with FakeTensorMode():
+        w = torch.empty(6144, 1024, dtype=torch.bfloat16, device="cuda")
+        for m in (0, 1, 256, 257, 8192):
+            x = torch.empty(m, 1024, dtype=torch.bfloat16, device="cuda")
+            for packed in (None, w):
+                for mode in (linear.GEMM_PARTS, linear.GEMM_SILU_MUL):
+                    got = linear.stream_operand(x, w, packed, mode, internal=True)
+                    assert (got is w) == (0 < m <= 256)
+    assert {a[0] for a in asked} == {1, 256}

@@ -205,7 +205,8 @@ def stream_parts(k: int) -> int:
     return 0
 
 
-# Rows up to which a packed weight is streamed (xv_dense_gemm).
+# Rows up to which a weight is streamed in place (xv_stream_gemm), and from a packed copy (xv_dense_gemm).
+IN_PLACE_MAX_ROWS = 256
 STREAM_MAX_ROWS = 64
 
 
@@ -294,7 +295,9 @@ def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int, *, inter
     norm stream only there (unless they stay `internal` to the layer); and with gradients asked of x or w the library
     keeps the product (streaming has no backward; a packed model is inference
     only)."""
-    if not x.is_cuda or x.device != w.device or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2:
+    if x.dim() != 2 or not 0 < x.shape[0] <= IN_PLACE_MAX_ROWS:  # first: a prefill step's layers ask three times each
+        return None
+    if not x.is_cuda or x.device != w.device or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return None
     m, k = x.shape
     n = w.shape[0]
