@@ -164,3 +164,27 @@ def test_layouts_the_library_takes(dev, m):
                 # both sides round g, u, the activation and the product to bf16: 2^-8 each
                 rel = (out.double() - want.double()).norm() / want.double().norm()
                 assert rel < 4 * 2.0**-8, (name, tuple(x.stride()), rel.item())
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("m", [8, 100, 300])
+def test_compiles_as_one_graph(dev, m, packed):
+    """torch.compile traces the MLP without a break at every row count, onto
+    the library's products (Qwen3-0.6B, whose products the library does not split)."""
+    from xvllm.models.qwen3 import Qwen3MLP
+
+    g = torch.Generator(device=dev).manual_seed(m)
+    with torch.device(dev):
+        mlp = Qwen3MLP(1024, 3072).to(torch.bfloat16)
+    with torch.no_grad():
+        for p in mlp.parameters():
+            p.normal_(0.0, 0.02, generator=g)
+        x = torch.randn((m, 1024), generator=g, device=dev).to(torch.bfloat16)
+        mlp.split_k = False
+        want = mlp(x)
+        mlp.split_k = True
+        if packed and m > 64:  # (a packed model's shorter batches check their weights, which no trace holds)
+            mlp.pack()
+        torch._dynamo.reset()
+        got = torch.compile(mlp, backend="eager", fullgraph=True)(x)
+    assert torch.equal(got, want)

@@ -289,12 +289,14 @@ def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int, *, inter
     """What streamed_silu_mul / streamed_into_norm read the weight w [N, K]
     from for activations x: w itself where the in-place kernel takes the
     shape, else its packed copy (if it has one) up to STREAM_MAX_ROWS rows,
-    else None (the library GEMM).  `packed` is the operand a packed model
+    else None (the library GEMM; also under torch.compile).  `packed` is the operand a packed model
     holds, None for a model that was not packed.  Such a model's callers get
     PartialSums only where linear_into_norm splits, so its products into a
     norm stream only there (unless they stay `internal` to the layer); and with gradients asked of x or w the library
     keeps the product (streaming has no backward; a packed model is inference
     only)."""
+    if torch.compiler.is_compiling():  # the shape rule is a C call, which a compiler's trace cannot hold
+        return None
     if x.dim() != 2 or not 0 < x.shape[0] <= IN_PLACE_MAX_ROWS:  # first: a prefill step's layers ask three times each
         return None
     if not x.is_cuda or x.device != w.device or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
