@@ -188,3 +188,37 @@ def test_compiles_as_one_graph(dev, m, packed):
         torch._dynamo.reset()
         got = torch.compile(mlp, backend="eager", fullgraph=True)(x)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m,packed", [(8, False), (64, False), (100, False), (100, True), (256, True)])
+def test_gradients_keep_the_library(dev, m, packed):
+    """With gradients on, an unpacked MLP's products and a packed one's above
+    64 rows carry them (Qwen3-0.6B, whose products the library does not split;
+    silu_and_mul has no backward, so gate_up is frozen)."""
+    from xvllm.layers.linear import GEMM_PARTS, stream_operand
+    from xvllm.models.qwen3 import Qwen3MLP
+
+    g = torch.Generator(device=dev).manual_seed(m)
+    with torch.device(dev):
+        mlp = Qwen3MLP(1024, 3072).to(torch.bfloat16)
+    mlp.gate_up_proj.requires_grad_(False)
+    with torch.no_grad():
+        for p in mlp.parameters():
+            p.normal_(0.0, 0.02, generator=g)
+    x = torch.randn((m, 1024), generator=g, device=dev).to(torch.bfloat16)
+    go = torch.randn((m, 1024), generator=g, device=dev).to(torch.bfloat16)
+    mlp.split_k = False
+    want, = torch.autograd.grad(mlp(x), mlp.down_proj, go)
+    mlp.split_k = True
+    mlp.pack(packed)
+    out = mlp(x)
+    assert isinstance(out, torch.Tensor) and out.requires_grad
+    got, = torch.autograd.grad(out, mlp.down_proj, go)
+    # gate_up streams, so the activation behind the gradient is one bf16 rounding apart
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() < 2 * 2.0**-8
+    # the decode step's qkv product, which stays internal to its layer
+    w = torch.nn.Parameter(torch.randn((4096, 1024), generator=g, device=dev).to(torch.bfloat16))
+    assert stream_operand(x, w, None, GEMM_PARTS, internal=True) is None
+    assert stream_operand(x.clone().requires_grad_(), w.detach(), None, GEMM_PARTS, internal=True) is None
+    with torch.no_grad():
+        assert stream_operand(x, w, None, GEMM_PARTS, internal=True) is w

@@ -293,8 +293,8 @@ def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int, *, inter
     holds, None for a model that was not packed.  Such a model's callers get
     PartialSums only where linear_into_norm splits, so its products into a
     norm stream only there (unless they stay `internal` to the layer); and with gradients asked of x or w the library
-    keeps the product (streaming has no backward; a packed model is inference
-    only)."""
+    keeps the product (streaming has no backward; a packed model's batches of
+    up to STREAM_MAX_ROWS rows are inference only)."""
     if torch.compiler.is_compiling():  # the shape rule is a C call, which a compiler's trace cannot hold
         return None
     if x.dim() != 2 or not 0 < x.shape[0] <= IN_PLACE_MAX_ROWS:  # first: a prefill step's layers ask three times each
@@ -303,11 +303,10 @@ def stream_operand(x: torch.Tensor, w: torch.Tensor, packed, mode: int, *, inter
         return None
     m, k = x.shape
     n = w.shape[0]
-    if packed is None:
-        if mode == GEMM_PARTS and not internal and split_factor(m, n, k) == 1:
-            return None
-        if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
-            return None
+    if packed is None and mode == GEMM_PARTS and not internal and split_factor(m, n, k) == 1:
+        return None
+    if (packed is None or m > STREAM_MAX_ROWS) and torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return None
     if _streams_in_place(w) and in_place_parts(m, n, k, mode) > 0:
         return w
     return packed if isinstance(packed, PackedWeight) and stream_rows(x) else None
