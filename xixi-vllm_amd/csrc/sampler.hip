@@ -2363,9 +2363,14 @@ __global__ __launch_bounds__(kThreads) void row_count_kernel(SegArgs a) {
 
 // Workspace: one 128-byte line per row (a 64-bit slot and a 32-bit arrival
 // counter) for the multi-workgroup greedy path, then the segments' counts of
-// the multi-workgroup sampled path, or room for kMaxCand candidates per row,
-// which the top-k path's lists use (it sets how many rows that path takes).
+// the multi-workgroup sampled path, or kTopRowBytes per row, which the top-k
+// path's lists use.
 namespace {
+// Sets how many rows the top-k path takes: the lists of all of them (R
+// kTopList 8-byte entries each) share the region of kSegMaxBatch rows.  At V
+// 151936 that is 4101 rows; past it one workgroup takes a row (3450 rows 376
+// us with lists, 1150 without; 4101 rows 449 and 1381).
+constexpr size_t kTopRowBytes = 77936;
 struct SegLayout {
   int R, seg_len;
   size_t best, cnt, total;
@@ -2382,7 +2387,7 @@ SegLayout seg_layout(int batch, int vocab) {
   size_t o = 0;  // offsets within the sampled path's region
   L.best = o;  o = align256(o + BR * 8);
   L.cnt = o;   o = align256(o + BR * kSegWords * 4);
-  L.total = max(o, align256(B * kMaxCand * 8));  // at least the top-k path's lists
+  L.total = max(o, align256(B * kTopRowBytes));
   return L;
 }
 
