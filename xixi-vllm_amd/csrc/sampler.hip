@@ -173,7 +173,6 @@ struct Shared {
   uint32_t red_u[kWaves];
   float red_f[kWaves];
   int64_t red_l[kWaves];
-  int64_t red_l2[kWaves];
   uint32_t cnt[256];
   unsigned long long mass[256];
   // broadcast slots
@@ -182,8 +181,6 @@ struct Shared {
   int64_t b_id;
   int64_t b_total;
   int b_hb;
-  int b_int[8];
-  int64_t b_long[8];
 };
 
 // LDS of the fast path: per-wave bucket histograms, then the candidate list
@@ -837,31 +834,13 @@ XV_INLINE bool fast_boundary(Shared& s, FastShared& fs, const bf16_t* row, int V
   key_cut = 1u;
   id_cut = kTieAll;
   M = total;
-  if (!(use_k || use_p || use_m)) return true;
+  if (!(use_p || use_m)) return true;
 
   // ---- bucket of each cut-off ----
-  int bk = kBuckets;
-  int64_t ck_before = 0, mk_before = 0;
-  if (use_k) {
-    int64_t c = 0, m = 0;
-    for (int bkt = 0; bkt < kBuckets; ++bkt) {
-      if (c + s.cnt[bkt] >= (uint32_t)top_k) { bk = bkt; ck_before = c; mk_before = m; break; }
-      c += s.cnt[bkt];
-      m += (int64_t)s.mass[bkt];
-    }
-  }
-  int64_t total_k = total;
-  int nk = 0;
-  if (bk < kBuckets) {
-    if (s.cnt[bk] > (uint32_t)kMaxCand) return false;  // known before gathering
-    nk = gather_bucket(fs, row, V, vec_ok, inv_t, zmax, bs, bk);
-    if (nk > kMaxCand) return false;
-    total_k = mk_before + list_mass_prefix(s, fs, nk, top_k - ck_before, inv_t, zmax);
-  }
   int bp = kBuckets;
   int64_t thr = 0, mp_before = 0;
   if (use_p) {
-    thr = (int64_t)floor((double)top_p * (double)total_k);
+    thr = (int64_t)floor((double)top_p * (double)total);
     int64_t m = 0;
     for (int bkt = 0; bkt < kBuckets; ++bkt) {
       if (m + (int64_t)s.mass[bkt] > thr) { bp = bkt; mp_before = m; break; }
@@ -870,17 +849,13 @@ XV_INLINE bool fast_boundary(Shared& s, FastShared& fs, const bf16_t* row, int V
   }
   int bm = kBuckets;
   if (use_m && kminp != 0xffffffffu) bm = bucket_of(log2_ratio(key_to_bits(kminp), inv_t, zmax), bs);
-  const int bf = min(bk, min(bp, bm));
+  const int bf = min(bp, bm);
   if (bf >= kBuckets) return true;  // no cut-off limits the row: everything kept
-  int n = nk;
-  if (bf != bk) {
-    if (s.cnt[bf] > (uint32_t)kMaxCand) return false;
-    n = gather_bucket(fs, row, V, vec_ok, inv_t, zmax, bs, bf);
-    if (n > kMaxCand) return false;
-  }
+  if (s.cnt[bf] > (uint32_t)kMaxCand) return false;
+  const int n = gather_bucket(fs, row, V, vec_ok, inv_t, zmax, bs, bf);
+  if (n > kMaxCand) return false;
   // ---- exact cut inside the boundary bucket ----
   int64_t jcut = kTieAll;
-  if (bk == bf) jcut = min(jcut, (int64_t)top_k - ck_before - 1);
   if (bp == bf) jcut = min(jcut, list_first_exceed(s, fs, n, mp_before, thr, inv_t, zmax));
   if (bm == bf) jcut = min(jcut, list_count_ge(s, fs, n, kminp) - 1);
   if (jcut >= n) jcut = n - 1;
