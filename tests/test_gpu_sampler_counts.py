@@ -69,3 +69,116 @@ def test_count_path_matches_the_oracle(dev, kind, v):
         want = S.sample(bits, temps.numpy(), tps.numpy(), tks.numpy(), mps.numpy(), u.numpy(), flags)
         got = sample(*g, use_top_k=bool(flags & 2), use_top_p=bool(flags & 4), use_min_p=bool(flags & 8))
         assert np.array_equal(got.cpu().numpy(), want), (flags, got.cpu().numpy(), want)
+
+
+def near_zero(kind, b, v, rng):
+    """Rows whose largest logits, and so their cuts, lie at zero."""
+    x = rng.standard_normal((b, v)).astype(np.float32) * 2
+    x -= x.max(1, keepdims=True)  # "shifted": each row's maximum is 0
+    if kind == "log_probs":  # of a row with one likely id
+        x[:, v // 3] = 25.0
+        x -= np.log(np.exp(x.astype(np.float64)).sum(1, keepdims=True)).astype(np.float32)
+    elif kind == "zeros":
+        x[rng.random((b, v)) < 0.7] = 0
+        x[rng.random((b, v)) < 0.2] *= -1
+    elif kind == "all_zero":
+        x[:] = np.where(rng.random((b, v)) < 0.5, np.float32(0), np.float32(-0.0))
+    elif kind in ("listed", "listed_flat"):  # values of both signs listed beside the counts, repeated ones, zeros between
+        x = np.minimum(x, -0.5 if kind == "listed" else -8.0)
+        for row in x:
+            ids = rng.permutation(v)[: min(v, 80)]
+            row[ids[:56]] = rng.choice(rng.choice([-1, 1], 30) * 2.0 ** -rng.uniform(22.1, 120, 30), ids[:56].size)
+            row[ids[56:68]] = 0
+            row[ids[68:]] = -0.0
+    elif kind == "listed_hot":  # their masses differ: read at a temperature of 1e-5 or so
+        x = np.minimum(x, -0.5)
+        x[:, rng.permutation(v)[:40]] = rng.uniform(-2e-7, 2e-7, (b, min(v, 40)))
+    elif kind == "too_many":  # more listed values than one row's list takes
+        x = np.minimum(x, -0.5)
+        x[:, ::7] = rng.uniform(-2e-7, 2e-7, x[:, ::7].shape)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["shifted", "log_probs", "zeros", "all_zero", "listed", "listed_flat", "listed_hot",
+                                  "too_many"])
+@pytest.mark.parametrize("v", [33, 2048, 16391, 65537])
+def test_cuts_at_zero_match_the_oracle(dev, kind, v):
+    import oracle.sampler as S
+    from xvllm.sampler import sample
+
+    rng = np.random.default_rng(v + len(kind))
+    b = 24
+    logits = torch.from_numpy(near_zero(kind, b, v, rng).astype(np.float32)).to(torch.bfloat16)
+    temps = torch.full((b,), 1.2e-5 if kind == "listed_hot" else 0.9)
+    u = torch.from_numpy(rng.random(b).astype(np.float32))
+    tps = torch.from_numpy(rng.uniform(0.02, 1.0, b).astype(np.float32))
+    tks = torch.from_numpy(rng.integers(1, min(v, 100), b).astype(np.int32))  # ranks among the listed values and zeros
+    tks[::3] = torch.from_numpy(rng.integers(1, v, tks[::3].numel()).astype(np.int32))
+    mps = torch.from_numpy((10.0 ** rng.uniform(-6, -0.1, b)).astype(np.float32))
+    mps[::4] = 1.0
+    bits = logits.view(torch.int16).numpy().view(np.uint16)
+    g = [t.to(dev) for t in (logits, temps, tps, tks, mps, u)]
+    for flags in (0, 2, 4, 8, 2 | 4, 2 | 4 | 8):
+        want = S.sample(bits, temps.numpy(), tps.numpy(), tks.numpy(), mps.numpy(), u.numpy(), flags)
+        got = sample(*g, use_top_k=bool(flags & 2), use_top_p=bool(flags & 4), use_min_p=bool(flags & 8))
+        assert np.array_equal(got.cpu().numpy(), want), (flags, got.cpu().numpy(), want)
+
+
+def call_us(logits, **kw):
+    """Time of a sampled call inside a graph of 20, the fastest of 7."""
+    from xvllm.sampler import reserve_workspace, sample
+
+    b, v = logits.shape
+    reserve_workspace(logits.device, b, v)
+    temps, u = torch.ones(b, device=logits.device), torch.full((b,), 0.37, device=logits.device)
+    sample(logits, temps, uniforms=u, **kw)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(20):
+            sample(logits, temps, uniforms=u, **kw)
+    best = 1e30
+    for _ in range(7):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        graph.replay()
+        e[1].record()
+        e[1].synchronize()
+        best = min(best, e[0].elapsed_time(e[1]) * 50)
+    return best
+
+
+def usual_and(dev, make, b=32, v=151936):
+    """Logits N(0, 2) and make(them), on the device."""
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn((b, v), generator=g, device=dev) * 2
+    return x.to(torch.bfloat16), make(x.clone()).to(torch.bfloat16)
+
+
+def no_slower(dev, make, modes, most):
+    """Calls on make(usual logits) take at most `most` times those on usual
+    ones: the counts settle the rows.  A row left to the one-workgroup path
+    takes four times as long and more."""
+    usual, rows = usual_and(dev, make)
+    b = usual.shape[0]
+    args = {"plain": {}, "top_p": dict(top_ps=torch.full((b,), 0.95, device=dev), use_top_p=True),
+            "top_k": dict(top_ks=torch.full((b,), 50, dtype=torch.int32, device=dev), use_top_k=True),
+            "min_p": dict(min_ps=torch.full((b,), 0.05, device=dev), use_min_p=True)}
+    for mode in modes:
+        a, c = call_us(usual, **args[mode]), call_us(rows, **args[mode])
+        assert c <= most * a, f"{mode}: {c:.1f} us, usual rows {a:.1f}"
+
+
+@pytest.mark.parametrize("kind", ["shifted", "log_probs", "max_zero", "all_zero"])
+def test_rows_near_zero_are_settled_by_the_counts(dev, kind):
+    def make(x):
+        if kind == "log_probs":
+            x[:, 7] = 30.0
+            return torch.log_softmax(x, -1)
+        if kind == "max_zero":
+            x = -x.abs()
+            x[:, 7] = 0
+            return x
+        return torch.zeros_like(x) if kind == "all_zero" else x - x.amax(1, keepdim=True)
+
+    no_slower(dev, make, ["plain", "top_p", "top_k", "min_p"], 2.5 if kind == "all_zero" else 1.5)

@@ -1840,9 +1840,12 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(SegArgs a) {
 // rank whose inclusive mass exceeds floor(top_p * mass), the rank of the
 // lowest key that reaches min_p; the smallest of them cuts.  Between the
 // positive and the negative window lie the zeros and the listed magnitudes
-// below 2^-22 (`mid`), after the window the values of -2^10 and below
-// (`far`).  Rows the counts don't settle (a value of 2^10 or above, a maximum
-// or a cut in mid, far values with mass, no value at all) run sample_row.
+// below 2^-22 (`mid`: the maximum of a row shifted to 0, or of
+// log-probabilities, lies there), after the window the values of -2^10 and
+// below (`far`).  A cut in mid is found in the sorted list, the zeros of each
+// sign counting as one key.  Rows the counts don't settle (a value of 2^10 or
+// above, more listed magnitudes than the lists hold, far values with mass, no
+// value at all) run sample_row.
 //
 // One workgroup works alone on its CU, so the time is latency and issue, not
 // bandwidth: wave w takes positions 256 w .. of each half, four per lane, so
@@ -1859,12 +1862,14 @@ constexpr int kCntLoads = 8;        // segments whose counts load together
 static_assert(kHalfPos == 4 * kThreads, "four positions per thread and half");
 
 struct RowCut {
-  int pos;       // the cut key's position; 2 * kMagBins: none (every window key kept)
+  int pos;       // the cut key's position, window positions before it being kept whole; 2 * kMagBins: every one is
   int ties;      // ids of the cut key kept
   int64_t M;     // kept mass
   int n;         // rank of the cut (2^31 - 1: none)
-  int fail;      // the cut falls in mid
+  int mid;       // the cut lies in mid: pos is kMagBins, n and M the rank and the mass before mid (until `resolve` adds
+                 // mid's), the cut mid's rank `ties`, or with ties 0 its first rank whose inclusive mass exceeds `left`
 };
+constexpr int kListMax = 64;  // mid's listed values of a row whose cut lies in mid: one per lane
 struct RowShared {
   RowCut cut[3];  // the top-k set's end, top-p's cut, the row's cut
   int ccnt[32];        // totals of the chunks (half, wave)
@@ -1872,6 +1877,9 @@ struct RowShared {
   int nm[kWaves];
   unsigned long long segm[kMaxSegs];  // kept masses of the window keys before the cut's
   int64_t midq[kMaxSegs];
+  uint32_t list[kListMax];  // mid's listed values: order key << 16 | segment
+  int mties[kMaxSegs];      // listed ids of the cut key
+  int64_t left;
   int t0;        // the draw: the thread whose ids hold the draw point, its mass and ties before
   int tie;
   int64_t cum;
@@ -1926,7 +1934,10 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   const uint32_t* head = cnts + (int64_t)min(lane, a.R - 1) * kSegWords + kMagBins;
   const uint4 h0 = *reinterpret_cast<const uint4*>(head), h1 = *reinterpret_cast<const uint4*>(head + 4);
   if (t < 3) s.cut[t] = RowCut{2 * kMagBins, 0, 0, 0x7fffffff, 0};
-  if (t < kMaxSegs) s.segm[t] = 0ull;
+  if (t < kMaxSegs) {
+    s.segm[t] = 0ull;
+    s.mties[t] = 0;
+  }
   uint32_t c[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
   each_group([&](int r0, const uint2 (&kc)[kCntLoads][2]) {
 #pragma unroll
@@ -1943,8 +1954,24 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   const uint32_t zeros = seg_lane ? h0.x + h0.y : 0u, ntiny = seg_lane ? h1.y : 0u;
   const bool has_mid = __ballot(zeros | ntiny) != 0, has_far = __ballot(seg_lane && h0.z) != 0;
   const float inv_t = 1.0f / p.temp;
-  const float zmax = bf16_to_f32(pos_bits(min(first, 2 * kMagBins - 1))) * inv_t;
-  bool settled = first < 2 * kMagBins && !(first >= kMagBins && has_mid) && __builtin_isfinite(zmax) &&
+  // f(segment, its listed value on this lane, 0xffff past its list)
+  auto each_tiny = [&](auto&& f) {
+    for (unsigned long long m = __ballot(ntiny != 0); m; m &= m - 1) {
+      const int r = __builtin_ctzll(m);
+      const int n = min((int)__shfl((int)ntiny, r), kTinyList);
+      const uint16_t* list = reinterpret_cast<const uint16_t*>(cnts + (int64_t)r * kSegWords + kMagBins + kHWords);
+      f(r, lane < n ? (uint32_t)list[lane] : 0xffffu);
+    }
+  };
+  uint32_t kmax = first < 2 * kMagBins ? order_key(pos_bits(first)) : 0u;
+  if (first >= kMagBins && has_mid) {  // the largest value lies in mid
+    kmax = __ballot(seg_lane && h0.x) ? 0x8000u : __ballot(seg_lane && h0.y) ? 0x7fffu : 0u;
+    each_tiny([&](int, uint32_t bits) { kmax = max(kmax, order_key(bits)); });
+    kmax = wave_max_u(kmax);
+  }
+  kmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)kmax);
+  const float zmax = bf16_to_f32(key_to_bits(kmax)) * inv_t;
+  bool settled = kmax != 0u && __builtin_isfinite(zmax) &&
                  !__ballot(seg_lane && (h1.x != 0u || ntiny > (uint32_t)kTinyList));
   int far = 0;
   if (has_far) {
@@ -1955,25 +1982,24 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   }
   // mid: counts and masses, lane r its segment's
   int64_t mid_q = 0;
-  int mid_c = 0;
+  int mid_c = 0, nlist = 0;
   bool mid_in = false;  // mid reaches min_p (all of it, or the row isn't settled)
   if (settled && has_mid) {
     const float ez = exp_of(0u, inv_t, zmax);
     int64_t mid_qr = (int64_t)zeros * mass_of(ez);
     bool any_in = zeros && ez >= p.min_p, any_out = zeros && !(ez >= p.min_p);
-    for (unsigned long long m = __ballot(ntiny != 0); m; m &= m - 1) {
-      const int r = __builtin_ctzll(m);
-      const int n = (int)__shfl((int)ntiny, r);
-      float e = 0.0f;
-      if (lane < n) {
-        const uint16_t* list = reinterpret_cast<const uint16_t*>(cnts + (int64_t)r * kSegWords + kMagBins + kHWords);
-        e = exp_of(list[lane], inv_t, zmax);
+    each_tiny([&](int r, uint32_t bits) {
+      const uint32_t key = order_key(bits);
+      const float e = exp_of(bits, inv_t, zmax);  // (padding: 0)
+      if (key) {
         any_in |= e >= p.min_p;
         any_out |= !(e >= p.min_p);
+        if (t < 64 && nlist + lane < kListMax) s.list[nlist + lane] = key << 16 | (uint32_t)r;
       }
+      nlist += __popcll(__ballot(key != 0u));
       const int64_t q = wave_sum_l(mass_of(e));
       mid_qr += lane == r ? q : 0;
-    }
+    });
     if (p.use_m) {
       mid_in = __ballot(any_in) != 0;
       settled = !(mid_in && __ballot(any_out) != 0);
@@ -1982,7 +2008,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     mid_q = wave_sum_l(mid_qr);
     if (t < a.R) s.midq[t] = mid_qr;
   }
-  if (!settled) return false;
+  if (!__builtin_amdgcn_readfirstlane((int)settled)) return false;
 
   // masses; per half, the rank and mass prefixes over its positions
   int cex[2], cn[2], nm[2];  // exclusive rank prefixes, counts, ranks reaching min_p
@@ -2071,7 +2097,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
       int left = n - cex[h] - (h ? pre_c : 0);
       int64_t m = mex[h] + (h ? pre_q : 0);
       if (left <= 0) {
-        cut.fail = 1;
+        cut = RowCut{kMagBins, n - cex[h], mex[h], cex[h], 1};
         continue;
       }
       int pos = 2 * kMagBins, ties = 0;
@@ -2087,11 +2113,45 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
           left -= (int)c[h][j];
         }
       }
-      cut.pos = pos;  // a rank in far (left > 0 still): every window key kept, far has no mass
-      cut.ties = ties;
-      cut.M = m;
-      cut.n = n;
+      // a rank in far (left > 0 still): every window key kept, far has no mass
+      cut = RowCut{pos, ties, m, n, 0};
     }
+  };
+  // A cut in mid: its key, by each wave for itself from the sorted list, the
+  // +0s and the -0s between the listed positive and negative values.  False
+  // if the list does not hold mid.
+  uint32_t mid_key = 0u;  // the last resolved cut's key, where that lies in mid
+  auto resolve = [&](RowCut& cut) -> bool {
+    if (!__builtin_amdgcn_readfirstlane(cut.mid)) return true;
+    if (nlist > kListMax) return false;
+    const uint32_t key = wave_sort_desc32(lane < nlist ? s.list[lane] : 0u) >> 16;
+    const uint4 hz = *reinterpret_cast<const uint4*>(head);
+    const int npz = (int)wave_sum_l(seg_lane ? hz.x : 0u), nz = npz + (int)wave_sum_l(seg_lane ? hz.y : 0u);
+    const int np = __popcll(__ballot(key > 0x8000u));
+    const int64_t qz = mass_of(exp_of(0u, inv_t, zmax));
+    const int64_t incl = wave_incl_scan_l(key ? mass_of(exp_of(key_to_bits(key), inv_t, zmax)) : 0);
+    const int64_t above = np ? __shfl(incl, np - 1) : 0;  // mass of the listed positive values
+    int rank = cut.ties;
+    if (rank == 0) {
+      const int64_t left = s.left;
+      rank = (int)wave_first(lane < np && incl > left, -1) + 1;
+      if (rank == 0 && left < above + nz * qz) rank = np + 1 + (int)((left - above) / qz);
+      if (rank == 0) rank = nz + 1 + (int)wave_first(lane >= np && incl + nz * qz > left, nlist - 1);
+    }
+    cut.n += rank;
+    if (rank > np && rank <= np + nz) {
+      const int i = rank - np;
+      mid_key = i <= npz ? 0x8000u : 0x7fffu;
+      cut.ties = i <= npz ? i : i - npz;
+      cut.M += above + i * qz;
+    } else {
+      const int j = rank <= np ? rank - 1 : rank - 1 - nz;
+      mid_key = __shfl(key, j);
+      cut.ties = __popcll(__ballot(lane <= j && key == mid_key));
+      cut.M += __shfl(incl, j) + (rank <= np ? 0 : nz * qz);
+    }
+    mid_key = (uint32_t)__builtin_amdgcn_readfirstlane((int)mid_key);
+    return true;
   };
   int n = ctot;
   if (p.use_k && p.top_k < n) n = p.top_k;
@@ -2099,8 +2159,9 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   if (p.use_p && n < ctot) {
     locate(n, s.cut[0]);
     __syncthreads();
-    base = s.cut[0].M;
-    if (s.cut[0].fail) return false;
+    RowCut cut = s.cut[0];
+    if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return false;
+    base = cut.M;
   }
   if (p.use_p) {
     // the first rank whose inclusive mass exceeds thr (a negative thr: the first rank)
@@ -2115,7 +2176,8 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
         int k = cex[h];
         if (h) {
           if (left < pre_q) {
-            s.cut[1].fail = 1;
+            s.cut[1] = RowCut{kMagBins, 0, m, k, 1};
+            s.left = left;
             continue;
           }
           left -= pre_q;
@@ -2155,29 +2217,37 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   }
   __syncthreads();
   RowCut cut = s.cut[1];  // no top-p: none
-  if (cut.fail) return false;
+  if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return false;
   n = min(n, cut.n);
   if (p.use_m) {
     n_m = (int)wave_max_u(lane < kWaves ? (uint32_t)s.nm[lane] : 0u);
     if (n_m > 0) n = min(n, n_m);
   }
   if (n >= ctot) {
-    cut.pos = 2 * kMagBins;
-    cut.ties = 0;
-    cut.M = mtot;
+    cut = RowCut{2 * kMagBins, 0, mtot, n, 0};
   } else if (n != cut.n) {
     locate(n, s.cut[2]);
     __syncthreads();
     cut = s.cut[2];
-    if (cut.fail) return false;
+    if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return false;
   }
   const int pos = __builtin_amdgcn_readfirstlane(cut.pos), cut_ties = __builtin_amdgcn_readfirstlane(cut.ties);
+  const bool in_mid = __builtin_amdgcn_readfirstlane(cut.mid) != 0;
+  // keys above the cut's are kept whole
+  const uint32_t cut_key = in_mid ? mid_key : pos < 2 * kMagBins ? order_key(pos_bits(pos)) : 0u;
   const int64_t cut_m = cut.M;
+  const uint32_t cut_bits = cut_key ? key_to_bits(cut_key) : 0x10000u;  // no cut key: equals no logit
+  const int64_t q_cut = mass_of(exp_of(cut_bits & 0xffffu, inv_t, zmax));
 
   // each segment's kept mass: its positions before the cut's, then (lane r)
   // mid and its share of the cut key's ids, the lowest ids first
   uint32_t tie_word = 0;
-  if (pos < 2 * kMagBins && seg_lane) tie_word = cnts[(int64_t)lane * kSegWords + (pos >> 1)];
+  if (!in_mid && pos < 2 * kMagBins && seg_lane) tie_word = cnts[(int64_t)lane * kSegWords + (pos >> 1)];
+  if (in_mid && t < nlist) {  // (nlist <= 64)
+    const uint32_t x = s.list[t], key = x >> 16;
+    if (key > cut_key) atomicAdd(&s.segm[x & 0xffffu], (unsigned long long)mass_of(exp_of(key_to_bits(key), inv_t, zmax)));
+    if (key == cut_key) atomicAdd(&s.mties[x & 0xffffu], 1);
+  }
   bool some = false;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -2223,13 +2293,20 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     });
   }
   __syncthreads();
-  const uint32_t cut_bits = pos < 2 * kMagBins ? pos_bits(pos) : 0x10000u;  // no cut key: equals no logit
-  const int64_t q_cut = mass_of(exp_of(cut_bits & 0xffffu, inv_t, zmax));
-  const int tie_cr = (int)((tie_word >> (16 * (pos & 1))) & 0xffffu);
+  int tie_cr = (int)((tie_word >> (16 * (pos & 1))) & 0xffffu);
+  int64_t sm = seg_lane ? (int64_t)s.segm[lane] : 0;
+  if (in_mid) {
+    if (seg_lane) {
+      const uint4 hz = *reinterpret_cast<const uint4*>(head);
+      tie_cr = s.mties[lane] + (int)(cut_key == 0x8000u ? hz.x : cut_key == 0x7fffu ? hz.y : 0u);
+      sm += (int64_t)((cut_key < 0x8000u ? hz.x : 0u) + (cut_key < 0x7fffu ? hz.y : 0u)) * mass_of(exp_of(0u, inv_t, zmax));
+    }
+  } else if (seg_lane && has_mid && pos >= kMagBins) {
+    sm += s.midq[lane];
+  }
   const int tie_ex = wave_incl_scan_i(tie_cr) - tie_cr;
   const int ties_r = max(0, min(tie_cr, cut_ties - tie_ex));
-  int64_t sm = seg_lane ? (int64_t)s.segm[lane] : 0;
-  if (seg_lane) sm += ties_r * q_cut + (has_mid && pos >= kMagBins ? s.midq[lane] : 0);
+  if (seg_lane) sm += ties_r * q_cut;
 
   // the draw: the segment holding floor(u * M), then in id order the first
   // kept id whose inclusive mass exceeds the rest.  Each thread sums a run of
@@ -2244,11 +2321,11 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   const int C = ((end - beg + kThreads - 1) / kThreads + 7) / 8 * 8;
   const int i0 = min(end, beg + t * C), i1 = min(end, i0 + C);
   // mass of an id before the cut key (0 for others)
-  const bool mid_kept = has_mid && pos >= kMagBins;
+  const bool mid_kept = has_mid && pos >= kMagBins;  // (of a cut in mid, the keys above it)
   auto id_mass = [&](uint32_t bits) -> double {
     const uint32_t mag = bits & 0x7fffu, m = mag - kMagLo;
     if (m < (uint32_t)kMagBins) return qtab[(bits >> 15) * kMagBins + m];
-    return mid_kept && mag < kMagLo ? mass_d(exp_of(bits, inv_t, zmax)) : 0.0;
+    return mid_kept && mag < kMagLo && order_key(bits) > cut_key ? mass_d(exp_of(bits, inv_t, zmax)) : 0.0;
   };
   double mine_d = 0.0;
   int mties = 0;
@@ -2327,7 +2404,7 @@ __global__ __launch_bounds__(kThreads) void row_count_kernel(SegArgs a) {
     }
     return;
   }
-  if (!row_from_counts(a, p, rs, reinterpret_cast<double*>(fs.cand), b)) {
+  if (!__builtin_amdgcn_readfirstlane((int)row_from_counts(a, p, rs, reinterpret_cast<double*>(fs.cand), b))) {
     int rb = b;
     __asm__ volatile("" : "+s"(rb)::"memory");
     sample_row(s, fs, rb, a.logits, a.stride, a.V, a.temps, a.top_ps, a.top_ks, a.min_ps, a.uniforms,
