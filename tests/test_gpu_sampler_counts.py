@@ -93,6 +93,13 @@ def near_zero(kind, b, v, rng):
     elif kind == "listed_hot":  # their masses differ: read at a temperature of 1e-5 or so
         x = np.minimum(x, -0.5)
         x[:, rng.permutation(v)[:40]] = rng.uniform(-2e-7, 2e-7, (b, min(v, 40)))
+    elif kind == "one_mass":  # more small values than any list takes, a maximum that makes them equal
+        x[:, ::2] *= 1e-8
+        x[:, v // 2] = 9.0
+    elif kind == "nearly_one_mass":  # a maximum at which the small values' distances just differ
+        x[:, ::2] = rng.uniform(-2.3e-7, 2.3e-7, x[:, ::2].shape)
+        x[:, 1::2] = np.minimum(x[:, 1::2], -1)
+        x[:, v // 2] = rng.choice([1.0, 2.0, 3.99, 4.0, 5.0, 7.99], b)
     elif kind == "too_many":  # more listed values than one row's list takes
         x = np.minimum(x, -0.5)
         x[:, ::7] = rng.uniform(-2e-7, 2e-7, x[:, ::7].shape)
@@ -100,7 +107,7 @@ def near_zero(kind, b, v, rng):
 
 
 @pytest.mark.parametrize("kind", ["shifted", "log_probs", "zeros", "all_zero", "listed", "listed_flat", "listed_hot",
-                                  "too_many"])
+                                  "one_mass", "nearly_one_mass", "too_many"])
 @pytest.mark.parametrize("v", [33, 2048, 16391, 65537])
 def test_cuts_at_zero_match_the_oracle(dev, kind, v):
     import oracle.sampler as S
@@ -182,3 +189,14 @@ def test_rows_near_zero_are_settled_by_the_counts(dev, kind):
         return torch.zeros_like(x) if kind == "all_zero" else x - x.amax(1, keepdim=True)
 
     no_slower(dev, make, ["plain", "top_p", "top_k", "min_p"], 2.5 if kind == "all_zero" else 1.5)
+
+
+@pytest.mark.parametrize("modes", ["plain", "top_k", "min_p"])
+def test_many_small_values_are_settled_by_the_counts(dev, modes):
+    """Half of a row's ids below 2^-22, of one mass beside a maximum of 8 and
+    more (calls whose cut lies among them excepted)."""
+    def make(x):
+        x[:, ::2] *= 1e-8
+        return x
+
+    no_slower(dev, make, [modes], 1.9)

@@ -1971,8 +1971,14 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   }
   kmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)kmax);
   const float zmax = bf16_to_f32(key_to_bits(kmax)) * inv_t;
-  bool settled = kmax != 0u && __builtin_isfinite(zmax) &&
-                 !__ballot(seg_lane && (h1.x != 0u || ntiny > (uint32_t)kTinyList));
+  // All of mid has one mass where its two ends lie at the same distance from
+  // the maximum: 2^-22 past a maximum of 8 is below its last place.  The lists
+  // are not read then and need not be whole (half of a row's ids in (0, 2^-22),
+  // 32 rows, top-k 50: 140 us with the row left to the one-workgroup path, 28 now).
+  const bool one_mass = log2_ratio(kMagLo - 1u, inv_t, zmax) == log2_ratio(0x8000u | (kMagLo - 1u), inv_t, zmax);
+  const bool whole = !__ballot(ntiny > (uint32_t)kTinyList);  // the lists hold every small value
+  bool settled = kmax != 0u && __builtin_isfinite(zmax) && !__ballot(seg_lane && h1.x != 0u) &&
+                 (whole || (one_mass && first < kMagBins));
   int far = 0;
   if (has_far) {
     far = (int)wave_sum_l(seg_lane ? h0.z : 0u);
@@ -1982,24 +1988,21 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   }
   // mid: counts and masses, lane r its segment's
   int64_t mid_q = 0;
-  int mid_c = 0, nlist = 0;
+  int mid_c = 0;
   bool mid_in = false;  // mid reaches min_p (all of it, or the row isn't settled)
   if (settled && has_mid) {
     const float ez = exp_of(0u, inv_t, zmax);
-    int64_t mid_qr = (int64_t)zeros * mass_of(ez);
-    bool any_in = zeros && ez >= p.min_p, any_out = zeros && !(ez >= p.min_p);
-    each_tiny([&](int r, uint32_t bits) {
-      const uint32_t key = order_key(bits);
-      const float e = exp_of(bits, inv_t, zmax);  // (padding: 0)
-      if (key) {
-        any_in |= e >= p.min_p;
-        any_out |= !(e >= p.min_p);
-        if (t < 64 && nlist + lane < kListMax) s.list[nlist + lane] = key << 16 | (uint32_t)r;
-      }
-      nlist += __popcll(__ballot(key != 0u));
-      const int64_t q = wave_sum_l(mass_of(e));
-      mid_qr += lane == r ? q : 0;
-    });
+    const uint32_t equal = one_mass ? zeros + ntiny : zeros;
+    int64_t mid_qr = (int64_t)equal * mass_of(ez);
+    bool any_in = equal && ez >= p.min_p, any_out = equal && !(ez >= p.min_p);
+    if (!one_mass)
+      each_tiny([&](int r, uint32_t bits) {
+        const float e = exp_of(bits, inv_t, zmax);  // (padding: 0)
+        any_in |= bits != 0xffffu && e >= p.min_p;
+        any_out |= bits != 0xffffu && !(e >= p.min_p);
+        const int64_t q = wave_sum_l(mass_of(e));
+        mid_qr += lane == r ? q : 0;
+      });
     if (p.use_m) {
       mid_in = __ballot(any_in) != 0;
       settled = !(mid_in && __ballot(any_out) != 0);
@@ -2117,13 +2120,21 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
       cut = RowCut{pos, ties, m, n, 0};
     }
   };
-  // A cut in mid: its key, by each wave for itself from the sorted list, the
-  // +0s and the -0s between the listed positive and negative values.  False
-  // if the list does not hold mid.
+  // A cut in mid: its key, by each wave for itself (every wave writes the same
+  // list) from the sorted list, the +0s and the -0s between the listed positive
+  // and negative values.  False if the lists do not hold mid.
   uint32_t mid_key = 0u;  // the last resolved cut's key, where that lies in mid
+  int nlist = 0;
   auto resolve = [&](RowCut& cut) -> bool {
     if (!__builtin_amdgcn_readfirstlane(cut.mid)) return true;
+    if (!whole) return false;
+    nlist = 0;
+    each_tiny([&](int r, uint32_t bits) {
+      if (bits != 0xffffu && nlist + lane < kListMax) s.list[nlist + lane] = order_key(bits) << 16 | (uint32_t)r;
+      nlist += __popcll(__ballot(bits != 0xffffu));
+    });
     if (nlist > kListMax) return false;
+    __builtin_amdgcn_wave_barrier();
     const uint32_t key = wave_sort_desc32(lane < nlist ? s.list[lane] : 0u) >> 16;
     const uint4 hz = *reinterpret_cast<const uint4*>(head);
     const int npz = (int)wave_sum_l(seg_lane ? hz.x : 0u), nz = npz + (int)wave_sum_l(seg_lane ? hz.y : 0u);
@@ -2322,10 +2333,12 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   const int i0 = min(end, beg + t * C), i1 = min(end, i0 + C);
   // mass of an id before the cut key (0 for others)
   const bool mid_kept = has_mid && pos >= kMagBins;  // (of a cut in mid, the keys above it)
+  const double q_zero = mid_kept ? mass_d(exp_of(0u, inv_t, zmax)) : 0.0;
   auto id_mass = [&](uint32_t bits) -> double {
     const uint32_t mag = bits & 0x7fffu, m = mag - kMagLo;
     if (m < (uint32_t)kMagBins) return qtab[(bits >> 15) * kMagBins + m];
-    return mid_kept && mag < kMagLo && order_key(bits) > cut_key ? mass_d(exp_of(bits, inv_t, zmax)) : 0.0;
+    if (!(mid_kept && mag < kMagLo && order_key(bits) > cut_key)) return 0.0;
+    return mag == 0u || one_mass ? q_zero : mass_d(exp_of(bits, inv_t, zmax));
   };
   double mine_d = 0.0;
   int mties = 0;
