@@ -200,3 +200,63 @@ def test_many_small_values_are_settled_by_the_counts(dev, modes):
         return x
 
     no_slower(dev, make, [modes], 1.9)
+
+
+def large(kind, b, v, rng):
+    """Rows with logits of 2^10 and above."""
+    x = rng.standard_normal((b, v)).astype(np.float32) * 2
+    few = min(v, 30)
+    ids = np.stack([rng.permutation(v)[:few] for _ in range(b)])
+    if kind == "one":
+        x[:, v // 3] = 1500
+    elif kind == "some":  # a few within reach of each other, repeated values
+        np.put_along_axis(x, ids, (rng.integers(150, 154, (b, few)) * 8).astype(np.float32), 1)
+    elif kind == "around":  # the cut on either side of 2^10, and in mid or far with them
+        x = x * 5 + 1010
+        np.put_along_axis(x, ids, rng.choice([0.0, -0.0, 1e-8, -1e5], (b, few)).astype(np.float32), 1)
+        x[:, few + 5:] = np.minimum(x[:, few + 5:], 1020)  # few of them at or past it
+    elif kind == "spread":  # a third of the row
+        x *= 600
+    elif kind == "level":  # more of them with mass than a list holds
+        x += 2000
+    elif kind == "top_far":  # everything past the counted magnitudes
+        x = np.where(x > 4, np.float32(3000), np.float32(-3000)) + x
+    elif kind == "huge":  # scaled past 2^20
+        x = np.exp2(x * 10 + 25)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["one", "some", "around", "spread", "level", "top_far", "huge"])
+@pytest.mark.parametrize("v", [33, 2048, 16391, 65537])
+@pytest.mark.parametrize("t", [0.9, 20.0])
+def test_large_logits_match_the_oracle(dev, kind, v, t):
+    import oracle.sampler as S
+    from xvllm.sampler import sample
+
+    rng = np.random.default_rng(v + len(kind))
+    b = 24
+    logits = torch.from_numpy(large(kind, b, v, rng).astype(np.float32)).to(torch.bfloat16)
+    temps = torch.full((b,), t)
+    u = torch.from_numpy(rng.random(b).astype(np.float32))
+    tps = torch.from_numpy(rng.uniform(0.02, 1.0, b).astype(np.float32))
+    tks = torch.from_numpy(rng.integers(1, min(v, 40), b).astype(np.int32))
+    mps = torch.from_numpy((10.0 ** rng.uniform(-14, -0.1, b)).astype(np.float32))
+    mps[::4] = 1.0
+    bits = logits.view(torch.int16).numpy().view(np.uint16)
+    g = [x.to(dev) for x in (logits, temps, tps, tks, mps, u)]
+    for flags in (0, 2, 4, 8, 2 | 4, 2 | 4 | 8):
+        want = S.sample(bits, temps.numpy(), tps.numpy(), tks.numpy(), mps.numpy(), u.numpy(), flags)
+        got = sample(*g, use_top_k=bool(flags & 2), use_top_p=bool(flags & 4), use_min_p=bool(flags & 8))
+        assert np.array_equal(got.cpu().numpy(), want), (flags, got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("kind", ["one", "spread"])
+def test_rows_with_large_logits_are_settled_by_the_counts(dev, kind):
+    def make(x):
+        if kind == "spread":
+            return x * 600
+        x[:, 7] = 1500
+        return x
+
+    # two more passes over such a segment and its list: 1.6 to 1.75 times a usual row where a third of the ids are large
+    no_slower(dev, make, ["plain", "top_p", "top_k", "min_p"], 2.5 if kind == "spread" else 1.5)

@@ -39,6 +39,10 @@
 #pragma clang fp contract(off)
 
 
+// Rare cases out of the way of the code most rows run through.
+#define XV_LIKELY(c) __builtin_expect(!!(c), 1)
+#define XV_UNLIKELY(c) __builtin_expect(!!(c), 0)
+
 namespace {
 
 constexpr int kThreads = 1024;
@@ -1289,15 +1293,23 @@ XV_INLINE void for_seg(const bf16_t* row, bool vec_ok, int beg, int end, F&& f) 
 // the 2 * kMagBins window keys in descending order (position pos < kMagBins:
 // the positive magnitude kMagLo + kMagBins - 1 - pos, past it the negative one
 // kMagLo + pos - kMagBins; two to a word), then the header, then up to
-// kTinyList 16-bit logits of magnitudes in (0, 2^-22).
+// kTinyList 16-bit logits of magnitudes in (0, 2^-22) and as many of 2^10 and
+// above: those that can have mass beside the segment's largest.
 constexpr int kMagBins = 4096;                  // 32 octaves of 128 bf16 magnitudes
 constexpr uint32_t kMagLo = (127 - 22) << 7;    // 2^-22; the window ends at 2^10
 constexpr uint32_t kInfMag = 0x7f80u;
 constexpr int kTinyList = 64;
 constexpr int kMaxSegIds = 65528;               // a count fits 16 bits
-// header words; kHFarMag and kHFirst hold 0xffff - value (a cleared word is "none")
-enum : int { kHPosZero = 0, kHNegZero, kHFar, kHFarMag, kHTop, kHTiny, kHFirst, kHWords = 8 };
-constexpr int kSegWords = (kMagBins + kHWords + kTinyList / 2 + 63) / 64 * 64;
+// header words; kHFarMag and kHFirst hold 0xffff - value (a cleared word is
+// "none"), kHTopMax the largest value of 2^10 and above (raw bits), kHTop the
+// count of those listed
+enum : int { kHPosZero = 0, kHNegZero, kHFar, kHFarMag, kHTop, kHTiny, kHFirst, kHTopMax, kHWords = 8 };
+constexpr int kTopsAt = kMagBins + kHWords + kTinyList / 2;  // the list of values of 2^10 and above
+constexpr int kSegWords = (kTopsAt + kTinyList / 2 + 63) / 64 * 64;
+// A value this many temperatures below another has no mass beside it (2^40
+// 2^d is below 1 at 27.8; the rest is rounding of d: where l / T is large
+// enough for more, so is the step between bf16 values).
+constexpr float kMasslessT = 28.5f;
 // Window position of raw bits with m = magnitude - kMagLo < kMagBins, and back.
 XV_INLINE uint32_t window_pos(uint32_t bits, uint32_t m) {
   return (bits & 0x8000u) ? (uint32_t)kMagBins + m : (uint32_t)(kMagBins - 1) - m;
@@ -1353,7 +1365,7 @@ __global__ __launch_bounds__(kThreads) void seg_count_kernel(SegArgs a) {
           ++far;
           far_mag = min(far_mag, mag);
         } else {
-          head[kHTop] = 1u;
+          head[kHTopMax] = 1u;  // found below
         }
       } else if (mag == 0u) {
         if (bits) ++nz; else ++pz;
@@ -1390,6 +1402,26 @@ __global__ __launch_bounds__(kThreads) void seg_count_kernel(SegArgs a) {
                                       : v.w ? 8 * t + (v.w & 0xffffu ? 6 : 7) : 0xffffu;
   const uint32_t first = wave_min_u(at);
   if (lane == 0) wbest[t >> 6] = 0xffffu - first;
+  if (XV_UNLIKELY(head[kHTopMax])) {  // (uniform) the largest value of 2^10 and above, then those that can have mass beside it
+    auto each_top = [&](auto&& f) {
+      for_seg(row, vec_ok, beg, end, [&](uint32_t bits, int) {
+        if (bits >= kMagLo + (uint32_t)kMagBins && bits <= kInfMag) f(bits);
+      });
+    };
+    uint32_t top = 0;
+    each_top([&](uint32_t bits) { top = max(top, bits); });
+    top = wave_max_u(top);
+    __syncthreads();  // every thread has read the flag
+    if (lane == 0) atomicMax(&head[kHTopMax], top);
+    __syncthreads();
+    const float least = bf16_to_f32(head[kHTopMax]) - kMasslessT * a.temps[b];
+    uint16_t* tops = reinterpret_cast<uint16_t*>(h + kTopsAt);
+    each_top([&](uint32_t bits) {
+      if (!(bf16_to_f32(bits) >= least)) return;
+      const uint32_t i = atomicAdd(&head[kHTop], 1u);
+      if (i < (uint32_t)kTinyList) tops[i] = (uint16_t)bits;
+    });
+  }
   __syncthreads();
   if (t < kSegWords / 4 - kThreads) {
     uint4 x = h4[kThreads + t];
@@ -1841,11 +1873,13 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(SegArgs a) {
 // lowest key that reaches min_p; the smallest of them cuts.  Between the
 // positive and the negative window lie the zeros and the listed magnitudes
 // below 2^-22 (`mid`: the maximum of a row shifted to 0, or of
-// log-probabilities, lies there), after the window the values of -2^10 and
-// below (`far`).  A cut in mid is found in the sorted list, the zeros of each
-// sign counting as one key.  Rows the counts don't settle (a value of 2^10 or
-// above, more listed magnitudes than the lists hold, far values with mass, no
-// value at all) run sample_row.
+// log-probabilities, lies there), before the positive window the listed
+// values of 2^10 and above (`top`; those not listed have no mass, and nor has
+// any value below them, so ranks without them give the same masses), after the
+// negative one the values of -2^10 and below (`far`).  A cut in top or mid is
+// found in the sorted list, the zeros of each sign counting as one key.  Rows
+// the counts don't settle (more listed values than the lists hold, far values
+// with mass, no value at all) run sample_row.
 //
 // One workgroup works alone on its CU, so the time is latency and issue, not
 // bandwidth: wave w takes positions 256 w .. of each half, four per lane, so
@@ -1866,10 +1900,12 @@ struct RowCut {
   int ties;      // ids of the cut key kept
   int64_t M;     // kept mass
   int n;         // rank of the cut (2^31 - 1: none)
-  int mid;       // the cut lies in mid: pos is kMagBins, n and M the rank and the mass before mid (until `resolve` adds
-                 // mid's), the cut mid's rank `ties`, or with ties 0 its first rank whose inclusive mass exceeds `left`
+  int in;        // the cut lies in a group, kInTop or kInMid: pos is the group's (0, kMagBins), n and M the rank and the
+                 // mass before it (until `resolve` adds the group's), the cut the group's rank `ties`, or with ties 0
+                 // its first rank whose inclusive mass exceeds `left`
 };
-constexpr int kListMax = 64;  // mid's listed values of a row whose cut lies in mid: one per lane
+enum : int { kInTop = 1, kInMid = 2 };
+constexpr int kListMax = 64;  // listed values of the group a row's cut lies in: one per lane
 struct RowShared {
   RowCut cut[3];  // the top-k set's end, top-p's cut, the row's cut
   int ccnt[32];        // totals of the chunks (half, wave)
@@ -1877,8 +1913,9 @@ struct RowShared {
   int nm[kWaves];
   unsigned long long segm[kMaxSegs];  // kept masses of the window keys before the cut's
   int64_t midq[kMaxSegs];
-  uint32_t list[kListMax];  // mid's listed values: order key << 16 | segment
-  int mties[kMaxSegs];      // listed ids of the cut key
+  int64_t topq[kMaxSegs];
+  uint32_t list[kListMax];  // the group's listed values: order key << 16 | segment
+  int lties[kMaxSegs];      // listed ids of the cut key
   int64_t left;
   int t0;        // the draw: the thread whose ids hold the draw point, its mass and ties before
   int tie;
@@ -1936,7 +1973,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   if (t < 3) s.cut[t] = RowCut{2 * kMagBins, 0, 0, 0x7fffffff, 0};
   if (t < kMaxSegs) {
     s.segm[t] = 0ull;
-    s.mties[t] = 0;
+    s.lties[t] = 0;
   }
   uint32_t c[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
   each_group([&](int r0, const uint2 (&kc)[kCntLoads][2]) {
@@ -1954,17 +1991,22 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   const uint32_t zeros = seg_lane ? h0.x + h0.y : 0u, ntiny = seg_lane ? h1.y : 0u;
   const bool has_mid = __ballot(zeros | ntiny) != 0, has_far = __ballot(seg_lane && h0.z) != 0;
   const float inv_t = 1.0f / p.temp;
-  // f(segment, its listed value on this lane, 0xffff past its list)
-  auto each_tiny = [&](auto&& f) {
-    for (unsigned long long m = __ballot(ntiny != 0); m; m &= m - 1) {
+  // f(segment, its listed value on this lane, 0xffff past its list) for the
+  // lists at word `at` of the segments, `count` (lane r: segment r's) long
+  auto each_listed = [&](uint32_t count, int at, auto&& f) {
+    for (unsigned long long m = __ballot(count != 0); m; m &= m - 1) {
       const int r = __builtin_ctzll(m);
-      const int n = min((int)__shfl((int)ntiny, r), kTinyList);
-      const uint16_t* list = reinterpret_cast<const uint16_t*>(cnts + (int64_t)r * kSegWords + kMagBins + kHWords);
+      const int n = min((int)__shfl((int)count, r), kTinyList);
+      const uint16_t* list = reinterpret_cast<const uint16_t*>(cnts + (int64_t)r * kSegWords + at);
       f(r, lane < n ? (uint32_t)list[lane] : 0xffffu);
     }
   };
+  auto each_tiny = [&](auto&& f) { each_listed(ntiny, kMagBins + kHWords, f); };
+  const bool has_top = __ballot(seg_lane && h1.w) != 0;
   uint32_t kmax = first < 2 * kMagBins ? order_key(pos_bits(first)) : 0u;
-  if (first >= kMagBins && has_mid) {  // the largest value lies in mid
+  if (XV_UNLIKELY(has_top)) {
+    kmax = order_key(wave_max_u(seg_lane ? h1.w : 0u));
+  } else if (XV_UNLIKELY(first >= kMagBins && has_mid)) {  // the largest value lies in mid
     kmax = __ballot(seg_lane && h0.x) ? 0x8000u : __ballot(seg_lane && h0.y) ? 0x7fffu : 0u;
     each_tiny([&](int, uint32_t bits) { kmax = max(kmax, order_key(bits)); });
     kmax = wave_max_u(kmax);
@@ -1977,10 +2019,10 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   // 32 rows, top-k 50: 140 us with the row left to the one-workgroup path, 28 now).
   const bool one_mass = log2_ratio(kMagLo - 1u, inv_t, zmax) == log2_ratio(0x8000u | (kMagLo - 1u), inv_t, zmax);
   const bool whole = !__ballot(ntiny > (uint32_t)kTinyList);  // the lists hold every small value
-  bool settled = kmax != 0u && __builtin_isfinite(zmax) && !__ballot(seg_lane && h1.x != 0u) &&
-                 (whole || (one_mass && first < kMagBins));
+  bool settled = kmax != 0u && __builtin_isfinite(zmax) && !__ballot(seg_lane && h1.x > (uint32_t)kTinyList) &&
+                 (whole || (one_mass && (has_top || first < kMagBins)));
   int far = 0;
-  if (has_far) {
+  if (XV_UNLIKELY(has_far)) {
     far = (int)wave_sum_l(seg_lane ? h0.z : 0u);
     const uint32_t far_mag = 0xffffu - wave_max_u(seg_lane ? h0.w : 0u);
     const float e = exp_of(0x8000u | far_mag, inv_t, zmax);  // the largest: the others' masses are no larger
@@ -1990,7 +2032,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   int64_t mid_q = 0;
   int mid_c = 0;
   bool mid_in = false;  // mid reaches min_p (all of it, or the row isn't settled)
-  if (settled && has_mid) {
+  if (XV_UNLIKELY(settled && has_mid)) {
     const float ez = exp_of(0u, inv_t, zmax);
     const uint32_t equal = one_mass ? zeros + ntiny : zeros;
     int64_t mid_qr = (int64_t)equal * mass_of(ez);
@@ -2012,18 +2054,44 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     if (t < a.R) s.midq[t] = mid_qr;
   }
   if (!__builtin_amdgcn_readfirstlane((int)settled)) return false;
+  // top: the listed values that have mass, their count and mass, and the rank of the last to reach min_p
+  int top_c = 0, top_m = 0;
+  int64_t top_q = 0;
+  uint32_t top_low = 0xffffu;  // the lowest key with mass
+  if (XV_UNLIKELY(has_top)) {
+    const uint32_t ntop = seg_lane ? h1.x : 0u;
+    int64_t top_qr = 0;
+    uint32_t kmin = 0xffffu;  // the lowest key that reaches min_p
+    each_listed(ntop, kTopsAt, [&](int r, uint32_t bits) {
+      const float e = exp_of(bits, inv_t, zmax);  // (padding: 0)
+      const int64_t m = mass_of(e);
+      if (m) top_low = min(top_low, order_key(bits));
+      if (m && e >= p.min_p) kmin = min(kmin, order_key(bits));
+      top_c += __popcll(__ballot(m != 0));
+      const int64_t q = wave_sum_l(m);
+      top_qr += lane == r ? q : 0;
+    });
+    kmin = wave_min_u(kmin);
+    each_listed(ntop, kTopsAt, [&](int, uint32_t bits) {
+      top_m += __popcll(__ballot(mass_of(exp_of(bits, inv_t, zmax)) != 0 && order_key(bits) >= kmin));
+    });
+    top_q = wave_sum_l(top_qr);
+    if (t < a.R) s.topq[t] = top_qr;
+    top_low = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_min_u(top_low));
+  }
 
   // masses; per half, the rank and mass prefixes over its positions
   int cex[2], cn[2], nm[2];  // exclusive rank prefixes, counts, ranks reaching min_p
   int64_t mex[2], ms[2];
-  const int pre_c = t == 0 ? mid_c : 0;  // mid: before half 1's first position
-  const int64_t pre_q = t == 0 ? mid_q : 0;
+  // top and mid: before half 0's and half 1's first position
+  const int pre_c[2] = {t == 0 ? top_c : 0, t == 0 ? mid_c : 0};
+  const int64_t pre_q[2] = {t == 0 ? top_q : 0, t == 0 ? mid_q : 0};
   // position pos's entry of the table
   auto tab_of = [](int pos) { return pos < kHalfPos ? kHalfPos - 1 - pos : pos; };
   {
     // one position per step of a rolled loop (the counts rotate through c[0][0])
-    int n_h = 0, nm_h = 0;
-    int64_t m_h = 0;
+    int n_h = pre_c[0], nm_h = t == 0 ? top_m : 0;
+    int64_t m_h = pre_q[0];
 #pragma unroll 1
     for (int i = 0; i < 8; ++i) {
       const uint32_t ci = c[0][0];
@@ -2042,7 +2110,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
       qtab[tab_of(pos)] = qd;
       if (i == 3) {
         cn[0] = n_h, ms[0] = m_h, nm[0] = nm_h;
-        n_h = pre_c, m_h = pre_q, nm_h = mid_in ? pre_c : 0;
+        n_h = pre_c[1], m_h = pre_q[1], nm_h = mid_in ? pre_c[1] : 0;
       }
     }
     cn[1] = n_h + (t == kThreads - 1 ? far : 0), ms[1] = m_h, nm[1] = nm_h;
@@ -2097,10 +2165,10 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       if (!(cex[h] < n && n <= cex[h] + cn[h])) continue;
-      int left = n - cex[h] - (h ? pre_c : 0);
-      int64_t m = mex[h] + (h ? pre_q : 0);
+      int left = n - cex[h] - pre_c[h];
+      int64_t m = mex[h] + pre_q[h];
       if (left <= 0) {
-        cut = RowCut{kMagBins, n - cex[h], mex[h], cex[h], 1};
+        cut = RowCut{h * kMagBins, n - cex[h], mex[h], cex[h], h ? kInMid : kInTop};
         continue;
       }
       int pos = 2 * kMagBins, ties = 0;
@@ -2120,24 +2188,30 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
       cut = RowCut{pos, ties, m, n, 0};
     }
   };
-  // A cut in mid: its key, by each wave for itself (every wave writes the same
-  // list) from the sorted list, the +0s and the -0s between the listed positive
-  // and negative values.  False if the lists do not hold mid.
-  uint32_t mid_key = 0u;  // the last resolved cut's key, where that lies in mid
+  // A cut in a group: its key, by each wave for itself (every wave writes the
+  // same list) from the sorted list, in mid the +0s and the -0s between the
+  // positive and the negative values.  False if the lists do not hold the group.
+  uint32_t in_key = 0u;  // the last resolved cut's key, where that lies in a group
   int nlist = 0;
   auto resolve = [&](RowCut& cut) -> bool {
-    if (!__builtin_amdgcn_readfirstlane(cut.mid)) return true;
-    if (!whole) return false;
+    const int in = __builtin_amdgcn_readfirstlane(cut.in);
+    if (XV_LIKELY(!in)) return true;
+    if (in == kInMid && !whole) return false;
+    const uint4 hz = *reinterpret_cast<const uint4*>(head);
     nlist = 0;
-    each_tiny([&](int r, uint32_t bits) {
-      if (bits != 0xffffu && nlist + lane < kListMax) s.list[nlist + lane] = order_key(bits) << 16 | (uint32_t)r;
-      nlist += __popcll(__ballot(bits != 0xffffu));
-    });
+    each_listed(in == kInMid ? ntiny : seg_lane ? head[kHTop] : 0u, in == kInMid ? kMagBins + kHWords : kTopsAt,
+                [&](int r, uint32_t bits) {
+                  const bool on = bits != 0xffffu && (in == kInMid || mass_of(exp_of(bits, inv_t, zmax)) != 0);
+                  const unsigned long long all = __ballot(on);
+                  const int i = nlist + __popcll(all & ((1ull << lane) - 1));
+                  if (on && i < kListMax) s.list[i] = order_key(bits) << 16 | (uint32_t)r;
+                  nlist += __popcll(all);
+                });
     if (nlist > kListMax) return false;
     __builtin_amdgcn_wave_barrier();
     const uint32_t key = wave_sort_desc32(lane < nlist ? s.list[lane] : 0u) >> 16;
-    const uint4 hz = *reinterpret_cast<const uint4*>(head);
-    const int npz = (int)wave_sum_l(seg_lane ? hz.x : 0u), nz = npz + (int)wave_sum_l(seg_lane ? hz.y : 0u);
+    const int npz = in == kInMid ? (int)wave_sum_l(seg_lane ? hz.x : 0u) : 0;
+    const int nz = in == kInMid ? npz + (int)wave_sum_l(seg_lane ? hz.y : 0u) : 0;
     const int np = __popcll(__ballot(key > 0x8000u));
     const int64_t qz = mass_of(exp_of(0u, inv_t, zmax));
     const int64_t incl = wave_incl_scan_l(key ? mass_of(exp_of(key_to_bits(key), inv_t, zmax)) : 0);
@@ -2152,16 +2226,16 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     cut.n += rank;
     if (rank > np && rank <= np + nz) {
       const int i = rank - np;
-      mid_key = i <= npz ? 0x8000u : 0x7fffu;
+      in_key = i <= npz ? 0x8000u : 0x7fffu;
       cut.ties = i <= npz ? i : i - npz;
       cut.M += above + i * qz;
     } else {
       const int j = rank <= np ? rank - 1 : rank - 1 - nz;
-      mid_key = __shfl(key, j);
-      cut.ties = __popcll(__ballot(lane <= j && key == mid_key));
+      in_key = __shfl(key, j);
+      cut.ties = __popcll(__ballot(lane <= j && key == in_key));
       cut.M += __shfl(incl, j) + (rank <= np ? 0 : nz * qz);
     }
-    mid_key = (uint32_t)__builtin_amdgcn_readfirstlane((int)mid_key);
+    in_key = (uint32_t)__builtin_amdgcn_readfirstlane((int)in_key);
     return true;
   };
   int n = ctot;
@@ -2185,16 +2259,14 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
         if (!(mex[h] <= thr && thr < mex[h] + ms[h])) continue;
         int64_t left = thr - mex[h], m = mex[h];
         int k = cex[h];
-        if (h) {
-          if (left < pre_q) {
-            s.cut[1] = RowCut{kMagBins, 0, m, k, 1};
-            s.left = left;
-            continue;
-          }
-          left -= pre_q;
-          k += pre_c;
-          m += pre_q;
+        if (left < pre_q[h]) {
+          s.cut[1] = RowCut{h * kMagBins, 0, m, k, h ? kInMid : kInTop};
+          s.left = left;
+          continue;
         }
+        left -= pre_q[h];
+        k += pre_c[h];
+        m += pre_q[h];
         int64_t qk = 1;
         int pos = -1;
 #pragma unroll
@@ -2243,9 +2315,9 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return false;
   }
   const int pos = __builtin_amdgcn_readfirstlane(cut.pos), cut_ties = __builtin_amdgcn_readfirstlane(cut.ties);
-  const bool in_mid = __builtin_amdgcn_readfirstlane(cut.mid) != 0;
+  const int in = __builtin_amdgcn_readfirstlane(cut.in);
   // keys above the cut's are kept whole
-  const uint32_t cut_key = in_mid ? mid_key : pos < 2 * kMagBins ? order_key(pos_bits(pos)) : 0u;
+  const uint32_t cut_key = in ? in_key : pos < 2 * kMagBins ? order_key(pos_bits(pos)) : 0u;
   const int64_t cut_m = cut.M;
   const uint32_t cut_bits = cut_key ? key_to_bits(cut_key) : 0x10000u;  // no cut key: equals no logit
   const int64_t q_cut = mass_of(exp_of(cut_bits & 0xffffu, inv_t, zmax));
@@ -2253,11 +2325,11 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   // each segment's kept mass: its positions before the cut's, then (lane r)
   // mid and its share of the cut key's ids, the lowest ids first
   uint32_t tie_word = 0;
-  if (!in_mid && pos < 2 * kMagBins && seg_lane) tie_word = cnts[(int64_t)lane * kSegWords + (pos >> 1)];
-  if (in_mid && t < nlist) {  // (nlist <= 64)
+  if (!in && pos < 2 * kMagBins && seg_lane) tie_word = cnts[(int64_t)lane * kSegWords + (pos >> 1)];
+  if (XV_UNLIKELY(in && t < nlist)) {  // (nlist <= 64)
     const uint32_t x = s.list[t], key = x >> 16;
     if (key > cut_key) atomicAdd(&s.segm[x & 0xffffu], (unsigned long long)mass_of(exp_of(key_to_bits(key), inv_t, zmax)));
-    if (key == cut_key) atomicAdd(&s.mties[x & 0xffffu], 1);
+    if (key == cut_key) atomicAdd(&s.lties[x & 0xffffu], 1);
   }
   bool some = false;
 #pragma unroll
@@ -2306,14 +2378,16 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   __syncthreads();
   int tie_cr = (int)((tie_word >> (16 * (pos & 1))) & 0xffffu);
   int64_t sm = seg_lane ? (int64_t)s.segm[lane] : 0;
-  if (in_mid) {
-    if (seg_lane) {
+  if (seg_lane) {
+    if (in) tie_cr = s.lties[lane];
+    if (XV_UNLIKELY(in == kInMid)) {
       const uint4 hz = *reinterpret_cast<const uint4*>(head);
-      tie_cr = s.mties[lane] + (int)(cut_key == 0x8000u ? hz.x : cut_key == 0x7fffu ? hz.y : 0u);
+      tie_cr += (int)(cut_key == 0x8000u ? hz.x : cut_key == 0x7fffu ? hz.y : 0u);
       sm += (int64_t)((cut_key < 0x8000u ? hz.x : 0u) + (cut_key < 0x7fffu ? hz.y : 0u)) * mass_of(exp_of(0u, inv_t, zmax));
+    } else if (has_mid && pos >= kMagBins) {
+      sm += s.midq[lane];
     }
-  } else if (seg_lane && has_mid && pos >= kMagBins) {
-    sm += s.midq[lane];
+    if (has_top && in != kInTop) sm += s.topq[lane];
   }
   const int tie_ex = wave_incl_scan_i(tie_cr) - tie_cr;
   const int ties_r = max(0, min(tie_cr, cut_ties - tie_ex));
@@ -2333,12 +2407,16 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   const int i0 = min(end, beg + t * C), i1 = min(end, i0 + C);
   // mass of an id before the cut key (0 for others)
   const bool mid_kept = has_mid && pos >= kMagBins;  // (of a cut in mid, the keys above it)
+  const bool others = mid_kept || has_top;
   const double q_zero = mid_kept ? mass_d(exp_of(0u, inv_t, zmax)) : 0.0;
   auto id_mass = [&](uint32_t bits) -> double {
     const uint32_t mag = bits & 0x7fffu, m = mag - kMagLo;
     if (m < (uint32_t)kMagBins) return qtab[(bits >> 15) * kMagBins + m];
-    if (!(mid_kept && mag < kMagLo && order_key(bits) > cut_key)) return 0.0;
-    return mag == 0u || one_mass ? q_zero : mass_d(exp_of(bits, inv_t, zmax));
+    if (!others) return 0.0;
+    const uint32_t key = order_key(bits);
+    const bool small = mag < kMagLo;
+    if (!(small ? mid_kept : key >= top_low) || key <= cut_key) return 0.0;  // (far, NaN: none)
+    return small && (mag == 0u || one_mass) ? q_zero : mass_d(exp_of(bits, inv_t, zmax));
   };
   double mine_d = 0.0;
   int mties = 0;
