@@ -260,3 +260,48 @@ def test_rows_with_large_logits_are_settled_by_the_counts(dev, kind):
 
     # two more passes over such a segment and its list: 1.6 to 1.75 times a usual row where a third of the ids are large
     no_slower(dev, make, ["plain", "top_p", "top_k", "min_p"], 2.5 if kind == "spread" else 1.5)
+
+
+@pytest.mark.parametrize("v", [33, 2048, 65537])
+def test_rows_without_mass_match_the_oracle(dev, v):
+    """A scaled maximum that is not finite leaves no mass anywhere: +inf once
+    and twice, beside NaN and -inf; -inf alone; finite values past fp32's range
+    once scaled, of either sign; and rows that only look so."""
+    import oracle.sampler as S
+    from xvllm.sampler import sample
+
+    rng = np.random.default_rng(v)
+    x = rng.standard_normal((12, v)).astype(np.float32) * 2
+    x[0, v // 2] = np.inf
+    x[1, [v // 3, v - 1]] = np.inf
+    x[2, :5] = [np.nan, -np.inf, np.inf, np.nan, 3e38]
+    x[3] = -np.inf
+    x[4] = np.where(rng.random(v) < 0.5, np.nan, -np.inf)
+    x[5, 7] = 3e38
+    x[6] = -3e38
+    x[7] = np.where(rng.random(v) < 0.5, np.float32(-2e38), -np.inf)
+    x[8] = np.nan
+    x[9] = -1e5  # finite once scaled: every id alike
+    x[10] = np.where(rng.random(v) < 0.9, -np.inf, np.float32(-2000))
+    x[11, ::2] = -np.inf
+    temps = torch.full((12,), 0.45)
+    u = torch.from_numpy(rng.random(12).astype(np.float32))
+    tps, mps = torch.full((12,), 0.7), torch.full((12,), 0.1)
+    tks = torch.full((12,), 9, dtype=torch.int32)
+    logits = torch.from_numpy(x).to(torch.bfloat16)
+    bits = logits.view(torch.int16).numpy().view(np.uint16)
+    g = [y.to(dev) for y in (logits, temps, tps, tks, mps, u)]
+    for flags in (0, 2, 4, 8, 2 | 4 | 8):
+        want = S.sample(bits, temps.numpy(), tps.numpy(), tks.numpy(), mps.numpy(), u.numpy(), flags)
+        got = sample(*g, use_top_k=bool(flags & 2), use_top_p=bool(flags & 4), use_min_p=bool(flags & 8))
+        assert np.array_equal(got.cpu().numpy(), want), (flags, got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf")])
+def test_rows_without_mass_take_one_scan(dev, value):
+    """The largest key is known from the counts: one more pass over the row, not two."""
+    def make(x):
+        x[:, 9 if value > 0 else slice(None)] = value
+        return x
+
+    no_slower(dev, make, ["plain", "top_p", "top_k", "min_p"], 1.6)

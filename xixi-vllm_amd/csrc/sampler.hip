@@ -1943,10 +1943,12 @@ XV_INLINE int64_t wave_sum8(int64_t (&v)[8]) {
 XV_INLINE double mass_d(float e) { return __builtin_trunc((double)e * 1099511627776.0); }
 constexpr uint32_t kExactIds = 4095;  // ids per thread and half whose mass sum (of both halves) is exact in fp64
 
-// Sampled row b from its segments' counts; false (on every thread) if the
-// counts don't settle it.  qtab: masses of the 2 * kMagBins window keys by
-// magnitude (kMagBins + magnitude for negative ones).
-XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& s, double* qtab, int b) {
+// Sampled row b from its segments' counts.  kRowLeft (on every thread) if the
+// counts don't settle it; the largest key if no id has mass, the row's answer
+// then being the lowest id that holds it.  qtab: masses of the 2 * kMagBins
+// window keys by magnitude (kMagBins + magnitude for negative ones).
+enum : uint32_t { kRowDone = 0, kRowLeft = 0x10000 };
+XV_INLINE uint32_t row_from_counts(const SegArgs& a, const RowParams& p, RowShared& s, double* qtab, int b) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const bf16_t* row = a.logits + (int64_t)b * a.stride;
   const bool vec_ok = ((reinterpret_cast<uintptr_t>(row) & 15u) == 0);
@@ -2011,20 +2013,23 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     each_tiny([&](int, uint32_t bits) { kmax = max(kmax, order_key(bits)); });
     kmax = wave_max_u(kmax);
   }
+  const uint32_t far_mag = XV_UNLIKELY(has_far) ? 0xffffu - wave_max_u(seg_lane ? h0.w : 0u) : 0u;  // its smallest
+  const bool only_far = has_far && !has_top && !has_mid && first >= 2 * kMagBins;
+  if (XV_UNLIKELY(only_far)) kmax = order_key(0x8000u | far_mag);
   kmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)kmax);
   const float zmax = bf16_to_f32(key_to_bits(kmax)) * inv_t;
+  if (XV_UNLIKELY(kmax != 0u && !__builtin_isfinite(zmax))) return kmax;
   // All of mid has one mass where its two ends lie at the same distance from
   // the maximum: 2^-22 past a maximum of 8 is below its last place.  The lists
   // are not read then and need not be whole (half of a row's ids in (0, 2^-22),
   // 32 rows, top-k 50: 140 us with the row left to the one-workgroup path, 28 now).
   const bool one_mass = log2_ratio(kMagLo - 1u, inv_t, zmax) == log2_ratio(0x8000u | (kMagLo - 1u), inv_t, zmax);
   const bool whole = !__ballot(ntiny > (uint32_t)kTinyList);  // the lists hold every small value
-  bool settled = kmax != 0u && __builtin_isfinite(zmax) && !__ballot(seg_lane && h1.x > (uint32_t)kTinyList) &&
+  bool settled = kmax != 0u && !only_far && !__ballot(seg_lane && h1.x > (uint32_t)kTinyList) &&
                  (whole || (one_mass && (has_top || first < kMagBins)));
   int far = 0;
   if (XV_UNLIKELY(has_far)) {
     far = (int)wave_sum_l(seg_lane ? h0.z : 0u);
-    const uint32_t far_mag = 0xffffu - wave_max_u(seg_lane ? h0.w : 0u);
     const float e = exp_of(0x8000u | far_mag, inv_t, zmax);  // the largest: the others' masses are no larger
     settled = settled && mass_of(e) == 0 && !(p.use_m && e >= p.min_p);
   }
@@ -2053,7 +2058,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     mid_q = wave_sum_l(mid_qr);
     if (t < a.R) s.midq[t] = mid_qr;
   }
-  if (!__builtin_amdgcn_readfirstlane((int)settled)) return false;
+  if (!__builtin_amdgcn_readfirstlane((int)settled)) return kRowLeft;
   // top: the listed values that have mass, their count and mass, and the rank of the last to reach min_p
   int top_c = 0, top_m = 0;
   int64_t top_q = 0;
@@ -2245,7 +2250,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     locate(n, s.cut[0]);
     __syncthreads();
     RowCut cut = s.cut[0];
-    if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return false;
+    if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return kRowLeft;
     base = cut.M;
   }
   if (p.use_p) {
@@ -2300,7 +2305,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
   }
   __syncthreads();
   RowCut cut = s.cut[1];  // no top-p: none
-  if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return false;
+  if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return kRowLeft;
   n = min(n, cut.n);
   if (p.use_m) {
     n_m = (int)wave_max_u(lane < kWaves ? (uint32_t)s.nm[lane] : 0u);
@@ -2312,7 +2317,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     locate(n, s.cut[2]);
     __syncthreads();
     cut = s.cut[2];
-    if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return false;
+    if (!__builtin_amdgcn_readfirstlane((int)resolve(cut))) return kRowLeft;
   }
   const int pos = __builtin_amdgcn_readfirstlane(cut.pos), cut_ties = __builtin_amdgcn_readfirstlane(cut.ties);
   const int in = __builtin_amdgcn_readfirstlane(cut.in);
@@ -2459,7 +2464,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     }
   }
   __syncthreads();
-  if (t >= 64) return true;
+  if (t >= 64) return kRowDone;
   const int t0 = s.t0;
   int64_t cum = s.cum;
   int te = s.tie;
@@ -2478,7 +2483,7 @@ XV_INLINE bool row_from_counts(const SegArgs& a, const RowParams& p, RowShared& 
     cum = __shfl(inc, 63);
     te += __popcll(__ballot(tie));
   }
-  return true;
+  return kRowDone;
 }
 
 __global__ __launch_bounds__(kThreads) void row_count_kernel(SegArgs a) {
@@ -2495,7 +2500,15 @@ __global__ __launch_bounds__(kThreads) void row_count_kernel(SegArgs a) {
     }
     return;
   }
-  if (!__builtin_amdgcn_readfirstlane((int)row_from_counts(a, p, rs, reinterpret_cast<double*>(fs.cand), b))) {
+  const uint32_t left =
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)row_from_counts(a, p, rs, reinterpret_cast<double*>(fs.cand), b));
+  if (left != kRowDone) {
+    if (left != kRowLeft) {
+      const bf16_t* row = a.logits + (int64_t)b * a.stride;
+      const int64_t id = lowest_id_of_key(s, row, a.V, (reinterpret_cast<uintptr_t>(row) & 15u) == 0, left);
+      if (t == 0) a.out_ids[b] = id;
+      return;
+    }
     int rb = b;
     __asm__ volatile("" : "+s"(rb)::"memory");
     sample_row(s, fs, rb, a.logits, a.stride, a.V, a.temps, a.top_ps, a.top_ks, a.min_ps, a.uniforms,
