@@ -1,11 +1,12 @@
 """The rule of the in-place streaming GEMM (xv_stream_gemm_parts) and its
 argument checks, on the CPU: every shape it takes cuts into whole tiles,
 stages and 192 (gate/up) or 224 to 256 workgroups, the calls around its edges are refused
-before anything is launched, and CPU or gradient inputs keep the library path."""
+before anything is launched, every kernel the rule picks exists, and CPU inputs and long batches keep the library path."""
 import random
 
 import pytest
 import torch
+from helpers import STREAM_CLASSES, stream_kernel, stream_kernel_shapes
 
 INVALID, A = 1, 1 << 20  # hipErrorInvalidValue; an aligned address no call reaches
 
@@ -103,3 +104,23 @@ def test_long_batches_do_not_ask_the_library(monkeypatch):
                     got = linear.stream_operand(x, w, packed, mode, internal=True)
                     assert (got is w) == (0 < m <= 256)
     assert {a[0] for a in asked} == {1, 256}
+
+
+def test_every_picked_kernel_exists(lib):
+    """Shapes of all sizes pick only kernels that stream_kernel_shapes names
+    (the GPU test runs each of those), and a call of each gets as far as its
+    launch: without a device that fails, and 0 would mean none was made."""
+    shapes = stream_kernel_shapes(lib)
+    rng = random.Random(11)
+    for _ in range(40000):
+        m, mode, k = rng.randint(1, 256), rng.choice([1, 2]), 64 * rng.randint(1, 400)
+        n = 16 * rng.choice([rng.randint(1, 3300), 16 * rng.randint(1, 200)])
+        kernel = stream_kernel(lib, m, n, k, mode)
+        assert kernel is None or kernel in shapes, (m, n, k, kernel)
+    assert {c for _, c, _ in shapes} == set(STREAM_CLASSES)
+    if torch.cuda.is_available():  # (the addresses are not real)
+        return
+    for (mode, m, _), (n, k) in shapes.items():
+        width = n if mode == 1 else n // 2
+        rc = lib.xv_stream_gemm(A, k, A, k, A, width, m * n, m, n, k, mode, lib.xv_stream_gemm_parts(m, n, k, mode), None)
+        assert rc not in (0, INVALID), (mode, m, n, k, rc)

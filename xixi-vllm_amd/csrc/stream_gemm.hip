@@ -268,6 +268,10 @@ __global__ __launch_bounds__(MW * KW * 64) void stream_gemm_kernel(StreamArgs a)
   }
 }
 
+// The most tiles per workgroup that a row class has a kernel for: with more its
+// ring is too shallow, or (10) its accumulators too many.
+constexpr int max_tiles(int m) { return m <= 16 ? 6 : m <= 64 ? 8 : 10; }
+
 // The tile count and K split of one product (bnt 0: not taken).
 struct StreamPlan {
   int bnt, parts;
@@ -307,7 +311,7 @@ StreamPlan stream_plan(int m, int n, int k, int mode) {
     if (c > cost) continue;  // ties: the larger split
     for (int bnt : {1, 2, 4, 5, 6, 8, 10}) {  // the most workgroups up to 256
       if (tiles % bnt || (int64_t)tiles / bnt * parts > 256) continue;
-      if ((int64_t)tiles / bnt * parts < 224 || (bnt == 10 && m <= 64) || (bnt == 8 && m <= 16)) break;
+      if ((int64_t)tiles / bnt * parts < 224 || bnt > max_tiles(m)) break;
       best = StreamPlan{bnt, parts};
       cost = c;
       break;
@@ -316,13 +320,18 @@ StreamPlan stream_plan(int m, int n, int k, int mode) {
   return best;
 }
 
+// False: no such kernel.
 template <int MW, int MTW, int KW, int BNT, int KS, int XT, int DEPTH>
-void launch(const StreamArgs& a, int mode, unsigned blocks, hipStream_t stream) {
+bool launch(const StreamArgs& a, int mode, unsigned blocks, hipStream_t stream) {
   if (mode == kModeParts) {
     stream_gemm_kernel<MW, MTW, KW, BNT, KS, XT, DEPTH, kModeParts><<<blocks, MW * KW * 64, 0, stream>>>(a);
-  } else if constexpr (BNT % 2 == 0) {
-    stream_gemm_kernel<MW, MTW, KW, BNT, KS, XT, DEPTH, kModeSiluMul><<<blocks, MW * KW * 64, 0, stream>>>(a);
+    return true;
   }
+  if constexpr (BNT % 2 == 0) {
+    stream_gemm_kernel<MW, MTW, KW, BNT, KS, XT, DEPTH, kModeSiluMul><<<blocks, MW * KW * 64, 0, stream>>>(a);
+    return true;
+  }
+  return false;
 }
 
 // Waves, stage and ring depth per row class: the waves split the stage's K
@@ -330,20 +339,21 @@ void launch(const StreamArgs& a, int mode, unsigned blocks, hipStream_t stream) 
 // MFMAs need the overlap: 200 rows 54 us, with half the waves 63), and the
 // ring takes what fits of 160 KB.
 template <int BNT>
-void launch_rows(const StreamArgs& a, int mode, unsigned blocks, hipStream_t stream) {
+bool launch_rows(const StreamArgs& a, int mode, unsigned blocks, hipStream_t stream) {
   if (a.m <= 16) {
-    if constexpr (BNT <= 6) launch<1, 1, 4, BNT, 128, 1, BNT == 1 ? 8 : BNT == 6 || BNT == 5 ? 5 : 6>(a, mode, blocks, stream);
+    if constexpr (BNT <= max_tiles(16)) return launch<1, 1, 4, BNT, 128, 1, BNT == 1 ? 8 : BNT == 6 || BNT == 5 ? 5 : 6>(a, mode, blocks, stream);
   } else if (a.m <= 32) {
-    if constexpr (BNT <= 8) launch<2, 1, 4, BNT, 128, 2, BNT == 1 ? 10 : BNT == 2 ? 8 : BNT == 4 ? 6 : BNT == 5 ? 5 : 4>(a, mode, blocks, stream);
+    if constexpr (BNT <= max_tiles(32)) return launch<2, 1, 4, BNT, 128, 2, BNT == 1 ? 10 : BNT == 2 ? 8 : BNT == 4 ? 6 : BNT == 5 ? 5 : 4>(a, mode, blocks, stream);
   } else if (a.m <= 64) {
-    if constexpr (BNT <= 8) launch<4, 1, 2, BNT, 128, 4, BNT <= 2 ? 6 : BNT == 4 ? 5 : BNT == 5 ? 4 : 3>(a, mode, blocks, stream);
+    if constexpr (BNT <= max_tiles(64)) return launch<4, 1, 2, BNT, 128, 4, BNT <= 2 ? 6 : BNT == 4 ? 5 : BNT == 5 ? 4 : 3>(a, mode, blocks, stream);
   } else if (a.m <= 128) {
-    launch<8, 1, 2, BNT, 64, 8, BNT <= 2 ? 7 : BNT <= 5 ? 6 : BNT == 6 ? 5 : 4>(a, mode, blocks, stream);
+    return launch<8, 1, 2, BNT, 64, 8, BNT <= 2 ? 7 : BNT <= 5 ? 6 : BNT == 6 ? 5 : 4>(a, mode, blocks, stream);
   } else if constexpr (BNT == 10) {
-    launch<8, 2, 1, BNT, 64, 16, 3>(a, mode, blocks, stream);  // 20 accumulators: two waves per SIMD
+    return launch<8, 2, 1, BNT, 64, 16, 3>(a, mode, blocks, stream);  // 20 accumulators: two waves per SIMD
   } else {
-    launch<8, 2, 2, BNT, 64, 16, BNT <= 4 ? 4 : 3>(a, mode, blocks, stream);
+    return launch<8, 2, 2, BNT, 64, 16, BNT <= 4 ? 4 : 3>(a, mode, blocks, stream);
   }
+  return false;
 }
 
 }  // namespace
@@ -366,15 +376,17 @@ extern "C" int xv_stream_gemm(const void* x, int64_t x_stride, const void* w, in
   const StreamArgs a{(const bf16_t*)x, x_stride, (const bf16_t*)w, w_stride, out, out_stride, part_stride,
                      m, k / parts, mode == kModeSiluMul ? n / 2 : 0, parts};
   const unsigned blocks = (unsigned)(n / (16 * p.bnt) * parts);
+  bool done = false;
   switch (p.bnt) {
-    case 1: launch_rows<1>(a, mode, blocks, stream); break;
-    case 2: launch_rows<2>(a, mode, blocks, stream); break;
-    case 4: launch_rows<4>(a, mode, blocks, stream); break;
-    case 5: launch_rows<5>(a, mode, blocks, stream); break;
-    case 6: launch_rows<6>(a, mode, blocks, stream); break;
-    case 8: launch_rows<8>(a, mode, blocks, stream); break;
-    default: launch_rows<10>(a, mode, blocks, stream); break;
+    case 1: done = launch_rows<1>(a, mode, blocks, stream); break;
+    case 2: done = launch_rows<2>(a, mode, blocks, stream); break;
+    case 4: done = launch_rows<4>(a, mode, blocks, stream); break;
+    case 5: done = launch_rows<5>(a, mode, blocks, stream); break;
+    case 6: done = launch_rows<6>(a, mode, blocks, stream); break;
+    case 8: done = launch_rows<8>(a, mode, blocks, stream); break;
+    default: done = launch_rows<10>(a, mode, blocks, stream); break;
   }
+  if (!done) return (int)hipErrorInvalidValue;
   XV_CHECK_LAUNCH();
   return 0;
 }
