@@ -1,16 +1,17 @@
 """The in-place streaming GEMM (xv_stream_gemm) against a float64 product of
 the same bf16 operands, at the edges of its row classes (16, 32, 64, 128, 256
-rows) and over every tile count its rule picks.  Partial sums: the fp32 sum
-of K products in any order is within K 2^-24 sum |x w| of the exact one.
-SiLU-and-mul: g and u are rounded to bf16 before it and the result after
-it, rtol/atol 2e-2 over the bf16-rounded products as the packed kernel's test."""
+rows): the decoder's shapes, then every kernel the rule picks (row class, tile
+count, form) over several turns of its ring.  Partial sums: the fp32 sum of K
+products in any order is within K 2^-24 sum |x w| of the exact one.
+SiLU-and-mul: at small K rtol/atol 2e-2 over the bf16-rounded products as the
+packed kernel's test, and over the rings' turns the bound its roundings give."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 ROWS = [1, 15, 16, 17, 32, 33, 64, 65, 128, 129, 200, 256]
-# (n, k): tiles per workgroup over the row classes 1, 2 / 1, 2 / 2, 4 / 2, 8 / 5, 10 / 6
+# (n, k): the tiles per workgroup are 1, 2 / 1, 2 / 1, 2 / 4, 8 / 5, 10 / 6 over the row classes
 SHAPES = [(1024, 2048), (1024, 3072), (4096, 1024), (4096, 12288), (5120, 25600), (6144, 4096)]
 
 
@@ -61,6 +62,45 @@ def test_silu_mul(dev, inter):
         assert torch.isfinite(out).all() and (err <= 0).all(), f"max excess {err.max().item():.3g}"
 
 
+def _silu_bound(x, w, inter):
+    """The exact silu(g) u and what its roundings may move it by: the fp32 sums
+    and the bf16 rounding (half of a last place, 2^-8 of the value) of g and u, that of the result, and 2^-18 for
+    the fp32 exponential, reciprocal and products between; |silu'| < 1.1."""
+    xd, wd = x.double(), w.double()
+    gu, mass = xd @ wd.T, xd.abs() @ wd.abs().T
+    d = mass * (x.shape[1] * 2.0**-24)
+    d += (gu.abs() + d) * 2.0**-8
+    g, u, dg, du = gu[:, :inter], gu[:, inter:], d[:, :inter], d[:, inter:]
+    silu = g * torch.sigmoid(g)
+    want = silu * u
+    bound = 1.1 * dg * (u.abs() + du) + silu.abs() * du
+    return want, bound + (want.abs() + bound) * (2.0**-8 + 2.0**-18) + 2.0**-133  # (subnormal results)
+
+
+@pytest.mark.parametrize("rows", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("mode", [1, 2])
+def test_every_kernel_over_turns_of_its_ring(dev, mode, rows):
+    """Each kernel of the row class, at the class's fewest and most rows, over
+    an odd number of stages past two turns of the deepest ring."""
+    from helpers import stream_kernel, stream_kernel_shapes
+    from xvllm import _C
+    from xvllm.layers.linear import streamed_into_norm, streamed_silu_mul
+
+    shapes = {k: v for k, v in stream_kernel_shapes(_C.lib()).items() if k[:2] == (mode, rows)}
+    assert shapes
+    for kernel, (n, k) in sorted(shapes.items()):
+        for m in (rows // 2 + 1 if rows > 16 else 1, rows):
+            assert stream_kernel(_C.lib(), m, n, k, mode) == kernel
+            print(f"stream gemm kernel {kernel} m {m} n {n} k {k}", flush=True)
+            x, w = _operands(dev, m, n, k, m + n)
+            if mode == 1:
+                _check_parts(streamed_into_norm(x, w), x, w)
+            else:
+                want, bound = _silu_bound(x, w, n // 2)
+                err = (streamed_silu_mul(x, w).double() - want).abs() - bound
+                assert (err <= 0).all(), f"max excess {err.max().item():.3g}"
+
+
 def test_strided_rows(dev):
     """x and w as row-strided views, and x off its 16-byte alignment (copied first)."""
     from xvllm.layers.linear import streamed_into_norm
@@ -94,8 +134,8 @@ def test_rows_are_independent(dev):
 def test_mlp_streams_and_matches_the_library(dev, m, width):
     """The MLP, packed or not: packed models stream up to 256 rows, others the
     products into a norm where linear_into_norm splits, all within the
-    bf16 tolerance of the library's product; with gradients on, an unpacked
-    model keeps the library's."""
+    bf16 tolerance of the library's product, with gradients on too (what
+    those calls run on is test_gradients_keep_the_library's)."""
     from xvllm.config import QWEN3_0_6B, QWEN3_8B
     from xvllm.layers.linear import PartialSums, split_factor
     from xvllm.models.qwen3 import Qwen3MLP
