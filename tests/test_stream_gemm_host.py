@@ -124,3 +124,32 @@ def test_every_picked_kernel_exists(lib):
         width = n if mode == 1 else n // 2
         rc = lib.xv_stream_gemm(A, k, A, k, A, width, m * n, m, n, k, mode, lib.xv_stream_gemm_parts(m, n, k, mode), None)
         assert rc not in (0, INVALID), (mode, m, n, k, rc)
+
+
+def test_packing_does_not_hold_weights_read_in_place():
+    """pack() keeps nothing of a weight that streams in place: replacing the
+    parameter frees it, and the operand is the new one."""
+    import gc
+    import weakref
+
+    import numpy as np
+    from xvllm.config import Qwen3Shape
+    from xvllm.models.qwen3 import Qwen3DecoderLayer
+
+    layer = Qwen3DecoderLayer(Qwen3Shape(1024, 16, 8, 128, 3072, 1, max_position_embeddings=64), 0).to(torch.bfloat16)
+    for module, name, operand in ((layer.mlp, "gate_up_proj", lambda: layer.mlp.packed[0]),
+                                  (layer.mlp, "down_proj", lambda: layer.mlp.packed[1]),
+                                  (layer.self_attn, "o_proj", lambda: layer.self_attn.packed_o)):
+        shape = getattr(module, name).shape
+        store = np.zeros(shape.numel(), np.int16)
+        freed = weakref.ref(store)
+        setattr(module, name, torch.nn.Parameter(torch.from_numpy(store).view(torch.bfloat16).view(shape), requires_grad=False))
+        del store
+        module.pack()
+        assert operand().data_ptr() == getattr(module, name).data_ptr() and freed() is not None
+        setattr(module, name, torch.nn.Parameter(torch.zeros(shape, dtype=torch.bfloat16), requires_grad=False))
+        gc.collect()
+        assert freed() is None, name
+        assert operand().data_ptr() == getattr(module, name).data_ptr()
+        module.pack(False)
+    assert layer.mlp.packed is None and layer.self_attn.packed_o is None

@@ -55,9 +55,9 @@ def _needs_copy(w: torch.Tensor, mode: int) -> bool:
     return any(in_place_parts(m, *w.shape, mode) == 0 for m in (16, STREAM_MAX_ROWS))
 
 
-def _decode_operand(p: nn.Parameter, mode: int):
-    """The weight itself where the in-place kernel streams it, else a packed copy."""
-    return pack_weight(p.data) if _needs_copy(p, mode) else p.data
+def _packed_copy(p: nn.Parameter, mode: int):
+    """The packed copy of a weight, None where the in-place kernel streams the weight itself."""
+    return pack_weight(p.data) if _needs_copy(p, mode) else None
 
 
 def _is_observed(attn: nn.Module) -> bool:
@@ -73,14 +73,14 @@ class Qwen3MLP(nn.Module):
         self.gate_up_proj = nn.Parameter(torch.empty(2 * inter, hidden))  # [gate; up] (linear.py:297-304)
         self.down_proj = nn.Parameter(torch.empty(hidden, inter))
         self.split_k = True
-        self.packed = None  # (gate_up, down) decode operands of pack()
+        self._copies = None  # pack(): the packed copies of (gate_up, down), None for one read in place
 
     def forward(self, x):
         """SiLU-MLP; the down GEMM may return PartialSums (split-K) for the
         next residual add + RMSNorm."""
         if not self.split_k:
             return F.linear(torch.ops.vllm.silu_and_mul(F.linear(x, self.gate_up_proj)), self.down_proj)
-        if self.packed is not None and stream_rows(x):
+        if self._copies is not None and stream_rows(x):
             _check_stamp(self, self._stamp, self.gate_up_proj, self.down_proj)
         gate_up, down = self.packed or (None, None)
         w = stream_operand(x, self.gate_up_proj, gate_up, GEMM_SILU_MUL)
@@ -91,12 +91,19 @@ class Qwen3MLP(nn.Module):
         w = stream_operand(act, self.down_proj, down, GEMM_PARTS)
         return streamed_into_norm(act, w) if w is not None else linear_into_norm(act, self.down_proj)
 
+    @property
+    def packed(self):
+        """The (gate_up, down) decode operands of pack(), None before it."""
+        if self._copies is None:
+            return None
+        return self._copies[0] or self.gate_up_proj, self._copies[1] or self.down_proj
+
     def pack(self, enabled: bool = True):
         if not enabled:
-            self.packed = None
-        elif self.packed is None and streamable(self.gate_up_proj, GEMM_SILU_MUL) and streamable(self.down_proj,
-                                                                                                   GEMM_PARTS):
-            self.packed = (_decode_operand(self.gate_up_proj, GEMM_SILU_MUL), _decode_operand(self.down_proj, GEMM_PARTS))
+            self._copies = None
+        elif self._copies is None and streamable(self.gate_up_proj, GEMM_SILU_MUL) and streamable(self.down_proj,
+                                                                                                    GEMM_PARTS):
+            self._copies = (_packed_copy(self.gate_up_proj, GEMM_SILU_MUL), _packed_copy(self.down_proj, GEMM_PARTS))
             self._stamp = _weight_stamp(self.gate_up_proj, self.down_proj)
 
 
@@ -116,7 +123,7 @@ class Qwen3Attention(nn.Module):
         self.attn = Attention(self.num_heads, self.head_dim, self.num_kv_heads, layer_id=layer_id)
         self.eps = cfg.rms_norm_eps
         self.split_k = True
-        self.packed_o = None  # o_proj decode operand of pack()
+        self._copies = None  # pack(): the packed copy of (o_proj,), None if read in place
 
     def forward(self, positions, hidden, attn: AttnInputs):
         """qkv -> q/k norm + RoPE -> attention -> o GEMM (PartialSums when
@@ -141,16 +148,21 @@ class Qwen3Attention(nn.Module):
             o = self.attn(q.view(q.shape[0], self.q_size), k, v, attn)
         if not self.split_k:
             return F.linear(o, self.o_proj)
-        if self.packed_o is not None and stream_rows(o):
+        if self._copies is not None and stream_rows(o):
             _check_stamp(self, self._stamp, self.o_proj)
         w = stream_operand(o, self.o_proj, self.packed_o, GEMM_PARTS)
         return streamed_into_norm(o, w) if w is not None else linear_into_norm(o, self.o_proj)
 
+    @property
+    def packed_o(self):
+        """The o_proj decode operand of pack(), None before it."""
+        return None if self._copies is None else self._copies[0] or self.o_proj
+
     def pack(self, enabled: bool = True):
         if not enabled:
-            self.packed_o = None
-        elif self.packed_o is None and streamable(self.o_proj, GEMM_PARTS):
-            self.packed_o = _decode_operand(self.o_proj, GEMM_PARTS)
+            self._copies = None
+        elif self._copies is None and streamable(self.o_proj, GEMM_PARTS):
+            self._copies = (_packed_copy(self.o_proj, GEMM_PARTS),)
             self._stamp = _weight_stamp(self.o_proj)
 
     def _views(self, qkv):
