@@ -283,8 +283,12 @@ struct StreamPlan {
 // 256 workgroups 11.3 us, 192 13.4).  A workgroup reads m x (k / parts) of x and writes m x 16 bnt
 // partial sums that the consumer reads back; with 256 workgroups bnt grows
 // with the split, and the two costs balance at parts^2 ~ k / (n / 16)
-// (Qwen3-8B, 64 rows: down 8 parts 20.1 us, 4 parts 21.4; o 4 parts 9.6, 8 parts
-// 10.1, 2 parts 10.6; 8 rows want half as many: o 2 parts 8.0, 4 parts 8.8).
+// (products alone, Qwen3-8B, 64 rows: down 8 parts 20.1 us, 4 parts 21.4; o 4 parts 9.6, 8 parts
+// 10.1, 2 parts 10.6; 8 rows want half as many: o 2 parts 8.0, 4 parts 8.8.
+// In a layer with the consumer that reads the parts, 80 to 256 rows: Qwen3-8B
+// o 2 parts +1.4 .. 4.1 us, 8 parts +1.6 .. 3.9, down 4 parts +1.5 .. 4.9,
+// Qwen3-32B o 8 parts +0.4 .. 3.5, down 4 parts +1.4 .. 7.5; Qwen3-0.6B's 1024
+// columns take 8 parts where 4 are 0.3 to 2.0 better).
 // Gate/up (no split) takes the block count nearest 256, at up to 16 rows
 // blocks of two tiles whatever their number (8 rows, Qwen3-8B: 768 blocks 31.0
 // us, 256 blocks 33.1).  Shapes outside these bounds are not taken: with n /

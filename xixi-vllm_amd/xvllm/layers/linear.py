@@ -3,19 +3,37 @@ the [N, K] weight in place (xv_stream_gemm: gate_up fused with SiLU-and-mul,
 down and o as split-K partials for the norm that follows them, reference
 src/compute/models/qwen3.py:64,115 feeding the norms of :150,:152, a decode
 batch's qkv as partials for its norm + RoPE + KV store), above that
-and for shapes it does not take PyTorch (hipBLASLt) with a split-K form for the
-latter two.  pack_weight / dense_gemm are the older streamed form over packed
+and for shapes it does not take PyTorch (hipBLASLt) with a split-K form for
+down and o.  A model that was not packed streams down and o only where that
+form splits (split_factor > 1), since its callers see PartialSums only there:
+Qwen3-0.6B's two, Qwen3-8B's down up to 16 rows and its o at 17 to 48, and
+Qwen3-32B's o up to 32 rows and at 65 to 80 stay on hipBLASLt.  A prefill
+batch's qkv does at every size (attention reads its q, k and v as bf16).
+pack_weight / dense_gemm are the older streamed form over packed
 weight tiles (at most 64 rows), kept where the in-place kernel does not take
 a shape: Qwen3-32B's gate_up (51200 x 5120) at 17 to 64 rows, 87 us at 32
 rows against hipBLASLt's 98.
 
-us with the weights streamed from HBM, hipBLASLt -> in place (gate_up with
-its SiLU; MI355X, graph replay, over 1 GB of weights cycled):
+us of the products alone with the weights streamed from HBM, hipBLASLt -> in
+place (gate_up with its SiLU; MI355X, graph replay, over 1 GB of weights cycled):
     Qwen3-8B    gate_up  M 8: 46.5 -> 31.0   M 64: 47.8 -> 34.6   M 200: 64.5 -> 54.9
                 down     M 8: 22.1 -> 18.1   M 64: 23.6 -> 20.1   M 200: 34.6 -> 31.7
                 o        M 8: 10.3 -> 8.0    M 64: 14.8 -> 9.6    M 200: 18.1 -> 16.6
                 qkv      M 8: 15.7 -> 11.3   M 64: 18.0 -> 11.9   M 200: 26.8 -> 21.1 (4 partial sums)
     Qwen3-0.6B  gate_up  M 8: 10.3 -> 5.1    down M 8: 12.1 -> 4.0   o M 8: 9.7 -> 3.4
+
+us that a decode layer takes longer with one of its products, and its
+consumer, on hipBLASLt instead (recorded model bodies of 4 to 24 packed layers,
+contexts of 64 tokens; runs of one side differ by up to 1 us, 3 at Qwen3-32B):
+    Qwen3-0.6B  (58 .. 81 a layer)    qkv 3 .. 6   gate_up 2 .. 5    o -0.2 .. 2.7   down -2.2 .. 0
+    Qwen3-8B    (118 .. 185)          qkv 5 .. 21  gate_up 7 .. 13   o -0.8 .. 2.7   down 1.4 .. 5.7
+    Qwen3-32B   (235 .. 372)          qkv 10 .. 30 (no gate_up)      o 3 .. 13       down -0.4 .. 22
+    hidden 2048, MLP 6144 (72 .. 106) qkv 0.5 .. 11  gate_up 1.5 .. 7  o 0.8 .. 3.8  down 0.5 .. 6.5
+    hidden 2560, MLP 9728 (99 .. 156) (qkv not timed, no gate_up)      o 2 .. 11     down 4 .. 15
+at M 72 to 256.  Only Qwen3-0.6B's down loses (packed models, above 72 rows:
+from 96 rows on its 8 partial sums, written and read, are more bytes than the
+weight), by less than its gate_up gains.  Up to 16 rows a gate_up that has a packed copy runs
+in place too: Qwen3-32B 4 rows 2.9 us faster, 12 rows even, 16 rows 2.5 slower.
 
 The split-K measurements below are the hipBLASLt path.
 

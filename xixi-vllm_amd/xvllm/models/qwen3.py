@@ -5,10 +5,11 @@ Per layer: input RMSNorm (fused with the residual add after layer 0), fused
 qkv GEMM, per-head q/k RMSNorm + NeoX RoPE (one kernel, `xv::qk_norm_rope`),
 `vllm::attention` (KV store + paged decode / prefill), o GEMM, fused add +
 RMSNorm, gate_up GEMM, SiLU-and-mul, down GEMM.  Batches of up to 256 rows
-stream gate_up (with the SiLU-and-mul), down and o in place (xv_stream_gemm),
-down and o as split-K partials into the next norm, decode batches also qkv, as
-partials into the norm + RoPE + KV store kernel; larger ones and shapes
-that kernel does not take run on PyTorch (hipBLASLt).  Weights are plain
+stream gate_up (with the SiLU-and-mul) in place (xv_stream_gemm), decode
+batches also qkv, as partials into the norm + RoPE + KV store kernel, and
+down and o as split-K partials into the next norm: a packed model at every
+size, others where the library's product would split too.  Larger batches and
+the products and shapes outside this run on PyTorch (hipBLASLt).  Weights are plain
 tensors (random init for the benchmarks; the reference's checkpoint loader is
 out of scope).
 """
