@@ -331,7 +331,7 @@ def kernel_suite(torch, dev) -> dict:
         # max_top_k as the serving loop passes it (the reference's Batch.max_top_k)
         rec(f"sampler_k50_p0.9_B{bsz}", _time(torch, lambda: sample(logits, temps, tps, tks, None, u, use_top_k=True,
                                                                     use_top_p=True, max_top_k=50), 20), bsz * V * 2)
-        if bsz in (64, 256):  # the same call without the bound: the histogram chain / one workgroup per row
+        if bsz in (64, 256):  # the same call without the bound: the per-key counts
             rec(f"sampler_k50_p0.9_B{bsz}_no_max_top_k",
                 _time(torch, lambda: sample(logits, temps, tps, tks, None, u, use_top_k=True, use_top_p=True), 20),
                 bsz * V * 2)
@@ -345,7 +345,8 @@ def kernel_suite(torch, dev) -> dict:
     u = torch.rand(bsz, generator=g, device=dev)
     rec("sampler_p0.95_flat_B32", _time(torch, lambda: sample(logits, temps, tps, None, None, u, use_top_p=True), 20),
         bsz * V * 2)
-    # Decode GEMMs on the weight-streaming kernel (packed weights, enough
+    # Decode GEMMs on the kernel over packed weight tiles (the decoder reads
+    # these shapes in place, see decode_e2e; packed weights, enough
     # weight sets cycled to pass 600 MB: past the 256 MB MALL, as the model's
     # 15 GB of weights are) against hipBLASLt over the [N, K]
     # weights (the unsplit GEMM + SiLU-and-mul kernel for gate_up, the split-K

@@ -432,7 +432,7 @@ int xv_sample(const void* logits, int64_t logits_stride, int batch, int vocab,
  * MergedColumnParallelLinear.forward src/compute/layers/linear.py:306, with
  * the SiLU-and-mul after it, activation.py:6-8; down_proj,
  * RowParallelLinear.forward linear.py:141) and o_proj (qwen3.py:115,
- * linear.py:141); prefill and larger batches keep them on hipBLASLt.
+ * linear.py:141), where xv_stream_gemm does not take their shape.
  *   w_packed  w in 16-row x 64-column tiles of 2 KB, row blocks outermost,
  *             tile (nb, sg): w[16 nb + l % 16][64 sg + 8 (l / 16) + e] at
  *             8 l + e and w[16 nb + l % 16][64 sg + 32 + 8 (l / 16) + e] at
